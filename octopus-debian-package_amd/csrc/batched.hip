@@ -22,11 +22,15 @@
 
 namespace octhip {
 void h_apply_args(const octhip_hamiltonian_s* h, const double* in, int L, double* ksum, ApplyArgs& a);
-int zmarch_items(octhip_nl_operator_s* op, int zs);
-int zmarch_zseg(const octhip_nl_operator_s* op, int nchunk, int lc, int resident, bool alone);
-int zmarch_reg_blocks(int lc, int lpt, int epi, bool nl, bool multi);
+int zmarch_plan(octhip_nl_operator_s* op, int zs, octhip_nl_operator_s::ZPlan** out);
+std::vector<int4> zmarch_deal(const std::vector<int4>& all);
+std::vector<int2> zmarch_items(const octhip_nl_operator_s* op, int zs);
+extern const int ZM_SEGS[7];
+double zmarch_makespan(const std::vector<int>& planes, int lc, int resident);
+int zmarch_nt(const octhip_nl_operator_s* op, const ApplyArgs& a);
+int zmarch_resident(int lc, int lpt, int epi, bool nl, bool multi);
 bool zmarch_fits(const octhip_nl_operator_s* op, const ApplyArgs& a);
-int launch_zmarch_multi(const ZArgs* zs, const int4* sched, int len, int lc, int lpt, int epi, bool nl, int zseg,
+int launch_zmarch_multi(const ZArgs* zs, const int4* sched, int len, int lc, int lpt, int epi, bool nl,
                         hipStream_t s);
 }  // namespace octhip
 
@@ -43,12 +47,8 @@ struct Pair {
   double* proj = nullptr;
   double* ksum = nullptr;
   double* y[3] = {nullptr, nullptr, nullptr};  // Taylor powers (three for order 4)
-  // the operator's z-march items and their index tables, one plan per epilogue ([0] plain
-  // store, [1] Taylor): the two instances keep different numbers of workgroups resident
-  const int4* items[2] = {nullptr, nullptr};
-  const int* tab[2] = {nullptr, nullptr};
-  const int* tab_off[2] = {nullptr, nullptr};
-  int nitems[2] = {0, 0};
+  // the operator's z-march items, one plan per epilogue ([0] plain store, [1] Taylor)
+  const octhip_nl_operator_s::ZPlan* plan[2] = {nullptr, nullptr};
 };
 
 // a device table of argument blocks plus block offsets for one multi-segment kernel
@@ -85,12 +85,11 @@ struct octhip_batched_s {
   double dt = 0.0;
   bool mfma = true, nl = false;
   int lc = 16, lpt = 2;
-  int zseg[2] = {8, 8};                 // per plan: longest segment (LDS size)
   std::complex<double> zf[33];
   Seg zero, reduce, ket, ksum;
   std::vector<Seg> bra;                 // [0] H-apply input psi, [k] Taylor order k input
   std::vector<ZArgs*> zdesc;            // [0] H-apply (store to hpsi), [k] Taylor order k
-  int4* sched[2] = {nullptr, nullptr};  // per plan: blockIdx -> (pair, item, lane chunk)
+  int4* sched[2] = {nullptr, nullptr};  // per plan: blockIdx -> {first record, planes, lane chunk, pair}
   int sched_len[2] = {0, 0};
 };
 
@@ -172,6 +171,8 @@ int build_zdesc(octhip_batched_s* b, int k, ZArgs** out) {
     std::memset(&z, 0, sizeof(z));
     const double* in = pass_input(p, k, b->order);
     h_apply_args(p.h, in, p.L, p.ksum, z.a);
+    z.a.reuse = k > 0;
+    z.a.nt = zmarch_nt(op, z.a);
     const bool deferred = taylor_deferred(b->order);
     if (k == 0) {
       z.a.fo = p.hpsi;
@@ -208,14 +209,11 @@ int build_zdesc(octhip_batched_s* b, int k, ZArgs** out) {
         z.a.c2i = b->zf[k].imag();
       }
     }
-    const int plan = pass_epi(b, k);
-    z.items = p.items[plan];
-    z.tab = p.tab[plan];
-    z.tab_off = p.tab_off[plan];
+    z.rec = op->d_rec;
     z.sched = nullptr;
     // every pointer the kernel dereferences must exist
     // (the H-apply descriptor may lack fo: octhip_batched_apply refuses to run without hpsi)
-    const bool ok = z.a.fi && z.items && z.tab && z.tab_off && (!z.a.kslot || z.a.ksum) &&
+    const bool ok = z.a.fi && z.rec && (!z.a.kslot || z.a.ksum) &&
                     (deferred ? (k == 0 || (k < b->order ? z.a.fo != nullptr : z.a.acc != nullptr))
                               : ((k < 2 || z.a.acc) && (k == 0 || k == b->order || z.a.yout)));
     if (!ok) return fail(OCTHIP_ERR_STATE, "batched: incomplete descriptor for pair %zu, pass %d", i, k);
@@ -240,8 +238,7 @@ int run_pass(octhip_batched_s* b, int k, hipStream_t s) {
   int rc = run_bra(b, b->bra[k], s);
   if (rc) return rc;
   const int epi = pass_epi(b, k);
-  return launch_zmarch_multi(b->zdesc[k], b->sched[epi], b->sched_len[epi], b->lc, b->lpt, epi, b->nl,
-                             b->zseg[epi], s);
+  return launch_zmarch_multi(b->zdesc[k], b->sched[epi], b->sched_len[epi], b->lc, b->lpt, epi, b->nl, s);
 }
 
 }  // namespace
@@ -279,8 +276,8 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
   b->mfma = minL >= 16;
   for (int i = 0; i < npairs; ++i) b->mfma = b->mfma && hms[i]->use_mfma;
   taylor_coefs(deltat, 0, order, b->zf);
-  const int resident[2] = {zmarch_reg_blocks(b->lc, b->lpt, EPI_STORE, b->nl, true),
-                           zmarch_reg_blocks(b->lc, b->lpt, EPI_TAYLOR, b->nl, true)};
+  const int resident[2] = {zmarch_resident(b->lc, b->lpt, EPI_STORE, b->nl, true),
+                           zmarch_resident(b->lc, b->lpt, EPI_TAYLOR, b->nl, true)};
   int rc = OCTHIP_SUCCESS;
   // pairs and their work buffers
   for (int i = 0; i < npairs && !rc; ++i) {
@@ -299,18 +296,32 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
     if (!rc) rc = dalloc((void**)&p.y[0], sizeof(double) * h->np * L);
     if (!rc) rc = dalloc((void**)&p.y[1], sizeof(double) * h->np * L);
     if (!rc && taylor_deferred(order) && order == 4) rc = dalloc((void**)&p.y[2], sizeof(double) * h->np * L);
-    // one plan per epilogue, segments for the residency of that instance
-    for (int plan = 0; plan < 2 && !rc; ++plan) {
-      rc = zmarch_items(h->kin, zmarch_zseg(h->kin, p.L / b->lc, b->lc, resident[plan], false));
-      if (!rc) {
-        p.items[plan] = h->kin->d_items;
-        p.tab[plan] = h->kin->d_tab;
-        p.tab_off[plan] = h->kin->d_tab_off;
-        p.nitems[plan] = h->kin->nitems;
-        b->zseg[plan] = std::max(b->zseg[plan], h->kin->zseg_built);
+    b->pairs.push_back(p);
+  }
+  // one plan per epilogue: the segment length with the smallest estimated time of the whole
+  // work list (an operator's own setting goes first)
+  for (int plan = 0; plan < 2 && !rc; ++plan) {
+    auto seg_of = [](const Pair& p, int zs) { return p.h->kin->zseg > 0 ? p.h->kin->zseg : zs; };
+    double best_t = 1e300;
+    int best = 8;
+    for (int zs : ZM_SEGS) {
+      std::vector<int> planes;
+      for (const Pair& p : b->pairs) {
+        const std::vector<int2> items = zmarch_items(p.h->kin, seg_of(p, zs));
+        for (int c = 0; c < p.L / b->lc; ++c)
+          for (const int2& it : items) planes.push_back(it.y);
+      }
+      const double t = zmarch_makespan(planes, b->lc, resident[plan]);
+      if (t < best_t) {
+        best_t = t;
+        best = zs;
       }
     }
-    b->pairs.push_back(p);
+    for (Pair& p : b->pairs) {
+      octhip_nl_operator_s::ZPlan* pl = nullptr;
+      if (!rc) rc = zmarch_plan(p.h->kin, seg_of(p, best), &pl);
+      p.plan[plan] = pl;
+    }
   }
   // boundary clear, reduce, ket, ket sums
   if (!rc) {
@@ -379,17 +390,9 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
     for (size_t i = 0; i < b->pairs.size(); ++i) {
       const int nchunk = b->pairs[i].L / b->lc;
       for (int c = 0; c < nchunk; ++c)
-        for (int it = 0; it < b->pairs[i].nitems[plan]; ++it) all.push_back(make_int4((int)i, it, c, 0));
+        for (const int2& it : b->pairs[i].plan[plan]->items) all.push_back(make_int4(it.x, it.y, c, (int)i));
     }
-    const int n = (int)all.size();
-    const int per = (n + 7) / 8;
-    std::vector<int4> sc((size_t)per * 8, make_int4(-1, 0, 0, 0));
-    for (int k = 0; k < 8; ++k)
-      for (int i = 0; i < per; ++i) {
-        const int g = k * per + i;
-        if (g >= n) break;
-        sc[(size_t)i * 8 + k] = all[g];
-      }
+    const std::vector<int4> sc = zmarch_deal(all);
     rc = upload(&b->sched[plan], sc.data(), sc.size(), nullptr);
     b->sched_len[plan] = (int)sc.size();
   }

@@ -274,13 +274,6 @@ int periodic_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, 
 }
 }  // namespace
 
-namespace octhip {
-int propagator_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, hipStream_t s) {
-  if (is_periodic(h)) return periodic_apply(h, psi, hpsi, ldf, 1, OCTHIP_TERM_ALL, 1, true, s);
-  return octhip_hamiltonian_apply_batch(h, psi, hpsi, ldf, 1, OCTHIP_TERM_ALL, 1, s);
-}
-}  // namespace octhip
-
 extern "C" int octhip_hamiltonian_create(octhip_nl_operator_t kinetic, double mass, const double* vlocal,
                                          int nmat, const int* offsets, const double* matrices,
                                          const int* maps, const double* scals, octhip_hamiltonian_t* out) {
@@ -355,16 +348,16 @@ extern "C" int octhip_hamiltonian_create(octhip_nl_operator_t kinetic, double ma
     }
     h->nchunk = (int)chunks.size();
     // ket row per mesh point: its sphere point if it lies in one sphere, else a summed row
-    std::vector<int> kslot(np, -1), multi_pos(1, 0), multi_g;
+    std::vector<int> kslot(np, 0), multi_pos(1, 0), multi_g;
     int nslot = 0;
     for (int p = 0; p < np; ++p) {
       const int ne = pos[p + 1] - pos[p];
       if (ne == 0) continue;
       ++nslot;
       if (ne == 1) {
-        kslot[p] = ent[pos[p]].x;
+        kslot[p] = ent[pos[p]].x + 1;
       } else {
-        kslot[p] = (int)total_points + (int)multi_pos.size() - 1;
+        kslot[p] = (int)total_points + (int)multi_pos.size();
         for (int e = pos[p]; e < pos[p + 1]; ++e) multi_g.push_back(ent[e].x);
         multi_pos.push_back((int)multi_g.size());
       }
@@ -533,16 +526,11 @@ extern "C" int octhip_hamiltonian_trim(octhip_hamiltonian_t h) {
   return OCTHIP_SUCCESS;
 }
 
-extern "C" int octhip_hamiltonian_apply_batch(octhip_hamiltonian_t h, double* psi, double* hpsi, int ldf,
-                                              int is_complex, int terms, int set_bc, void* stream) {
-  OCTHIP_RANGE("octhip_hamiltonian_apply_batch");
-  OCTHIP_REQUIRE_INIT();
-  OCTHIP_REQUIRE(h != nullptr, "null hamiltonian handle");
-  OCTHIP_REQUIRE(psi && hpsi && psi != hpsi, "bad batch pointers");
-  OCTHIP_REQUIRE(ldf >= 0 && ldf <= MAX_LDF, "ldf=%d outside 0..%d", ldf, MAX_LDF);
-  OCTHIP_REQUIRE(!is_complex || ldf >= 1, "complex batch needs ldf >= 1");
-  hipStream_t s = (hipStream_t)stream;
-  if (is_periodic(h)) return periodic_apply(h, psi, hpsi, ldf, is_complex, terms, set_bc, false, s);
+namespace {
+// H psi with the zero boundary (or the boundary rows as they are); reuse: the caller's next
+// kernel reads hpsi
+int finite_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, int terms, int set_bc, bool reuse,
+                 hipStream_t s) {
   const int L = 1 << ldf;
   const octhip_nl_operator_s* op = h->kin;
   int rc = ensure_work(h, ldf, s);
@@ -562,8 +550,30 @@ extern "C" int octhip_hamiltonian_apply_batch(octhip_hamiltonian_t h, double* ps
   a.fo = hpsi;
   a.L = L;
   a.lim = set_bc ? op->np : op->np_part;
+  a.reuse = reuse ? 1 : 0;
   return launch_operator(h->kin, a, EPI_STORE, s);
 }
+}  // namespace
+
+extern "C" int octhip_hamiltonian_apply_batch(octhip_hamiltonian_t h, double* psi, double* hpsi, int ldf,
+                                              int is_complex, int terms, int set_bc, void* stream) {
+  OCTHIP_RANGE("octhip_hamiltonian_apply_batch");
+  OCTHIP_REQUIRE_INIT();
+  OCTHIP_REQUIRE(h != nullptr, "null hamiltonian handle");
+  OCTHIP_REQUIRE(psi && hpsi && psi != hpsi, "bad batch pointers");
+  OCTHIP_REQUIRE(ldf >= 0 && ldf <= MAX_LDF, "ldf=%d outside 0..%d", ldf, MAX_LDF);
+  OCTHIP_REQUIRE(!is_complex || ldf >= 1, "complex batch needs ldf >= 1");
+  hipStream_t s = (hipStream_t)stream;
+  if (is_periodic(h)) return periodic_apply(h, psi, hpsi, ldf, is_complex, terms, set_bc, false, s);
+  return finite_apply(h, psi, hpsi, ldf, terms, set_bc, false, s);
+}
+
+namespace octhip {
+int propagator_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, hipStream_t s) {
+  if (is_periodic(h)) return periodic_apply(h, psi, hpsi, ldf, 1, OCTHIP_TERM_ALL, 1, true, s);
+  return finite_apply(h, psi, hpsi, ldf, OCTHIP_TERM_ALL, 1, true, s);
+}
+}  // namespace octhip
 
 namespace octhip {
 // zfact_k, k = 1..order: zfact *= (-i * deltat) / k (exponential.F90:720-724); deltat ->
@@ -851,6 +861,7 @@ int taylor_step(octhip_hamiltonian_s* h, double* psi, int ldf, double deltat, in
       a.fi = yin;
       a.L = L;
       a.lim = op->np;  // boundary rows are zero: psi's were just cleared, work buffers have none
+      a.reuse = 1;
       if (k < order) {
         a.fo = Y(k);
         rc = launch_operator(h->kin, a, EPI_STORE, s);
@@ -892,6 +903,7 @@ int taylor_step(octhip_hamiltonian_s* h, double* psi, int ldf, double deltat, in
     a.fi = yin;
     a.L = L;
     a.lim = op->np;  // boundary rows are zero: psi's were just cleared, work buffers have none
+    a.reuse = 1;
     if (order == 1) {
       a.fo = h->d_y[0];
       rc = launch_operator(h->kin, a, EPI_STORE, s);
@@ -1011,6 +1023,7 @@ int series_generic(octhip_hamiltonian_s* h, double* psi, int ldf, std::complex<d
       a.fo = yout;
       a.L = L;
       a.lim = h->np;
+      a.reuse = 1;
       rc = launch_operator(h->kin, a, EPI_STORE, s);
     }
     if (!rc) rc = launch_zaxpy(psi, yout, count, z[k].real(), z[k].imag(), s);
@@ -1046,6 +1059,7 @@ int series_fused(octhip_hamiltonian_s* h, double* psi, int ldf, std::complex<dou
     a.fi = yin;
     a.L = L;
     a.lim = h->np;
+    a.reuse = 1;
     if (k < order) {
       a.fo = h->d_y[k - 1];
       rc = launch_operator(h->kin, a, EPI_STORE, s);

@@ -40,7 +40,7 @@ struct ApplyArgs {
   double w[MAX_STENCIL];           // weights already multiplied by the factor
   // local potential (the dipole term, if any, is already folded in)
   const double* __restrict__ v;
-  // nonlocal ket: kslot[p] = row of ksum holding sum_a P_a proj_a at point p, or -1
+  // nonlocal ket: kslot[p] - 1 = row of ksum holding sum_a P_a proj_a at point p; 0: none
   const int* __restrict__ kslot;
   const double* __restrict__ ksum;
   int nk;                          // rows of ksum
@@ -63,6 +63,8 @@ struct ApplyArgs {
   double d1r, d1i, d2r, d2i, dar, dai, dbr, dbi;
   double* dpart;
   const double* dw;
+  int reuse;                       // the output rows are read again by the next pass
+  int nt;                          // z-march: non-temporal stores of the output rows
 };
 
 __device__ __forceinline__ int tile_of(int b, int chunk) {
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(BLOCK) void k_apply(const ApplyArgs a) {
     const int p = p0 + t;
     const int* qi = sidx + t * ss;
     const double vv = a.v ? a.v[p] : 0.0;
-    const int ks = a.kslot ? a.kslot[p] : -1;
+    const int ks = a.kslot ? a.kslot[p] - 1 : -1;
     double dsum = 0.0;  // EPI_TAYLOR_X: this thread's share of the point's density
     for (int l = lane0; l < a.L; l += tpp * LPT) {
       Vec<LPT> s;

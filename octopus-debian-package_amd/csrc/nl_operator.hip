@@ -5,6 +5,7 @@
 #include <deque>
 
 #include <map>
+#include <queue>
 
 #include "zmarch.h"
 
@@ -155,65 +156,121 @@ int build_march(octhip_nl_operator_s* op, hipStream_t s) {
 }  // namespace
 
 namespace octhip {
-int zmarch_reg_blocks(int lc, int lpt, int epi, bool nl, bool multi);
+int zmarch_resident(int lc, int lpt, int epi, bool nl, bool multi);
 
-// Segment length of a launch with nchunk lane chunks of lc lanes: the operator's setting,
-// or the candidate (48, 32, 28, 24, 22, 21, 20, 16, 12, 8 planes) with the smallest
-// estimated time, in plane steps of one workgroup:
-//   work  = nchunk * sum over items (planes + 8 overlap planes + ZM_PROLOGUE)
-//   time  = max(work / (CUs * g), longest item * r / g) * (1 + ZM_TAIL * idle)
-// where r = workgroups resident per CU (2 when the instance's registers allow it and the
-// segment's LDS fits twice, else 1) and g = the throughput of r resident workgroups
-// relative to one (ZM_TWO_GAIN for two).  The first term is the whole launch spread over
-// the chip, the second its critical path: long segments cost little overlap but leave
-// CUs idle on small meshes.  idle = the unused fraction of the last wave of workgroups on
-// an XCD (items per XCD over its resident slots, rounded up, minus the unrounded value;
-// counted when there is at least one full wave): near-equal items leave that many slots
-// empty at the end.  Measured on MI355X: R=12 sphere, 32 complex states: 24 planes with
-// two resident workgroups beat 48 with one by 7%, and 21-22 planes (3.7-3.8 waves per
-// XCD) beat 24 (3.4) and 28 (3.1) by 1%; the 64^3 Laplacian with 8 lanes: 8 planes
-// (24 us against 38 us at 32).
-constexpr double ZM_PROLOGUE = 4.0;  // item prologue, in plane steps
-constexpr double ZM_TWO_GAIN = 1.3;  // throughput of two resident workgroups against one
-constexpr double ZM_TAIL = 0.25;     // cost of the idle slots of a partial last wave
-// alone: the launch holds this operator's items only (a batched launch shares its grid
-// with other systems, so the last-wave term of one system does not apply)
-int zmarch_zseg(const octhip_nl_operator_s* op, int nchunk, int lc, int resident, bool alone) {
-  if (op->zseg > 0) return op->zseg;
-  const int rkey = resident | (alone ? 0 : 0x100);
-  for (const auto& c : op->zseg_cache)
-    if (c.x == nchunk && c.y == lc && c.z == rkey) return c.w;
+constexpr double ZM_OVERHEAD = 6.0;  // an item's prologue and tail, in plane steps
+// running workgroups per CU that saturate the chip, of 16 and of 8 lanes
+constexpr double ZM_FULL16 = 0.75, ZM_FULL8 = 2.0;
+
+// (tile, z-segment) work items {first record plane, planes} for segment length zs: the z range
+// of the mesh is cut into slabs of equal thickness of at most zs planes, and an item is a
+// tile's part of a slab.  Neighbouring tiles so start a slab at the same plane and stay
+// within a few planes of each other, which keeps their halo rows in L2 (462,781 points, 32
+// states: 520 MB read instead of 590 with segments of equal length per tile).  Slab by slab,
+// then tile rows.
+std::vector<int2> zmarch_items(const octhip_nl_operator_s* op, int zs) {
+  int lo = INT_MAX, hi = -1;
+  for (size_t t = 0; t < op->tile_zlo.size(); ++t)
+    if (op->tile_zhi[t] >= 0) {
+      lo = std::min(lo, op->tile_zlo[t]);
+      hi = std::max(hi, op->tile_zhi[t]);
+    }
+  std::vector<int> first(op->tile_zlo.size(), 0);
+  int plane = 0;
+  for (size_t t = 0; t < op->tile_zlo.size(); ++t) {
+    first[t] = plane;
+    if (op->tile_zhi[t] >= 0) plane += op->tile_zhi[t] - op->tile_zlo[t] + 9;
+  }
+  std::vector<int2> items;
+  if (hi < 0) return items;
+  const long len = hi - lo + 1, nslab = (len + zs - 1) / zs;
+  for (long s = 0; s < nslab; ++s) {
+    const int a = lo + (int)(len * s / nslab), b = lo + (int)(len * (s + 1) / nslab);
+    for (size_t t = 0; t < op->tile_zlo.size(); ++t) {
+      if (op->tile_zhi[t] < 0) continue;
+      const int z0 = std::max(a, op->tile_zlo[t]), z1 = std::min(b, op->tile_zhi[t] + 1);
+      if (z0 < z1) items.push_back(make_int2(first[t] + z0 - op->tile_zlo[t], z1 - z0));
+    }
+  }
+  return items;
+}
+
+// bounds of the 8 contiguous parts of equal work of a list of items, one part per XCD
+std::vector<size_t> zmarch_cuts(const std::vector<int>& planes) {
+  double total = 0.0;
+  for (int p : planes) total += p + ZM_OVERHEAD;
+  std::vector<size_t> cut(9, 0);
+  double sum = 0.0;
+  int k = 1;
+  for (size_t i = 0; i < planes.size(); ++i) {
+    const double w = planes[i] + ZM_OVERHEAD;
+    while (k < 8 && sum + 0.5 * w >= total * k / 8.0) cut[k++] = i;
+    sum += w;
+  }
+  while (k <= 8) cut[k++] = planes.size();
+  return cut;
+}
+
+// Estimated time, in plane steps of a workgroup that has a CU for itself, of a launch over the
+// work items of `planes` output planes each, in order, with `resident` workgroups of lc lanes
+// per CU.  The items are dealt to the XCDs in contiguous parts of equal work; an XCD starts
+// its next item when one ends; an item costs its planes and ZM_OVERHEAD steps (index and row
+// prologue, four planes behind the last one); and all workgroups slow down together once more
+// than ZM_FULL16 (ZM_FULL8) per CU run (they share LDS, the vector caches and the memory).  Fitted to sweeps on MI355X, 16 lanes: 0.47 us per step alone (57,777 points,
+// 8 complex states: 8 planes 13.3 us, 12: 15.1, 16: 16.6, 32: 24.5), 462,781 points, 32 states:
+// 12 planes 183 us, 16: 179, 24: 175, 32: 172, 48: 175; 155,331 points, 32 states: 8 planes
+// 60 us, 16: 52, 24: 55, 48: 49; 64^3 points, 8 real functions: 8 planes 13.8 us, 24: 17.2.
+double zmarch_makespan(const std::vector<int>& planes, int lc, int resident) {
   static int ncu = 0;
   if (ncu <= 0 && (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, current_device()) != hipSuccess ||
                    ncu <= 0))
     ncu = 256;
-  const bool two_ok = resident >= 2;
+  const size_t slots = (size_t)std::max(ncu / 8, 1) * std::max(resident, 1);
+  const double cap = ncu * (lc >= 16 ? ZM_FULL16 * 16.0 / lc : ZM_FULL8 * 8.0 / lc);
+  const std::vector<size_t> cut = zmarch_cuts(planes);
+  std::priority_queue<std::pair<double, int>, std::vector<std::pair<double, int>>, std::greater<>> ends;
+  size_t next[8];
+  for (int x = 0; x < 8; ++x)
+    for (next[x] = cut[x]; next[x] < std::min(cut[x] + slots, cut[x + 1]); ++next[x])
+      ends.push({planes[next[x]] + ZM_OVERHEAD, x});
+  double clock = 0.0, time = 0.0;  // steps done by every running workgroup, time passed
+  while (!ends.empty()) {
+    const auto [end, x] = ends.top();
+    time += (end - clock) * std::max(1.0, (double)ends.size() / cap);
+    clock = end;
+    ends.pop();
+    if (next[x] < cut[x + 1]) ends.push({end + planes[next[x]++] + ZM_OVERHEAD, x});
+  }
+  return time;
+}
+
+// Segment lengths tried for a launch.  Longer ones save overlap planes, but neighbouring tiles
+// drift apart over a long march and lose each other's halo rows (462,781 points, 32 states: 33
+// planes 172 us, 49 planes 174-181; the Taylor pass 311 against 331).
+extern const int ZM_SEGS[7];
+const int ZM_SEGS[7] = {8, 12, 16, 20, 24, 32, 40};
+
+// Segment length of a launch with nchunk lane chunks of lc lanes: the operator's setting, or
+// the one with the smallest estimated time.
+int zmarch_zseg(const octhip_nl_operator_s* op, int nchunk, int lc, int resident) {
+  if (op->zseg > 0) return op->zseg;
+  for (const auto& c : op->zseg_cache)
+    if (c.x == nchunk && c.y == lc && c.z == resident) return c.w;
   double best_t = 1e300;
   int best = 8;
-  for (int zs : {48, 32, 28, 24, 22, 21, 20, 16, 12, 8}) {
-    const size_t shm = zmarch_shmem(lc, zs);
-    if (shm > 160 * 1024) continue;
-    const int r = (two_ok && shm <= 80 * 1024) ? 2 : 1;
-    const double g = r == 2 ? ZM_TWO_GAIN : 1.0;
-    double work = 0.0, cmax = 0.0;
-    long items = 0;
-    for (size_t t = 0; t < op->tile_zlo.size(); ++t) {
-      if (op->tile_zhi[t] < 0) continue;
-      const int len = op->tile_zhi[t] - op->tile_zlo[t] + 1;
-      const int n = (len + zs - 1) / zs;
-      work += len + n * (8.0 + ZM_PROLOGUE);
-      cmax = std::max(cmax, (len + n - 1) / n + 8.0 + ZM_PROLOGUE);
-      items += n;
-    }
-    double tm = std::max(nchunk * work / (ncu * g), cmax * r / g);
-    const double waves = std::ceil((double)items * nchunk / 8.0) / (std::max(ncu / 8, 1) * (double)r);
-    if (alone && waves >= 1.0) tm *= 1.0 + ZM_TAIL * (std::ceil(waves) - waves);
-    if (tm < best_t) {
-      best_t = tm;
+  for (int zs : ZM_SEGS) {
+    const std::vector<int2> items = zmarch_items(op, zs);
+    std::vector<int> planes;
+    planes.reserve(items.size() * nchunk);
+    for (int c = 0; c < nchunk; ++c)
+      for (const int2& it : items) planes.push_back(it.y);
+    const double t = zmarch_makespan(planes, lc, resident);
+    if (t < best_t) {
+      best_t = t;
       best = zs;
     }
   }
-  op->zseg_cache.push_back(make_int4(nchunk, lc, rkey, best));
+  op->zseg_cache.push_back(make_int4(nchunk, lc, resident, best));
   return best;
 }
 
@@ -233,134 +290,85 @@ void zmarch_shape(const octhip_nl_operator_s* op, int L, int* lc, int* lpt) {
 int zmarch_zseg_for(const octhip_nl_operator_s* op, int L, int epi, bool nl) {
   int lc, lpt;
   zmarch_shape(op, L, &lc, &lpt);
-  return zmarch_zseg(op, L / lc, lc, zmarch_reg_blocks(lc, lpt, epi, nl, false), true);
+  return zmarch_zseg(op, L / lc, lc, zmarch_resident(lc, lpt, epi, nl, false));
 }
 
-// (tile, z-segment) work items for segment length zs; every list built stays allocated
-// until the operator is destroyed (graphs and batched launches may point at it)
-int zmarch_items(octhip_nl_operator_s* op, int zs) {
-  if (op->zseg_built == zs && op->d_items) return OCTHIP_SUCCESS;
-  // save the current schedules with their plan, then switch
-  for (auto& pl : op->plans)
-    if (pl.zseg == op->zseg_built) {
-      pl.sched = op->sched;
-      pl.sched_len = op->sched_len;
-    }
+// Index records of every tile (layout in zmarch.h), built once per operator.
+int zmarch_records(octhip_nl_operator_s* op) {
+  if (op->d_rec) return OCTHIP_SUCCESS;
+  size_t planes = 0;
+  for (size_t t = 0; t < op->tile_zlo.size(); ++t)
+    if (op->tile_zhi[t] >= 0) planes += (size_t)(op->tile_zhi[t] - op->tile_zlo[t] + 9);
+  if (planes * ZPLANE > (size_t)INT_MAX) return fail(OCTHIP_ERR_UNSUPPORTED, "z-march index tables too large");
+  std::vector<int> rec(planes * ZPLANE);
+  int* r = rec.data();
+  for (size_t t = 0; t < op->tile_zlo.size(); ++t) {
+    if (op->tile_zhi[t] < 0) continue;
+    const long x0 = (long)(t % op->ntx) * ZTX + ZR, y0 = (long)(t / op->ntx) * ZTY + ZR;
+    for (int z = op->tile_zlo[t] - 4; z <= op->tile_zhi[t] + 4; ++z)
+      for (int cy = 0; cy < ZTY; ++cy) {
+        const int* const row = op->mcube.data() + (size_t)op->mx * ((size_t)(y0 + cy) + (size_t)op->my * (size_t)z) + x0;
+        const int* const hrow = row + (long)op->mx * (cy < 4 ? -4 : 4);
+        for (int cx = 0; cx < ZTX; ++cx, r += ZREC) {
+          r[0] = row[cx] + 1;
+          r[1] = row[cx < 4 ? cx - 4 : cx + 4] + 1;
+          r[2] = hrow[cx] + 1;
+        }
+      }
+  }
+  return upload(&op->d_rec, rec.data(), rec.size(), nullptr);
+}
+
+int zmarch_plan(octhip_nl_operator_s* op, int zs, octhip_nl_operator_s::ZPlan** out) {
+  int rc = zmarch_records(op);
+  if (rc) return rc;
   for (auto& pl : op->plans)
     if (pl.zseg == zs) {
-      op->d_items = pl.d_items;
-      op->d_tab = pl.d_tab;
-      op->d_tab_off = pl.d_tab_off;
-      op->items = pl.items;
-      op->nitems = (int)pl.items.size();
-      op->sched = pl.sched;
-      op->sched_len = pl.sched_len;
-      op->zseg_built = zs;
+      *out = &pl;
       return OCTHIP_SUCCESS;
     }
-  std::vector<int4> items;
-  // A tile's z range of len planes is cut into ceil(len / zs) segments of equal length
-  // (+-1), so no item is a short remainder that pays a whole prologue and 8 overlap
-  // planes for a few outputs.  Segment-major, then tile rows: concurrently running items
-  // share halo rows in L2.
-  int maxseg = 0;
-  for (size_t t = 0; t < op->tile_zlo.size(); ++t)
-    if (op->tile_zhi[t] >= 0) maxseg = std::max(maxseg, (op->tile_zhi[t] - op->tile_zlo[t] + zs) / zs);
-  for (int sg = 0; sg < maxseg; ++sg)
-    for (int ty = 0; ty < op->nty; ++ty)
-      for (int tx = 0; tx < op->ntx; ++tx) {
-        const int t = tx + op->ntx * ty;
-        if (op->tile_zhi[t] < 0) continue;
-        const int len = op->tile_zhi[t] - op->tile_zlo[t] + 1;
-        const int n = (len + zs - 1) / zs;
-        if (sg >= n) continue;
-        const int base = len / n, rem = len % n;
-        const int zb = op->tile_zlo[t] + sg * base + std::min(sg, rem);
-        const int ze = zb + base + (sg < rem ? 1 : 0);
-        items.push_back(make_int4(tx, ty, zb, ze));
-      }
-  // Index table of every item, read by the kernel's prologue as one coalesced block: the
-  // point index (or -1) at the ZNC tile columns of planes zb-4 .. ze+3, then at the ZNH
-  // halo sites of the cross-shaped window (the kernel's slot order) of planes zb .. ze-1.
-  std::vector<int> tab, toff(items.size());
-  auto site = [&](long x, long y, long z) {
-    return op->mcube[(size_t)x + (size_t)op->mx * ((size_t)y + (size_t)op->my * (size_t)z)];
-  };
-  for (size_t i = 0; i < items.size(); ++i) {
-    const int4 it = items[i];
-    toff[i] = (int)tab.size();
-    const long x0 = (long)it.x * ZTX + ZR, y0 = (long)it.y * ZTY + ZR;
-    for (int P = it.z - 4; P < it.w + 4; ++P)
-      for (int t = 0; t < ZNC; ++t) tab.push_back(site(x0 + t % ZTX, y0 + t / ZTX, P));
-    for (int P = it.z; P < it.w; ++P)
-      for (int h = 0; h < ZNH; ++h) {
-        long hx, hy;
-        if (h < 4 * ZTY) { hx = x0 - 4 + h % 4; hy = y0 + h / 4; }
-        else if (h < 8 * ZTY) { hx = x0 + ZTX + (h - 4 * ZTY) % 4; hy = y0 + (h - 4 * ZTY) / 4; }
-        else if (h < 8 * ZTY + 4 * ZTX) { hx = x0 + (h - 8 * ZTY) % ZTX; hy = y0 - 4 + (h - 8 * ZTY) / ZTX; }
-        else { hx = x0 + (h - 8 * ZTY - 4 * ZTX) % ZTX; hy = y0 + ZTY + (h - 8 * ZTY - 4 * ZTX) / ZTX; }
-        tab.push_back(site(hx, hy, P));
-      }
-  }
-  if (tab.size() > (size_t)INT_MAX) return fail(OCTHIP_ERR_UNSUPPORTED, "z-march index tables too large");
-  int4* d = nullptr;
-  int* dt = nullptr;
-  int* dto = nullptr;
-  int rc = upload(&d, items.data(), items.size(), nullptr);
-  if (!rc) rc = upload(&dt, tab.data(), tab.size(), nullptr);
-  if (!rc) rc = upload(&dto, toff.data(), toff.size(), nullptr);
-  if (rc) {
-    dfree(d);
-    dfree(dt);
-    dfree(dto);
-    return rc;
-  }
-  op->plans.push_back({zs, d, dt, dto, items, {}, {}});
-  op->d_items = d;
-  op->d_tab = dt;
-  op->d_tab_off = dto;
-  op->items = items;
-  op->nitems = (int)items.size();
-  op->sched.clear();
-  op->sched_len.clear();
-  op->zseg_built = zs;
+  op->plans.push_back({zs, zmarch_items(op, zs), {}});
+  *out = &op->plans.back();
   return OCTHIP_SUCCESS;
 }
 
-// blockIdx -> (item, lane chunk): the (chunk, item) list is cut into 8 contiguous parts,
-// part k runs on XCD k (workgroups are dealt to XCDs round-robin by blockIdx).
-int zmarch_sched(octhip_nl_operator_s* op, int nchunk, const int2** out, int* len) {
-  for (size_t i = 0; i < op->sched.size(); ++i)
-    if (op->sched[i].first == nchunk) {
-      *out = op->sched[i].second;
-      *len = op->sched_len[i];
+// blockIdx -> work item of `all` in order: part k of zmarch_cuts runs on XCD k (workgroups are
+// dealt to XCDs round-robin by blockIdx); entries without planes pad the shorter parts.
+std::vector<int4> zmarch_deal(const std::vector<int4>& all) {
+  std::vector<int> planes;
+  planes.reserve(all.size());
+  for (const int4& e : all) planes.push_back(e.y);
+  const std::vector<size_t> cut = zmarch_cuts(planes);
+  size_t per = 0;
+  for (int x = 0; x < 8; ++x) per = std::max(per, cut[x + 1] - cut[x]);
+  std::vector<int4> sc(per * 8, make_int4(0, 0, 0, 0));
+  for (int x = 0; x < 8; ++x)
+    for (size_t i = cut[x]; i < cut[x + 1]; ++i) sc[(i - cut[x]) * 8 + x] = all[i];
+  return sc;
+}
+
+int zmarch_sched(octhip_nl_operator_s::ZPlan* pl, int nchunk, const int4** out, int* len) {
+  for (const auto& e : pl->sched)
+    if (e.nchunk == nchunk) {
+      *out = e.d;
+      *len = e.len;
       return OCTHIP_SUCCESS;
     }
-  const int n = op->nitems * nchunk;
-  const int per = (n + 7) / 8;
-  std::vector<int2> sc((size_t)per * 8, make_int2(-1, 0));
-  for (int k = 0; k < 8; ++k)
-    for (int i = 0; i < per; ++i) {
-      const int g = k * per + i;
-      if (g >= n) break;
-      sc[(size_t)i * 8 + k] = make_int2(g % op->nitems, g / op->nitems);
-    }
-  int2* d = nullptr;
+  std::vector<int4> all;
+  all.reserve(pl->items.size() * nchunk);
+  for (int c = 0; c < nchunk; ++c)
+    for (const int2& it : pl->items) all.push_back(make_int4(it.x, it.y, c, 0));
+  const std::vector<int4> sc = zmarch_deal(all);
+  int4* d = nullptr;
   int rc = upload(&d, sc.data(), sc.size(), nullptr);
   if (rc) return rc;
-  op->sched.push_back({nchunk, d});
-  op->sched_len.push_back((int)sc.size());
-  for (auto& pl : op->plans)
-    if (pl.zseg == op->zseg_built) {
-      pl.sched = op->sched;
-      pl.sched_len = op->sched_len;
-    }
+  pl->sched.push_back({nchunk, d, (int)sc.size()});
   *out = d;
   *len = (int)sc.size();
   return OCTHIP_SUCCESS;
 }
 
-int launch_zmarch(const ZArgs& z, int lc, int lpt, int epi, int grid, int zseg, hipStream_t s);
+int launch_zmarch(const ZArgs& z, int lc, int lpt, int epi, int grid, hipStream_t s);
 
 // The z-march addresses rows with 32-bit byte offsets: every row array it touches (psi
 // over np_part rows, the outputs over np, the ket rows) must satisfy
@@ -369,6 +377,17 @@ bool zmarch_fits(const octhip_nl_operator_s* op, const ApplyArgs& a) {
   const uint64_t rowb = (uint64_t)a.L * sizeof(double);
   const uint64_t lim = 1ull << 32;
   return (uint64_t)(op->np_part + 1) * rowb <= lim && (!a.kslot || (uint64_t)(a.nk + 1) * rowb <= lim);
+}
+
+// Whether the output rows of a pass are stored non-temporally: unless the next pass reads them
+// (the powers of a Taylor or Krylov chain) and an array of rows is small enough for the 256 MB
+// Infinity Cache to hold what a pass reads and what it writes.  Four passes of a Taylor-4 step,
+// cached against non-temporal: rows of 35 MB 147 against 163 us, 59 MB 247 / 260, 80 MB
+// 289 / 305, 118 MB 436 / 425, 188 MB 694 / 658, 237 MB 881 / 861; a lone apply, whose output
+// nothing reads: 59 MB 50.3 / 49.6 us, 80 MB 53.3 / 50.9, 118 MB 90 / 71, 237 MB 190 / 185.
+constexpr double ZM_CACHED_BYTES = 100e6;
+int zmarch_nt(const octhip_nl_operator_s* op, const ApplyArgs& a) {
+  return a.reuse && (double)op->np * a.L * sizeof(double) <= ZM_CACHED_BYTES ? 0 : 1;
 }
 
 // Build every lazily created device structure an apply with rows of L doubles needs (both
@@ -381,11 +400,12 @@ int prepare_operator(octhip_nl_operator_s* op, int L, bool nl) {
   zmarch_shape(op, L, &lc, &lpt);
   for (int epi : {EPI_STORE, EPI_TAYLOR, EPI_TAYLOR_X}) {
     if (epi != EPI_STORE && lc < 2) continue;
-    int rc = zmarch_items(op, zmarch_zseg_for(op, L, epi, nl));
+    octhip_nl_operator_s::ZPlan* pl = nullptr;
+    int rc = zmarch_plan(op, zmarch_zseg_for(op, L, epi, nl), &pl);
     if (rc) return rc;
-    const int2* sched = nullptr;
+    const int4* sched = nullptr;
     int len = 0;
-    rc = zmarch_sched(op, L / lc, &sched, &len);
+    rc = zmarch_sched(pl, L / lc, &sched, &len);
     if (rc) return rc;
   }
   return OCTHIP_SUCCESS;
@@ -410,23 +430,23 @@ int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t
   if (!zm) return launch_apply(a, op->lattice && a.n > 0, epi, s);
   int lc, lpt;
   zmarch_shape(op, a.L, &lc, &lpt);
-  int rc = zmarch_items(op, zmarch_zseg_for(op, a.L, epi, a.kslot != nullptr));
+  const int zs = zmarch_zseg_for(op, a.L, epi, a.kslot != nullptr);
+  if (zs > zmarch_max_seg(lc))
+    return fail(OCTHIP_ERR_INVALID, "z-march: lane chunk %d with z segment %d needs more than 160 KB of LDS", lc, zs);
+  octhip_nl_operator_s::ZPlan* pl = nullptr;
+  int rc = zmarch_plan(op, zs, &pl);
   if (rc) return rc;
-  if (op->nitems == 0 || a.np <= 0) return OCTHIP_SUCCESS;
-  if (zmarch_shmem(lc, op->zseg_built) > 160 * 1024)
-    return fail(OCTHIP_ERR_INVALID, "z-march: lane chunk %d with z segment %d needs more than 160 KB of LDS", lc,
-                op->zseg_built);
-  const int2* sched = nullptr;
+  if (pl->items.empty() || a.np <= 0) return OCTHIP_SUCCESS;
+  const int4* sched = nullptr;
   int len = 0;
-  rc = zmarch_sched(op, a.L / lc, &sched, &len);
+  rc = zmarch_sched(pl, a.L / lc, &sched, &len);
   if (rc) return rc;
   ZArgs z;
   z.a = a;
-  z.tab = op->d_tab;
-  z.tab_off = op->d_tab_off;
-  z.items = op->d_items;
+  z.a.nt = zmarch_nt(op, a);
+  z.rec = op->d_rec;
   z.sched = sched;
-  return launch_zmarch(z, lc, lpt, epi, len, op->zseg_built, s);
+  return launch_zmarch(z, lc, lpt, epi, len, s);
 }
 }  // namespace octhip
 
@@ -524,15 +544,9 @@ extern "C" int octhip_nl_operator_destroy(octhip_nl_operator_t op) {
   dfree(op->d_cidx);
   dfree(op->d_cube);
   dfree(op->d_dcube);
+  dfree(op->d_rec);
   for (auto& pl : op->plans)
-    if (pl.zseg == op->zseg_built) pl.sched = op->sched;
-  for (auto& pl : op->plans) {
-    dfree(pl.d_items);
-    dfree(pl.d_tab);
-    dfree(pl.d_tab_off);
-    for (auto& e : pl.sched) dfree(e.second);
-  }
-  for (void* p : op->retired) dfree(p);
+    for (auto& e : pl.sched) dfree(e.d);
   dfree(op->d_ri);
   dfree(op->d_rimap);
   for (int part = 0; part < 2; ++part) {

@@ -8,6 +8,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <deque>
 #include <vector>
 
 #include "octhip.h"
@@ -126,32 +127,24 @@ struct octhip_nl_operator_s {
   int zseg = 0;                          // output planes per work item, 0 = chosen per launch
   int lane_chunk = 0;                    // lanes per workgroup (0 = automatic)
   int lanes_per_thread = 0;              // doubles per thread (0 = automatic)
-  int zseg_built = 0;
-  mutable std::vector<int4> zseg_cache;  // automatic segment lengths: {nchunk, lc, resident (+0x100 in a batched launch), zseg}
+  mutable std::vector<int4> zseg_cache;  // automatic segment lengths: {nchunk, lc, resident, zseg}
   std::vector<int> tile_zlo, tile_zhi;   // per tile: inner plane range (cube z), -1 if empty
+  int* d_rec = nullptr;                  // index records of every tile (csrc/zmarch.h)
   int ntx = 0, nty = 0;
-  int4* d_items = nullptr;
-  int* d_tab = nullptr;                  // per item: site -> point index table (planes zb-4 .. ze+3)
-  int* d_tab_off = nullptr;              // per item: first int of its table
-  int nitems = 0;
-  std::vector<int4> items;
-  std::vector<std::pair<int, int2*>> sched;  // lane chunks -> device schedule
-  std::vector<int> sched_len;
-  // item lists built so far, one per segment length (the current one is mirrored in
-  // d_items / nitems / items / sched / zseg_built)
+  // item lists built so far, one per segment length, each with its schedules (one per number
+  // of lane chunks); all stay allocated until destroy: captured graphs and batched launches
+  // may still point at them
+  struct ZSched {
+    int nchunk;
+    int4* d;                             // blockIdx -> {first record plane, planes, lane chunk, 0}
+    int len;
+  };
   struct ZPlan {
     int zseg;
-    int4* d_items;
-    int* d_tab;
-    int* d_tab_off;
-    std::vector<int4> items;
-    std::vector<std::pair<int, int2*>> sched;
-    std::vector<int> sched_len;
+    std::vector<int2> items;             // {first record plane, planes}
+    std::vector<ZSched> sched;
   };
-  std::vector<ZPlan> plans;
-  // device buffers replaced by a rebuild stay allocated until destroy: captured graphs and
-  // batched launches may still point at them
-  std::vector<void*> retired;
+  std::deque<ZPlan> plans;               // a deque: callers keep references
 };
 
 struct octhip_hamiltonian_s {
@@ -184,7 +177,7 @@ struct octhip_hamiltonian_s {
   int* d_proj_mat = nullptr;    // projection index -> matrix
   int nslot = 0;                // mesh points inside at least one sphere
   int nmulti = 0;               // mesh points inside several spheres
-  int* d_kslot = nullptr;       // np: row of the ket buffer for each mesh point, or -1
+  int* d_kslot = nullptr;       // np: row of the ket buffer of each mesh point + 1, or 0
   int* d_multi_pos = nullptr;   // nmulti+1
   int* d_multi_g = nullptr;     // sphere points of the multi-sphere mesh points
   // Work buffers, one set per stream: applies on different streams (Octopus gives every

@@ -1,24 +1,32 @@
 // 2.5-D "z-march" apply for the order-4 star stencil on a lattice (gfx950).
 //
 // The gather kernel (k_apply) reads 25 full rows per point, so L2 has to deliver 25x the
-// HBM traffic.  Here a workgroup owns a ZM_TX x ZM_TY tile of lattice columns (8x8 by
-// default) and one chunk of LC lanes, and walks a segment of the tile's z range plane by
-// plane:
+// HBM traffic.  Here a workgroup owns an 8x8 tile of lattice columns and one chunk of LC
+// lanes, and walks a segment of the tile's z range plane by plane:
 //   * the current plane (tile + 4-site halo strips on the four sides) is staged in LDS
-//     (double-buffered): x and y neighbours are LDS reads;
-//   * each thread keeps its column's values at z-4..z+4 in registers: z neighbours cost
-//     nothing;
-//   * the site -> point indices of the item (precomputed per item on the host) and the
-//     ket slots of its own sites are staged in LDS once per item;
-//   * loads run a few planes ahead (own column values, halo values, and the potential,
-//     ket row and Taylor accumulator of the output point; depths in ZRings), into ring buffers
-//     with compile-time slots (the z loop is unrolled by the ring period); every load is
-//     unconditional, so the compiler's wait counts stay exact and a step waits only on
-//     loads issued planes earlier.
-// Per output point an 8x8 tile reads 1 own row chunk + 2 halo chunks (128 halo sites for
-// 64 columns) instead of 25 rows; rows go through raw buffer resources (below).  The lattice is a padded "march cube" of point indices;
-// sites that are not points hold -1.  Values follow the gather kernel exactly: point
-// q < lim -> its row, anything else -> 0, and the 25 terms are summed in stencil order
+//     (double-buffered) as a dense 16x16 window, so that the 16 x and y neighbours of a
+//     thread are one base address and compile-time offsets;
+//   * z neighbours never leave the registers: a thread keeps its column's values of the 4
+//     planes behind, and one partial sum for each of the 4 planes behind.  When plane z
+//     arrives it starts its own sum (x and y terms, then z-4..z-1) and adds the +1..+4
+//     terms to the four sums behind it; the sum of plane z-4 is then complete.  The terms of
+//     every sum still arrive in stencil order, and a plane's own values and its halo are
+//     needed at the same step: neighbouring tiles, which run side by side on one XCD, read
+//     each other's rows while they are in its L2 (keeping z-4..z+4 resident instead loads a
+//     column's own values three planes before its neighbours load them as halo);
+//   * the site -> point indices (own column and two halo sites per column) are one 12-byte
+//     record per column and plane, loaded a plane ahead of the rows they address;
+//   * loads run ahead (depths in ZDepth) in rings with compile-time slots (the z loop is
+//     unrolled by 8); every load but the ket rows is unconditional, so the compiler's wait
+//     counts stay exact and a step waits only on loads of the steps before it.
+// What bounds it (462,781 points, 32 complex states, H-apply with projectors: 163 us, 518 MB
+// read and 237 MB written for 289 + 237 MB of rows): 102 us go to the LDS reads (16 rows of 16
+// bytes per output) and the vector memory instructions alone, with every row out of range, and
+// the memory traffic overlaps with them only in part.  Measured and not kept: rows two or three
+// planes ahead (+1 to +4%), a quad of 2x2 columns per thread (half the LDS reads; 8-byte loads,
+// 215-237 us), 8-lane chunks (257 us), the lane chunks of an item side by side (177-200 us).
+// Rows go through raw buffer resources (below).  Values follow the gather kernel exactly:
+// point q < lim -> its row, anything else -> 0, and the 25 terms are summed in stencil order
 // (x -4..4, y -4..-1,1..4, z -4..-1,1..4) with fma, so results are bit-identical to it.
 #pragma once
 
@@ -26,45 +34,27 @@
 
 namespace octhip {
 
-#ifndef ZM_TX
-#define ZM_TX 8
-#endif
-#ifndef ZM_TY
-#define ZM_TY 8
-#endif
-constexpr int ZTX = ZM_TX;            // tile columns along x
-constexpr int ZTY = ZM_TY;            // tile columns along y
+constexpr int ZTX = 8, ZTY = 8;       // tile columns along x and y
 constexpr int ZR = 4;                 // stencil reach
 constexpr int ZNC = ZTX * ZTY;        // own columns of a tile
-constexpr int ZNH = 8 * (ZTX + ZTY);  // halo sites of the cross-shaped plane window
-constexpr int ZS = ZNC + ZNH;         // sites of the plane window
-constexpr int ZHU = (ZNH + ZNC - 1) / ZNC;  // halo sites loaded per column thread group
-static_assert((ZTX & (ZTX - 1)) == 0 && (ZTY & (ZTY - 1)) == 0 && ZS % 4 == 0, "tile shape");
+constexpr int ZHU = 2;                // halo sites per column: 128 for 64 columns
+constexpr int ZW = ZTX + 2 * ZR;      // window row length (x)
+constexpr int ZS = ZW * (ZTY + 2 * ZR);  // site slots of the window (the 4x4 corners stay unused)
+// march-cube padding below/above the inner points in z
 constexpr int ZPADZ = 8;
-// ints of the index table of an item of zs planes: own columns of zs + 8 planes, halo sites
-// of zs planes (a multiple of 4: the table is copied as int4)
-__host__ __device__ constexpr int zmarch_tab_ints(int zs) { return (zs + 8) * ZNC + zs * ZNH; }
-static_assert(ZNC % 4 == 0 && ZNH % 4 == 0, "index table copied as int4");             // march-cube padding below/above the inner points in z
-// Prefetch depths (planes loaded ahead) of the own column values, the halo values and the
-// output-point data, and the own-value ring length (= z loop unroll, >= own depth + 5).
-// A tile's own values of plane P are the halo of its neighbours, which load them HD
-// planes ahead of P, against own-depth planes ahead here: the smaller that gap, the more
-// of the halo reads hit in L2 (own 5 rather than 6 for the plain store: 2% less time on
-// the R=12 sphere).  The Taylor epilogue carries an accumulator row per plane more, so it
-// takes shallow rings (127 VGPRs: two 512-thread workgroups per CU, whose loads cover each
-// other's latency; 2.3% faster Taylor steps than with the deep rings at 143 VGPRs); the
-// plain store keeps two planes of halo and point data (126 VGPRs with ket rows, still two
-// per CU; the shallow ones cost the 8-lane Laplacian 12%).
+// Index records of a tile: for every plane from 4 below to 4 above its inner points and every
+// column, {own, halo 0, halo 1, 0} as point index + 1 (0: no point).  Column (cx, cy) carries the
+// halo sites (cx < 4 ? cx - 4 : cx + 4, cy) and (cx, cy < 4 ? cy - 4 : cy + 4) of the tile.
+constexpr int ZREC = 4;               // ints per record
+constexpr int ZPLANE = ZREC * ZNC;    // ints per plane of a tile
+
+// Prefetch depths in planes: rows (own and halo values) and output-point data (potential,
+// ket row, Taylor rows).  One plane each: 85-103 VGPRs, two 512-thread workgroups per CU; deeper
+// rings measured slower (rows 2: 166 against 163 us, output-point data 2: 163).
 template <int EPI>
-struct ZRings {
-  static constexpr int own = 5, halo = 2, aux = 2, ring = 12;
+struct ZDepth {
+  static constexpr int rows = 1, aux = 1;
 };
-template <>
-struct ZRings<EPI_TAYLOR> {
-  static constexpr int own = 5, halo = 1, aux = 1, ring = 10;
-};
-template <>
-struct ZRings<EPI_TAYLOR_X> : ZRings<EPI_TAYLOR> {};
 
 // Raw buffer resources over the row arrays (gfx9 range checking, stride 0): a load whose
 // byte offset lies at or beyond num_records returns zeros and such a store is dropped.
@@ -88,61 +78,56 @@ __device__ __forceinline__ Vec<LPT> bld(__amdgpu_buffer_rsrc_t r, uint32_t off) 
   }
   return v;
 }
-// Stores are marked non-temporal (cache policy NT): output rows are not read again in
-// the pass, and keeping them out of the way leaves the XCD's L2 to the input rows that
-// the neighbouring tiles read a few planes later as their halo (7% less read traffic and
-// 4% less time for the H-apply pass on the R=12 sphere).
+// Stores of output rows, cached or non-temporal (cache policy NT).  Rows that the next pass
+// finds in the 256 MB Infinity Cache are stored cached; beyond that, non-temporal stores leave
+// the XCD's L2 to the input rows that the neighbouring tiles read as their halo (see
+// zmarch_nt in nl_operator.hip for the line between them).
 constexpr int ZM_STORE_NT = 2;  // cache-policy operand: NT
 template <int LPT>
-__device__ __forceinline__ void bst(__amdgpu_buffer_rsrc_t r, uint32_t off, const Vec<LPT>& v) {
+__device__ __forceinline__ void bst(__amdgpu_buffer_rsrc_t r, uint32_t off, const Vec<LPT>& v, bool nt) {
   if constexpr (LPT == 2) {
     using U4 = decltype(__builtin_amdgcn_raw_buffer_load_b128(r, 0, 0, 0));
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, make_double2(v.v[0], v.v[1])), r, off, 0,
-                                           ZM_STORE_NT);
+    const U4 u = __builtin_bit_cast(U4, make_double2(v.v[0], v.v[1]));
+    if (nt) __builtin_amdgcn_raw_buffer_store_b128(u, r, off, 0, ZM_STORE_NT);
+    else __builtin_amdgcn_raw_buffer_store_b128(u, r, off, 0, 0);
   } else {
     using U2 = decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v.v[0]), r, off, 0, ZM_STORE_NT);
+    const U2 u = __builtin_bit_cast(U2, v.v[0]);
+    if (nt) __builtin_amdgcn_raw_buffer_store_b64(u, r, off, 0, ZM_STORE_NT);
+    else __builtin_amdgcn_raw_buffer_store_b64(u, r, off, 0, 0);
   }
 }
 
-// smallest divisor of rq above d: the length of a prefetch ring d planes deep whose slots
-// stay compile-time constants in a z loop unrolled rq times
-constexpr int ring_above(int rq, int d) {
-  for (int r = d + 1; r < rq; ++r)
-    if (rq % r == 0) return r;
-  return rq;
+// What the threads of a column share (its record, its potential) is loaded as one dword per lane
+// and handed round within each quad of lanes by DPP: a dword load occupies the vector memory
+// unit 4 cycles instead of 12 or 8 (with the ket rows skipped where a wave has none, 81 cycles
+// per plane and wave instead of 104: 462,781 points, 32 states 172 -> 163 us, 155,331 points
+// 49 -> 47 us).
+template <int K>
+__device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {  // lane K of each quad of lanes
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, K * 0x55, 0xf, 0xf, true);
 }
 
 struct ZArgs {
   ApplyArgs a;
-  const int4* __restrict__ items;    // {tile x, tile y, first plane, end plane} (cube z)
-  const int* __restrict__ tab;       // per item: index table (zmarch_tab_ints ints, layout below)
-  const int* __restrict__ tab_off;   // per item: first int of its table (a multiple of 4)
-  const int2* __restrict__ sched;    // blockIdx -> {item, lane chunk}
+  const int* __restrict__ rec;       // index records of every tile (ZREC ints each)
+  const int4* __restrict__ sched;    // blockIdx -> {first record plane, planes, lane chunk, -}
 };
 
-// One work item: tile it = {tile x, tile y, first plane, end plane}, lane chunk `chunk`.
+// One work item: `n` output planes of a tile, whose index records start (4 planes below the
+// first output plane) at plane rec0 of the table; lane chunk `chunk`.
 // za may live in kernel arguments (single operator) or in global memory (one descriptor
 // per system of a batched launch): every field is copied to a local once.
-// SHALLOW: the shallow prefetch rings whatever the epilogue (the batched instances, whose
-// descriptor handling costs a few registers more).
-template <int LPT, int LC, int EPI, bool NL, bool SHALLOW = false>
-__device__ __forceinline__ void zmarch_body(const ZArgs& za, const int4 it, const int item, const int chunk) {
+template <int LPT, int LC, int EPI, bool NL>
+__device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, const int n, const int chunk) {
   constexpr int PAIRS = LC / LPT;    // threads per column
-  constexpr int NT = ZNC * PAIRS;
   extern __shared__ double2 zsh2[];  // 16-byte aligned: row chunks move as ds_*_b128
   double* const zsh = reinterpret_cast<double*>(zsh2);
-  double* const lds0 = zsh;                              // plane buffer 0
-  double* const lds1 = zsh + ZS * LC;                    // plane buffer 1
-  int* const tidx = reinterpret_cast<int*>(zsh + 2 * ZS * LC);  // item index table
   const ApplyArgs& A = za.a;
   const int a_np = A.np;
   const double* const a_v = A.v;
-  const int* const a_kslot = A.kslot;
   double* const a_acc = A.acc;
-  const double a_c1r = A.c1r, a_c1i = A.c1i, a_c2r = A.c2r, a_c2i = A.c2i;
-  const int a_has_c1 = A.has_c1;
-  const double a_car = A.car, a_cai = A.cai, a_cbr = A.cbr, a_cbi = A.cbi;
+  const bool a_nt = A.nt != 0;
   double a_w[25];
 #pragma unroll
   for (int j = 0; j < 25; ++j) a_w[j] = A.w[j];
@@ -154,304 +139,274 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int4 it, cons
   const bool has_acc = TAY && a_acc != nullptr;
   // row q of an array starts at byte q << sh; arrays without a role here get no records
   const int sh = __builtin_ctz((unsigned)A.L) + 3;
-  const uint32_t lbyte = (uint32_t)l * 8u;
   const uint32_t np_bytes = (uint32_t)a_np << sh;
   const auto r_fi = zrsrc(A.fi, (uint32_t)A.lim << sh);
   const auto r_v = zrsrc(a_v, a_v ? (uint32_t)a_np * 8u : 0u);
+  const auto r_ks = zrsrc(A.kslot, NL ? (uint32_t)a_np * 4u : 0u);
   const auto r_k = zrsrc(A.ksum, NL ? (uint32_t)A.nk << sh : 0u);
   const auto r_ai = zrsrc(A.acc_in ? A.acc_in : a_acc, has_acc ? np_bytes : 0u);
   const auto r_fo = zrsrc(A.fo, EPI == EPI_STORE ? np_bytes : 0u);
-  const auto r_y = zrsrc(A.yout, A.yout ? np_bytes : 0u);
+  const auto r_y = zrsrc(A.yout, (TAY && A.yout) ? np_bytes : 0u);
   const auto r_acc = zrsrc(a_acc, has_acc ? np_bytes : 0u);
   const auto r_ya = zrsrc(A.ya, (has_acc && A.ya) ? np_bytes : 0u);  // earlier powers, last order
   const auto r_yb = zrsrc(A.yb, (has_acc && A.yb) ? np_bytes : 0u);
   // EPI_TAYLOR_X: second accumulator and density partials of this thread's state
   const auto r_a2 = zrsrc(A.acc2, (EPI == EPI_TAYLOR_X && has_acc && A.acc2) ? np_bytes : 0u);
-  double* const a_dpart = EPI == EPI_TAYLOR_X ? A.dpart : nullptr;
+  const auto r_dp = zrsrc(EPI == EPI_TAYLOR_X && A.dpart ? A.dpart + (size_t)chunk * a_np : nullptr,
+                          (EPI == EPI_TAYLOR_X && has_acc && A.dpart) ? (uint32_t)a_np * 8u : 0u);
   const double wl = (EPI == EPI_TAYLOR_X && A.dw) ? A.dw[l >> 1] : 0.0;
-  auto roff = [&](int q) { return ((uint32_t)q << sh) + lbyte; };
-  // halo units of this thread: halo site h = col + ZNC*i (if h < ZNH), same lane pair
-  int hlds[ZHU];
+  const auto r_rec = zrsrc(za.rec + (size_t)rec0 * ZPLANE, (uint32_t)(n + 8) * (uint32_t)(ZPLANE * 4));
+  // byte offset of this thread's lanes of row q1 - 1; q1 = 0 (no point) falls out of range
+  const uint32_t lrow = (uint32_t)l * 8u - (1u << sh);
+  auto roff = [&](uint32_t q1) { return (q1 << sh) + lrow; };
+  // byte offset of that point in an array of 2^b bytes per point
+  auto poff = [&](uint32_t ro, int b) { return ((ro - lrow) >> (sh - b)) - (1u << b); };
+  constexpr uint32_t NONE = ~0u - 7u;  // out of range of the arrays of 4 or 8 bytes per point
+  // window slots, in doubles, from the window's corner (so that every offset is positive)
+  const int corner = (cy * ZW + cx) * LC + kp * LPT;
+  constexpr int own_lds = (ZR * ZW + ZR) * LC;
+  const int hx_lds = ((cy + ZR) * ZW + (cx < 4 ? cx : cx + 8)) * LC + kp * LPT;
+  const int hy_lds = ((cy < 4 ? cy : cy + 8) * ZW + cx + ZR) * LC + kp * LPT;
+
+  constexpr int RD = ZDepth<EPI>::rows, AD = ZDepth<EPI>::aux;
+  static_assert(RD >= 1 && RD <= 3 && AD >= 1 && AD <= 3, "prefetch depths");
+  // rings, plane P (relative to the first output plane) in slot P mod the ring length:
+  //   ov   own values, P in z-4 .. z+RD;    hv  halo values, P in z .. z+RD
+  //   part partial sums, P in z-4 .. z-1;   ro  own row offsets, P in z-4 .. z+RD
+  //   rec  index records, P in z+RD .. z+RD+2
+  //   vr/kr/ar/ra/rb output-point data, P in z-4 .. z-4+AD;  ks  ket slots, P in z-4+AD .. z-3+AD
+  struct Rec {
+    uint32_t v[PAIRS >= 4 ? 1 : 3];
+  };
+  Vec<LPT> ov[8], hv[4][ZHU], part[4];
+  uint32_t ro[8], ks[4] = {0u, 0u, 0u, 0u};
+  Rec rec[4];
+  double vr[4];
+  uint32_t vd[4];  // QUAD: half of the potential per lane
+  Vec<LPT> kr[4], ar[TAY ? 4 : 1], ra[TAY ? 4 : 1], rb[TAY ? 4 : 1];
 #pragma unroll
-  for (int i = 0; i < ZHU; ++i) hlds[i] = (ZNC + col + ZNC * i) * LC + kp * LPT;
-  auto halo_ok = [&](int i) { return ZNC * (i + 1) <= ZNH || col + ZNC * i < ZNH; };
-  // Cross-shaped window in LDS, one LC-lane chunk per site slot ((x0, y0) = first tile
-  // column, W = ZTX, H = ZTY, N = W H):
-  //   slot c (0..N-1)               tile column c = cx + W cy
-  //   slot N + 4 r + k              left strip,   x = x0-4+k, y = y0+r   (k < 4, r < H)
-  //   slot N + 4 H + 4 r + k        right strip,  x = x0+W+k, y = y0+r
-  //   slot N + 8 H + W k + c        bottom strip, x = x0+c,   y = y0-4+k (c < W)
-  //   slot N + 8 H + 4 W + W k + c  top strip,    x = x0+c,   y = y0+H+k
-  const int own_lds = col * LC + kp * LPT;
-  auto xnb = [&](int dx) {  // LDS offset of the x-neighbour dx of this thread's column
-    const int xx = cx + dx;
-    const int slot = xx < 0 ? ZNC + 4 * cy + (xx + 4)
-                            : (xx >= ZTX ? ZNC + 4 * ZTY + 4 * cy + (xx - ZTX) : xx + ZTX * cy);
-    return slot * LC + kp * LPT;
+  for (int k = 0; k < 4; ++k) {
+    vr[k] = 0.0;
+    vd[k] = 0u;
+#pragma unroll
+    for (int i = 0; i < LPT; ++i) part[k].v[i] = kr[k].v[i] = 0.0;
+  }
+  // a quad's lanes share one column when it has at least 4 threads
+  constexpr bool QUAD = PAIRS >= 4;
+  // record of plane P (planes past the last record read 0)
+  auto load_rec = [&](int P) -> Rec {
+    Rec r;
+    const uint32_t o = (uint32_t)((P + 4) * ZNC + col) * (ZREC * 4u);
+    if constexpr (QUAD) {
+      r.v[0] = __builtin_amdgcn_raw_buffer_load_b32(r_rec, o + (threadIdx.x & 3) * 4u, 0, 0);
+    } else {
+      const auto v = __builtin_amdgcn_raw_buffer_load_b96(r_rec, o, 0, 0);
+      for (int k = 0; k < 3; ++k) r.v[k] = v[k];
+    }
+    return r;
   };
-  auto ynb = [&](int dy) {  // LDS offset of the y-neighbour dy
-    const int yy = cy + dy;
-    const int slot = yy < 0 ? ZNC + 8 * ZTY + ZTX * (yy + 4) + cx
-                            : (yy >= ZTY ? ZNC + 8 * ZTY + 4 * ZTX + ZTX * (yy - ZTY) + cx : cx + ZTX * yy);
-    return slot * LC + kp * LPT;
+  auto own_row = [&](const Rec& r) {
+    if constexpr (QUAD) return quad_bcast<0>(r.v[0] << sh) + lrow;
+    else return roff(r.v[0]);
   };
-
-  // value of point q (zero for boundary/non-points when q >= lim or q = -1)
-  auto val = [&](int q) { return bld<LPT>(r_fi, roff(q)); };
-  auto lds_st = [&](int buf, int off, const Vec<LPT>& v) {
-    double* b = buf ? lds1 : lds0;
-    stv<LPT>(b + off, v);
+  // halo rows, of output planes only
+  auto halo_row = [&](const Rec& r, int P, int i) {
+    const bool in = P >= 0 && P < n;
+    if constexpr (QUAD) {
+      const uint32_t o = (in ? r.v[0] : 0u) << sh;
+      return (i ? quad_bcast<2>(o) : quad_bcast<1>(o)) + lrow;
+    } else {
+      return in ? roff(r.v[1 + i]) : lrow;
+    }
   };
-  auto lds_ld = [&](int buf, int off) {
-    const double* b = buf ? lds1 : lds0;
-    return ldv<LPT>(b + off);
-  };
-
-  const int zb = it.z, ze = it.w;
-  // ---- index table of the item in LDS: the ZNC own columns of planes zb-4 .. ze+3, then
-  //      the ZNH halo sites of planes zb .. ze-1 (the only planes whose halo is read).
-  //      Precomputed per item, so the prologue is one coalesced block copy; index reads
-  //      then cost LDS, not the in-order global-load counter.
-  const int nown = (ze - zb + 8) * ZNC;
-  int* const tks = tidx + nown + (ze - zb) * ZNH;  // ket slots of the own sites
   {
-    // (through a buffer resource: the descriptors of a batched launch live in global
-    // memory, and a generic pointer loaded from there would be read with flat loads that
-    // the compiler must order against the LDS stores)
-    const int n4 = zmarch_tab_ints(ze - zb) / 4;
-    const auto r_tab = zrsrc(za.tab + za.tab_off[item], (uint32_t)n4 * 16u);
-    int4* const t4 = reinterpret_cast<int4*>(tidx);
-    for (int base = 0; base < n4; base += NT * 8) {
-      int4 tq[8];
+    Rec r0[4 + RD];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = base + threadIdx.x + u * NT;
-        tq[u] = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(r_tab, (uint32_t)e * 16u, 0, 0));
-      }
+    for (int P = -4; P < RD; ++P) r0[P + 4] = load_rec(P);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = base + threadIdx.x + u * NT;
-        if (e < n4) t4[e] = tq[u];
-      }
+    for (int P = RD; P < RD + 2; ++P) rec[P & 3] = load_rec(P);
+#pragma unroll
+    for (int P = -4; P < RD; ++P) {
+      ro[P & 7] = own_row(r0[P + 4]);
+      ov[P & 7] = bld<LPT>(r_fi, ro[P & 7]);
     }
+#pragma unroll
+    for (int P = 0; P < RD; ++P)
+#pragma unroll
+      for (int i = 0; i < ZHU; ++i) hv[P & 3][i] = bld<LPT>(r_fi, halo_row(r0[P + 4], P, i));
   }
-  __syncthreads();
-  auto own_idx = [&](int P) { return tidx[(P - zb + 4) * ZNC + col]; };
-  // (zb <= P < ze)
-  auto halo_idx = [&](int P, int i) { return halo_ok(i) ? tidx[nown + (P - zb) * ZNH + col + ZNC * i] : -1; };
-
-  // Rings with static slots (the z loop is unrolled by RQ, so every slot index is a
-  // compile-time constant and values stay in the registers their loads wrote):
-  //   ov[(P - zb + 4) % RQ]  own value of plane P,  P in z-4 .. z+OA (loaded OA planes ahead)
-  //   hv[(P - zb) % HR]      halo values of plane P, P in z .. z+HD (loaded HD planes ahead)
-  //   vr/kr/ar[(P - zb) % AR] output point data,     P in z .. z+AD (loaded AD planes ahead)
-  // The load counter retires in order, so the shortest distance sets how many planes of
-  // loads stay in flight: halo and point data go as deep as the own values allow.
-  using Rings = ZRings<SHALLOW ? EPI_TAYLOR : EPI>;
-  constexpr int RQ = Rings::ring, OA = Rings::own;
-  constexpr int HD = Rings::halo, AD = Rings::aux;
-  constexpr int HR = ring_above(RQ, HD);  // ring sizes dividing RQ
-  constexpr int AR = ring_above(RQ, AD);
-  static_assert(OA >= 5 && RQ >= OA + 5 && HR > HD && AR > AD, "ring sizes");
-  Vec<LPT> ov[RQ];
-  Vec<LPT> hv[HR][ZHU];
-  double vr[AR] = {};
-  Vec<LPT> kr[AR];
-  Vec<LPT> ar[AR];
-  Vec<LPT> ra[TAY ? AR : 1], rb[TAY ? AR : 1];
-  // Every global load below is issued unconditionally (out-of-range requests read zeros):
-  // with loads behind branches the compiler cannot count the loads still in flight and
-  // drains the whole prefetch queue at every plane.
-  // per-point data of plane P (< ze + 4) for its output point: potential, ket sum row,
-  // accumulator row
-  auto load_aux = [&](int slot, int P) {
-    const int q = own_idx(P);
-    const int qo = (P < ze && (unsigned)q < (unsigned)a_np) ? q : -1;
-    vr[slot] = bld<1>(r_v, (uint32_t)qo << 3).v[0];
-    if constexpr (NL) {
-      const int ks = tks[(P - zb + 4) * ZNC + col];
-      kr[slot] = bld<LPT>(r_k, roff(qo >= 0 ? ks : -1));
-    }
-    if constexpr (TAY) {
-      ar[slot] = bld<LPT>(r_ai, roff(qo));
-      ra[slot] = bld<LPT>(r_ya, roff(qo));  // zeros (no memory access) without ya / yb
-      rb[slot] = bld<LPT>(r_yb, roff(qo));
-    }
-  };
+  const int zend = n + 4;
+#pragma nounroll
+  for (int z0 = 0; z0 < zend; z0 += 8) {
 #pragma unroll
-  for (int k = 0; k < OA + 4; ++k) ov[k] = val(zb - 4 + k < ze + 4 ? own_idx(zb - 4 + k) : -1);
-#pragma unroll
-  for (int k = 0; k < HD; ++k)
-#pragma unroll
-    for (int i = 0; i < ZHU; ++i) hv[k][i] = val(zb + k < ze ? halo_idx(zb + k, i) : -1);
-  // ket slots of the own sites of the output planes zb .. ze-1 (entries (P - zb + 4) ZNC +
-  // col, as the own indices), looked up while the first planes' values are in flight (one
-  // unconditional range-checked load per entry; -1 where the site has no point)
-  if constexpr (NL) {
-    const auto r_ks = zrsrc(a_kslot, (uint32_t)a_np * 4u);
-    const int totk = (ze - zb + 4) * ZNC;
-    for (int base = 4 * ZNC; base < totk; base += NT * 8) {
-      int kq[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = min(base + (int)threadIdx.x + u * NT, totk - 1);
-        const int q = tidx[e];
-        const int k = (int)__builtin_amdgcn_raw_buffer_load_b32(r_ks, (uint32_t)q << 2, 0, 0);
-        kq[u] = (unsigned)q < (unsigned)a_np ? k : -1;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = base + threadIdx.x + u * NT;
-        if (e < totk) tks[e] = kq[u];
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int k = 0; k < AD; ++k) load_aux(k, zb + k);
-
-  for (int z0 = zb; z0 < ze; z0 += RQ) {
-#pragma unroll
-    for (int kk = 0; kk < RQ; ++kk) {
+    for (int kk = 0; kk < 8; ++kk) {
       const int z = z0 + kk;
-      if (z >= ze) break;
-      const int buf = kk & 1;
-      // prefetch: output-point data of plane z+AD, own column z+OA, halo of plane z+HD
-      load_aux((kk + AD) % AR, z + AD);
-      ov[(kk + 4 + OA) % RQ] = val(z + OA < ze + 4 ? own_idx(z + OA) : -1);
+      if (z >= zend) return;
+      // row of plane z - 4, completed in this step (stores outside the item are dropped)
+      const uint32_t qo = z >= 4 ? ro[(kk + 4) & 7] : lrow;
+      // ---- stage plane z
+      const Vec<LPT> xz = ov[kk & 7];        // own values of planes z and z - 4
+      const Vec<LPT> xf = ov[(kk + 4) & 7];
+      double* const win = zsh + (kk & 1) * (ZS * LC);
+      stv<LPT>(win + corner + own_lds, xz);
+      stv<LPT>(win + hx_lds, hv[kk & 3][0]);
+      stv<LPT>(win + hy_lds, hv[kk & 3][1]);
+      // ---- the +1..+4 terms of the planes behind; plane z - 4 is complete
+      Vec<LPT> s = part[kk & 3];
 #pragma unroll
-      for (int i = 0; i < ZHU; ++i) hv[(kk + HD) % HR][i] = val(z + HD < ze ? halo_idx(z + HD, i) : -1);
-      // stage plane z: tile centre and halo strips
-      lds_st(buf, own_lds, ov[(kk + 4) % RQ]);
+      for (int k = 0; k < LPT; ++k) {
+        s.v[k] = fma(a_w[24], xz.v[k], s.v[k]);
 #pragma unroll
-      for (int i = 0; i < ZHU; ++i)
-        if (halo_ok(i)) lds_st(buf, hlds[i], hv[kk % HR][i]);
-      __syncthreads();
-      // output point (x0+cx, y0+cy, z)
-      const int q0 = own_idx(z);
-      if ((unsigned)q0 < (unsigned)a_np) {
-        Vec<LPT> s;
-#pragma unroll
-        for (int k = 0; k < LPT; ++k) s.v[k] = 0.0;
-#pragma unroll
-        for (int j = 0; j < 25; ++j) {
-          Vec<LPT> x;
-          if (j < 9) {
-            const int dx = j - 4;
-            x = (dx == 0) ? ov[(kk + 4) % RQ] : lds_ld(buf, xnb(dx));
-          } else if (j < 17) {
-            const int dy = (j < 13) ? j - 13 : j - 12;
-            x = lds_ld(buf, ynb(dy));
-          } else {
-            const int dz = (j < 21) ? j - 21 : j - 20;
-            x = ov[(kk + 4 + dz + RQ) % RQ];
-          }
-#pragma unroll
-          for (int k = 0; k < LPT; ++k) s.v[k] = fma(a_w[j], x.v[k], s.v[k]);
-        }
-        const Vec<LPT> x = ov[(kk + 4) % RQ];
+        for (int d = 1; d < 4; ++d)
+          part[(kk - d) & 3].v[k] = fma(a_w[20 + d], xz.v[k], part[(kk - d) & 3].v[k]);
+      }
+      {
         if (a_v) {
-          const double vv = vr[kk % AR];
+          double vv = vr[kk & 3];
+          if constexpr (QUAD)
+            vv = __builtin_bit_cast(double, (uint64_t)quad_bcast<1>(vd[kk & 3]) << 32 | quad_bcast<0>(vd[kk & 3]));
 #pragma unroll
-          for (int k = 0; k < LPT; ++k) s.v[k] = fma(vv, x.v[k], s.v[k]);
+          for (int k = 0; k < LPT; ++k) s.v[k] = fma(vv, xf.v[k], s.v[k]);
         }
         if constexpr (NL) {
 #pragma unroll
-          for (int k = 0; k < LPT; ++k) s.v[k] = s.v[k] + kr[kk % AR].v[k];
+          for (int k = 0; k < LPT; ++k) s.v[k] = s.v[k] + kr[kk & 3].v[k];
         }
         if constexpr (EPI == EPI_STORE) {
-          bst<LPT>(r_fo, roff(q0), s);
+          bst<LPT>(r_fo, qo, s, a_nt);
         } else {
-          bst<LPT>(r_y, roff(q0), s);  // dropped when there is no yout
-          if (has_acc) {
-            Vec<LPT> av = ar[kk % AR];
-            const Vec<LPT> ua = ra[kk % AR], ub = rb[kk % AR];
+          bst<LPT>(r_y, qo, s, a_nt);  // dropped when there is no yout
+          Vec<LPT> av = ar[kk & 3];
+          const Vec<LPT> ua = ra[kk & 3], ub = rb[kk & 3];
+          // the other lane of each (re, im) pair: in this thread, or the neighbouring one
+          auto add = [&](Vec<LPT>& y, double zr, double zi, const Vec<LPT>& x) {
             if constexpr (LPT == 2) {
-              av.v[0] = av.v[0] + zmul_lane(a_car, a_cai, ua.v[0], ua.v[1], false);
-              av.v[1] = av.v[1] + zmul_lane(a_car, a_cai, ua.v[1], ua.v[0], true);
-              av.v[0] = av.v[0] + zmul_lane(a_cbr, a_cbi, ub.v[0], ub.v[1], false);
-              av.v[1] = av.v[1] + zmul_lane(a_cbr, a_cbi, ub.v[1], ub.v[0], true);
-              if (a_has_c1) {
-                av.v[0] = av.v[0] + zmul_lane(a_c1r, a_c1i, x.v[0], x.v[1], false);
-                av.v[1] = av.v[1] + zmul_lane(a_c1r, a_c1i, x.v[1], x.v[0], true);
-              }
-              av.v[0] = av.v[0] + zmul_lane(a_c2r, a_c2i, s.v[0], s.v[1], false);
-              av.v[1] = av.v[1] + zmul_lane(a_c2r, a_c2i, s.v[1], s.v[0], true);
+              const double re = zmul_lane(zr, zi, x.v[0], x.v[1], false);
+              const double im = zmul_lane(zr, zi, x.v[1], x.v[0], true);
+              y.v[0] = y.v[0] + re;
+              y.v[1] = y.v[1] + im;
             } else {
-              // the partner lane of a (re, im) pair is held by the neighbouring thread
-              const bool odd = (l & 1) != 0;
-              av.v[0] = av.v[0] + zmul_lane(a_car, a_cai, ua.v[0], __shfl_xor(ua.v[0], 1), odd);
-              av.v[0] = av.v[0] + zmul_lane(a_cbr, a_cbi, ub.v[0], __shfl_xor(ub.v[0], 1), odd);
-              if (a_has_c1) av.v[0] = av.v[0] + zmul_lane(a_c1r, a_c1i, x.v[0], __shfl_xor(x.v[0], 1), odd);
-              av.v[0] = av.v[0] + zmul_lane(a_c2r, a_c2i, s.v[0], __shfl_xor(s.v[0], 1), odd);
+              y.v[0] = y.v[0] + zmul_lane(zr, zi, x.v[0], __shfl_xor(x.v[0], 1), (l & 1) != 0);
             }
-            bst<LPT>(r_acc, roff(q0), av);
-            if constexpr (EPI == EPI_TAYLOR_X) {
-              Vec<LPT> dv = av;
-              if (A.acc2) {
-                // psib2: the same terms with the deltat2 factors, from the same base
-                Vec<LPT> a2 = ar[kk % AR];
-                if constexpr (LPT == 2) {
-                  a2.v[0] = a2.v[0] + zmul_lane(A.dar, A.dai, ua.v[0], ua.v[1], false);
-                  a2.v[1] = a2.v[1] + zmul_lane(A.dar, A.dai, ua.v[1], ua.v[0], true);
-                  a2.v[0] = a2.v[0] + zmul_lane(A.dbr, A.dbi, ub.v[0], ub.v[1], false);
-                  a2.v[1] = a2.v[1] + zmul_lane(A.dbr, A.dbi, ub.v[1], ub.v[0], true);
-                  if (a_has_c1) {
-                    a2.v[0] = a2.v[0] + zmul_lane(A.d1r, A.d1i, x.v[0], x.v[1], false);
-                    a2.v[1] = a2.v[1] + zmul_lane(A.d1r, A.d1i, x.v[1], x.v[0], true);
-                  }
-                  a2.v[0] = a2.v[0] + zmul_lane(A.d2r, A.d2i, s.v[0], s.v[1], false);
-                  a2.v[1] = a2.v[1] + zmul_lane(A.d2r, A.d2i, s.v[1], s.v[0], true);
-                } else {
-                  const bool odd = (l & 1) != 0;
-                  a2.v[0] = a2.v[0] + zmul_lane(A.dar, A.dai, ua.v[0], __shfl_xor(ua.v[0], 1), odd);
-                  a2.v[0] = a2.v[0] + zmul_lane(A.dbr, A.dbi, ub.v[0], __shfl_xor(ub.v[0], 1), odd);
-                  if (a_has_c1) a2.v[0] = a2.v[0] + zmul_lane(A.d1r, A.d1i, x.v[0], __shfl_xor(x.v[0], 1), odd);
-                  a2.v[0] = a2.v[0] + zmul_lane(A.d2r, A.d2i, s.v[0], __shfl_xor(s.v[0], 1), odd);
-                }
-                bst<LPT>(r_a2, roff(q0), a2);
-                dv = a2;
-              }
-              if (a_dpart) {
-                // |value|^2 of this thread's lanes times its state's weight, summed over
-                // the PAIRS consecutive threads of the column (one lane chunk)
-                double t = dv.v[0] * dv.v[0];
-                if constexpr (LPT == 2) t = t + dv.v[1] * dv.v[1];
-                t = wl * t;
+          };
+          add(av, A.car, A.cai, ua);
+          add(av, A.cbr, A.cbi, ub);
+          if (A.has_c1) add(av, A.c1r, A.c1i, xf);
+          add(av, A.c2r, A.c2i, s);
+          bst<LPT>(r_acc, qo, av, a_nt);  // dropped when there is no accumulator
+          if constexpr (EPI == EPI_TAYLOR_X) {
+            Vec<LPT> dv = av;
+            if (A.acc2) {
+              // psib2: the same terms with the deltat2 factors, from the same base
+              dv = ar[kk & 3];
+              add(dv, A.dar, A.dai, ua);
+              add(dv, A.dbr, A.dbi, ub);
+              if (A.has_c1) add(dv, A.d1r, A.d1i, xf);
+              add(dv, A.d2r, A.d2i, s);
+            }
+            bst<LPT>(r_a2, qo, dv, a_nt);
+            // density: |value|^2 of this thread's lanes times its state's weight, summed
+            // over the PAIRS consecutive threads of the column (one lane chunk)
+            double t = dv.v[0] * dv.v[0];
+            if constexpr (LPT == 2) t = t + dv.v[1] * dv.v[1];
+            t = wl * t;
 #pragma unroll
-                for (int off = PAIRS >> 1; off > 0; off >>= 1) t += __shfl_xor(t, off);
-                if (kp == 0) a_dpart[(size_t)chunk * a_np + q0] = t;
-              }
-            }
+            for (int off = PAIRS >> 1; off > 0; off >>= 1) t += __shfl_xor(t, off);
+            Vec<1> dt;
+            dt.v[0] = t;
+            bst<1>(r_dp, kp == 0 && z >= 4 ? poff(ro[(kk + 4) & 7], 3) : NONE, dt, false);
           }
         }
       }
+      __builtin_amdgcn_sched_barrier(0);
+      // ---- loads, into the registers that the plane staged and the plane completed have left;
+      // the ones consumed first in the next step first
+      const uint32_t kslot = ks[(kk + AD) & 3];  // of plane z - 4 + AD, loaded two steps ago
+      if constexpr (NL) {
+        const int P = z - 2 + AD;
+        const uint32_t qp = (P >= 0 && P < n) ? poff(ro[(kk + 6 + AD) & 7], 2) : NONE;
+        ks[(kk + 2 + AD) & 3] = __builtin_amdgcn_raw_buffer_load_b32(r_ks, qp, 0, 0);
+      }
+      rec[(kk + RD + 2) & 3] = load_rec(z + RD + 2);
+      {
+        const int P = z - 4 + AD;
+        const bool in = P >= 0 && P < n;
+        const uint32_t qp = ro[(kk + 4 + AD) & 7];
+        const uint32_t qa = in ? qp : lrow;
+        constexpr int M = 3;
+        const uint32_t qv = in ? poff(qp, 3) : NONE;
+        if constexpr (QUAD) vd[(kk + AD) & M] = __builtin_amdgcn_raw_buffer_load_b32(r_v, qv + (in ? (threadIdx.x & 1) * 4u : 0u), 0, 0);
+        else vr[(kk + AD) & M] = bld<1>(r_v, qv).v[0];
+        if constexpr (NL) {
+          // most waves have no ket row on a plane
+          Vec<LPT> kv;
+#pragma unroll
+          for (int k = 0; k < LPT; ++k) kv.v[k] = 0.0;
+          if (__builtin_amdgcn_ballot_w64(kslot != 0u) != 0ull) kv = bld<LPT>(r_k, roff(kslot));
+          kr[(kk + AD) & M] = kv;
+        }
+        if constexpr (TAY) {
+          ar[(kk + AD) & M] = bld<LPT>(r_ai, qa);
+          ra[(kk + AD) & M] = bld<LPT>(r_ya, qa);  // zeros (no memory access) without ya / yb
+          rb[(kk + AD) & M] = bld<LPT>(r_yb, qa);
+        }
+      }
+      {
+        const Rec& rn = rec[(kk + RD) & 3];
+        ro[(kk + RD) & 7] = own_row(rn);
+        ov[(kk + RD) & 7] = bld<LPT>(r_fi, ro[(kk + RD) & 7]);
+        hv[(kk + RD) & 3][0] = bld<LPT>(r_fi, halo_row(rn, z + RD, 0));
+        hv[(kk + RD) & 3][1] = bld<LPT>(r_fi, halo_row(rn, z + RD, 1));
+      }
+      // ---- start the sum of plane z: x, y, then z-4 .. z-1
+      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();
+      Vec<LPT> t;
+#pragma unroll
+      for (int k = 0; k < LPT; ++k) t.v[k] = 0.0;
+      if (z < n && ro[kk & 7] < np_bytes) {
+#pragma unroll
+        for (int j = 0; j < 17; ++j) {
+          const int d = j < 9 ? j - 4 : (j < 13 ? j - 13 : j - 12);
+          const Vec<LPT> x = j == 4 ? xz : ldv<LPT>(win + corner + own_lds + (j < 9 ? d : d * ZW) * LC);
+#pragma unroll
+          for (int k = 0; k < LPT; ++k) t.v[k] = fma(a_w[j], x.v[k], t.v[k]);
+          if (j == 4 || j == 8 || j == 12) __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+          for (int k = 0; k < LPT; ++k) t.v[k] = fma(a_w[17 + d], ov[(kk + 4 + d) & 7].v[k], t.v[k]);
+      }
+      part[kk & 3] = t;
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
 
+// Workgroups of up to 512 threads are held to 128 VGPRs: two of 512 threads per CU, whose
+// loads cover each other's latency.
 template <int LPT, int LC, int EPI, bool NL>
-__global__ __launch_bounds__(ZNC * LC / LPT) void k_zmarch(const ZArgs za) {
-  const int2 sc = za.sched[blockIdx.x];
-  if (sc.x < 0) return;              // padding entry of the schedule (whole workgroup)
-  zmarch_body<LPT, LC, EPI, NL>(za, za.items[sc.x], sc.x, sc.y);
+__global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch(const ZArgs za) {
+  const int4 sc = za.sched[blockIdx.x];
+  if (sc.y <= 0) return;             // padding entry of the schedule (whole workgroup)
+  zmarch_body<LPT, LC, EPI, NL>(za, sc.x, sc.y, sc.z);
 }
 
-// Several operators (systems) and batches in one launch: sched[b] = {descriptor, item,
-// lane chunk, -}; descriptors zs[] are ZArgs in device memory (their sched is unused).
+// Several operators (systems) and batches in one launch: sched[b] = {first record plane,
+// planes, lane chunk, descriptor}; descriptors zs[] are ZArgs in device memory (their sched is unused).
 template <int LPT, int LC, int EPI, bool NL>
-__global__ __launch_bounds__(ZNC * LC / LPT) void k_zmarch_multi(const ZArgs* __restrict__ zs,
-                                                                const int4* __restrict__ sched) {
+__global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_multi(const ZArgs* __restrict__ zs,
+                                                                   const int4* __restrict__ sched) {
   const int4 sc = sched[blockIdx.x];
-  if (sc.x < 0) return;
-  const ZArgs& za = zs[sc.x];
-  zmarch_body<LPT, LC, EPI, NL, true>(za, za.items[sc.y], sc.y, sc.z);
+  if (sc.y <= 0) return;
+  zmarch_body<LPT, LC, EPI, NL>(zs[sc.w], sc.x, sc.y, sc.z);
 }
 
-// dynamic LDS bytes of k_zmarch for a lane chunk and segment length: two plane buffers,
-// the item's index table and the ket slots of its own sites
-inline size_t zmarch_shmem(int lc, int zseg) {
-  return sizeof(double) * 2 * ZS * lc + sizeof(int) * ((size_t)zmarch_tab_ints(zseg) + (size_t)(zseg + 8) * ZNC);
-}
+// longest segment a launch accepts for a lane chunk
+constexpr int zmarch_max_seg(int lc) { return lc >= 32 ? 60 : 64; }
+
+// dynamic LDS bytes of k_zmarch for a lane chunk: two plane windows
+constexpr size_t zmarch_shmem(int lc) { return sizeof(double) * 2 * ZS * lc; }
 
 }  // namespace octhip

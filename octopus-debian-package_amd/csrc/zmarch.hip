@@ -28,8 +28,8 @@ int launch_nl(const ZArgs& z, int epi, int grid, size_t shmem, hipStream_t s) {
 }
 
 template <int LPT, int LC>
-int launch_lc(const ZArgs& z, int epi, int grid, int zseg, hipStream_t s) {
-  const size_t shmem = zmarch_shmem(LC, zseg);
+int launch_lc(const ZArgs& z, int epi, int grid, hipStream_t s) {
+  constexpr size_t shmem = zmarch_shmem(LC);
   ProfScope prof("k_zmarch", s);
   const int rc = z.a.kslot ? launch_nl<LPT, LC, true>(z, epi, grid, shmem, s)
                          : launch_nl<LPT, LC, false>(z, epi, grid, shmem, s);
@@ -39,9 +39,9 @@ int launch_lc(const ZArgs& z, int epi, int grid, int zseg, hipStream_t s) {
   return OCTHIP_SUCCESS;
 }
 template <int LPT, int LC>
-int launch_multi_lc(const ZArgs* zs, const int4* sched, int len, int epi, bool nl, int zseg, hipStream_t s) {
+int launch_multi_lc(const ZArgs* zs, const int4* sched, int len, int epi, bool nl, hipStream_t s) {
   constexpr int NT = ZNC * LC / LPT;
-  const size_t shmem = zmarch_shmem(LC, zseg);
+  constexpr size_t shmem = zmarch_shmem(LC);
   ProfScope prof("k_zmarch", s);
   if constexpr (NT > 1024) {
     return fail(OCTHIP_ERR_INVALID, "z-march: %d lanes per workgroup exceed 1024 threads", LC);
@@ -93,10 +93,9 @@ const void* kernel_of(int epi, bool nl, bool multi) {
 }
 }  // namespace
 
-// Workgroups of one z-march instance (k_zmarch, or k_zmarch_multi when multi) that its
-// registers alone let run on a CU (LDS not counted): the segment-length choice keeps the
-// LDS of that many resident.  Cached per instance; 1 for shapes without an instance.
-int zmarch_reg_blocks(int lc, int lpt, int epi, bool nl, bool multi) {
+// Workgroups of one z-march instance (k_zmarch, or k_zmarch_multi when multi) that fit on a
+// CU.  Cached per instance; 1 for shapes without an instance.
+int zmarch_resident(int lc, int lpt, int epi, bool nl, bool multi) {
   static int cache[2][2][6][3][2] = {};  // [multi][lpt-1][log2 lc][epi][nl], 0 = not asked yet
   int lg = 0;
   while ((1 << lg) < lc) ++lg;
@@ -124,45 +123,44 @@ int zmarch_reg_blocks(int lc, int lpt, int epi, bool nl, bool multi) {
     }
   }
   int nb = 1;
-  if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, ZNC * lc / lpt, 0) != hipSuccess || nb < 1) nb = 1;
+  if (!f || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, ZNC * lc / lpt, zmarch_shmem(lc)) !=
+                hipSuccess || nb < 1) nb = 1;
   c = nb;
   return nb;
 }
 
-int launch_zmarch_multi(const ZArgs* zs, const int4* sched, int len, int lc, int lpt, int epi, bool nl, int zseg,
+int launch_zmarch_multi(const ZArgs* zs, const int4* sched, int len, int lc, int lpt, int epi, bool nl,
                         hipStream_t s) {
   if (len <= 0) return OCTHIP_SUCCESS;
-  if (zmarch_shmem(lc, zseg) > 160 * 1024)
-    return fail(OCTHIP_ERR_INVALID, "z-march: lane chunk %d with z segment %d needs more than 160 KB of LDS", lc, zseg);
   if (lpt == 2) {
     switch (lc) {
-      case 2: return launch_multi_lc<2, 2>(zs, sched, len, epi, nl, zseg, s);
-      case 4: return launch_multi_lc<2, 4>(zs, sched, len, epi, nl, zseg, s);
-      case 8: return launch_multi_lc<2, 8>(zs, sched, len, epi, nl, zseg, s);
-      case 16: return launch_multi_lc<2, 16>(zs, sched, len, epi, nl, zseg, s);
+      case 2: return launch_multi_lc<2, 2>(zs, sched, len, epi, nl, s);
+      case 4: return launch_multi_lc<2, 4>(zs, sched, len, epi, nl, s);
+      case 8: return launch_multi_lc<2, 8>(zs, sched, len, epi, nl, s);
+      case 16: return launch_multi_lc<2, 16>(zs, sched, len, epi, nl, s);
       default: break;
     }
   }
   return fail(OCTHIP_ERR_INVALID, "no multi z-march instance for lane chunk %d, %d lanes per thread", lc, lpt);
 }
 
-int launch_zmarch(const ZArgs& z, int lc, int lpt, int epi, int grid, int zseg, hipStream_t s) {
+int launch_zmarch(const ZArgs& z, int lc, int lpt, int epi, int grid, hipStream_t s) {
   if (lpt == 2) {
     switch (lc) {
-      case 2: return launch_lc<2, 2>(z, epi, grid, zseg, s);
-      case 4: return launch_lc<2, 4>(z, epi, grid, zseg, s);
-      case 8: return launch_lc<2, 8>(z, epi, grid, zseg, s);
-      case 16: return launch_lc<2, 16>(z, epi, grid, zseg, s);
-      case 32: return launch_lc<2, 32>(z, epi, grid, zseg, s);
+      case 2: return launch_lc<2, 2>(z, epi, grid, s);
+      case 4: return launch_lc<2, 4>(z, epi, grid, s);
+      case 8: return launch_lc<2, 8>(z, epi, grid, s);
+      case 16: return launch_lc<2, 16>(z, epi, grid, s);
+      case 32: return launch_lc<2, 32>(z, epi, grid, s);
       default: break;
     }
   } else {
     switch (lc) {
-      case 1: return launch_lc<1, 1>(z, epi, grid, zseg, s);
-      case 2: return launch_lc<1, 2>(z, epi, grid, zseg, s);
-      case 4: return launch_lc<1, 4>(z, epi, grid, zseg, s);
-      case 8: return launch_lc<1, 8>(z, epi, grid, zseg, s);
-      case 16: return launch_lc<1, 16>(z, epi, grid, zseg, s);
+      case 1: return launch_lc<1, 1>(z, epi, grid, s);
+      case 2: return launch_lc<1, 2>(z, epi, grid, s);
+      case 4: return launch_lc<1, 4>(z, epi, grid, s);
+      case 8: return launch_lc<1, 8>(z, epi, grid, s);
+      case 16: return launch_lc<1, 16>(z, epi, grid, s);
       default: break;
     }
   }

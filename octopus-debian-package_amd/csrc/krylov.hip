@@ -18,11 +18,15 @@
 #include "kernels.h"
 
 namespace octhip {
-size_t dotp_scratch_bytes(int L, int is_complex);
-int launch_dotp(const double* a, const double* b, int L, int np, int is_complex, double vol, double* scratch,
-                hipStream_t s, double** result, double* dest = nullptr);
-int launch_axpy_cols(double* y, const double* x, int L, int np, int is_complex, const double* coef, hipStream_t s);
-int launch_scal_cols(double* x, int L, int np, int is_complex, const double* coef, hipStream_t s);
+size_t gs_scratch_bytes(int L);
+int launch_gs_dots(const double* const* x, int nv, const double* y, int L, int np, int nst, double vol,
+                   const double* nx, const double* ny, double* scratch, double* ov, double* coef, double* scale,
+                   hipStream_t s);
+int launch_gs_update(double* y, const double* src, const double* const* x, int nv, int L, int np, const double* scale,
+                     const double* coef, double* partial, hipStream_t s);
+int launch_gs_norms(const double* partial, int L, int np, int nst, double vol, double tiny, double* norm, double* kept,
+                    double* inv, hipStream_t s);
+int launch_gs_factors(const double* ov, int nv, int ncol, int nst, double* coef, hipStream_t s);
 int launch_cheby_update(double* out, const double* psi1, const double* b, const double* psi2, size_t count,
                         double mid, double span, std::complex<double> z, hipStream_t s);
 int launch_cheby_final(double* psib, const double* psi0, const double* psi2, size_t count, std::complex<double> z,
@@ -34,24 +38,32 @@ using cplx = std::complex<double>;
 
 namespace {
 
+constexpr int GS_MAX = 4;        // vectors per Gram-Schmidt pass (csrc/mesh_batch.hip)
+constexpr int KCOLS = 1 << (MAX_LDF - 1);  // most complex states of a row
+
 // Device buffers of one stream: nvec batches of np_part rows (Krylov vectors or the
-// Chebyshev recurrence) and a small block (per-state factors + dot-product scratch).
+// Chebyshev recurrence) and a small block, in doubles:
+//   res    [0]      overlaps of a step with two vectors (complex), then the norm: one copy to host
+//   coef   [RES]    factors of up to GS_MAX vectors and the scaling (complex)
+//   kept   [KEPT]   the norms the two latest Krylov vectors are kept with, by parity
+//   part   [PART]   partial sums
 struct KrylovBufs {
   double* vec = nullptr;
-  double* small = nullptr;
-  double* coef = nullptr;
-  double* dots = nullptr;
+  double *res = nullptr, *coef = nullptr, *scale = nullptr, *kept = nullptr, *part = nullptr;
+  double* host = nullptr;
+  hipEvent_t ready = nullptr;
 };
+constexpr size_t K_RES = 5 * KCOLS, K_COEF = 2 * KCOLS * (GS_MAX + 1), K_KEPT = 2 * KCOLS;
 
 int krylov_bufs(octhip_hamiltonian_s* h, hipStream_t s, int nvec, int ldf, KrylovBufs* out) {
   const size_t L = (size_t)1 << ldf;
   const size_t vec_bytes = sizeof(double) * (size_t)h->kin->np_part * L * nvec;
-  const size_t small_bytes = sizeof(double) * 2 * (1 << MAX_LDF) + dotp_scratch_bytes(1 << MAX_LDF, 0);
+  const size_t small_bytes = sizeof(double) * (K_RES + K_COEF + K_KEPT) + gs_scratch_bytes(1 << MAX_LDF) / 2;
   octhip_hamiltonian_s::KrylovSet* k = nullptr;
   for (auto& e : h->krylov)
     if (e.s == s) k = &e;
   if (!k) {
-    h->krylov.push_back({s, nullptr, 0, nullptr});
+    h->krylov.push_back({s, nullptr, 0, nullptr, nullptr, nullptr});
     k = &h->krylov.back();
   }
   if (k->bytes < vec_bytes) {
@@ -66,36 +78,38 @@ int krylov_bufs(octhip_hamiltonian_s* h, hipStream_t s, int nvec, int ldf, Krylo
     int rc = dalloc((void**)&k->small, small_bytes);
     if (rc) return rc;
   }
-  out->vec = k->vec;
-  out->small = k->small;
-  out->coef = k->small;
-  out->dots = k->small + 2 * (1 << MAX_LDF);
-  return OCTHIP_SUCCESS;
-}
-
-// per-state dot products <a|b> (complex, vol included) of the first nst states, on the host
-int dots(const double* a, const double* b, int L, int np, double vol, double* scratch, hipStream_t s, int nst,
-         std::vector<cplx>& out) {
-  double* res = nullptr;
-  int rc = launch_dotp(a, b, L, np, 1, vol, scratch, s, &res);
-  if (rc) return rc;
-  std::vector<double> host(2 * (size_t)nst);
-  OCTHIP_HIP(hipMemcpyAsync(host.data(), res, sizeof(double) * 2 * nst, hipMemcpyDeviceToHost, s));
-  OCTHIP_HIP(hipStreamSynchronize(s));
-  out.resize(nst);
-  for (int i = 0; i < nst; ++i) out[i] = cplx(host[2 * i], host[2 * i + 1]);
-  return OCTHIP_SUCCESS;
-}
-
-// per-state factors to the device: states nst.. of the row get `pad` (0 for axpy, 1 for scal)
-int upload_coefs(double* coef, const std::vector<cplx>& c, int ncol, cplx pad, hipStream_t s) {
-  std::vector<double> host(2 * (size_t)ncol);
-  for (int i = 0; i < ncol; ++i) {
-    const cplx v = i < (int)c.size() ? c[i] : pad;
-    host[2 * i] = v.real();
-    host[2 * i + 1] = v.imag();
+  if (!k->host && hipHostMalloc((void**)&k->host, sizeof(double) * K_RES, hipHostMallocDefault) != hipSuccess) {
+    k->host = nullptr;
+    (void)hipGetLastError();
+    return fail(OCTHIP_ERR_ALLOC, "hipHostMalloc(%zu bytes) failed", sizeof(double) * K_RES);
   }
-  OCTHIP_HIP(hipMemcpyAsync(coef, host.data(), sizeof(double) * 2 * ncol, hipMemcpyHostToDevice, s));
+  if (!k->ready) OCTHIP_HIP(hipEventCreateWithFlags(&k->ready, hipEventDisableTiming));
+  out->vec = k->vec;
+  out->res = k->small;
+  out->coef = out->res + K_RES;
+  out->scale = out->coef + 2 * KCOLS * GS_MAX;
+  out->kept = out->coef + K_COEF;
+  out->part = out->kept + K_KEPT;
+  out->host = k->host;
+  out->ready = k->ready;
+  return OCTHIP_SUCCESS;
+}
+
+// factors of the nv vectors (states nst.. of the row get 0) and the scaling (1) to the device
+int upload_factors(const std::vector<cplx>& c, int nv, int nst, int ncol, const std::vector<cplx>* scale, double* coef,
+                   double* dscale, hipStream_t s) {
+  std::vector<double> host(2 * (size_t)ncol * (nv + 1));
+  for (int v = 0; v <= nv; ++v)
+    for (int i = 0; i < ncol; ++i) {
+      const cplx z = v < nv ? (i < nst ? c[(size_t)v * nst + i] : cplx(0.0))
+                            : (scale && i < nst ? (*scale)[i] : cplx(1.0));
+      host[2 * ((size_t)v * ncol + i)] = z.real();
+      host[2 * ((size_t)v * ncol + i) + 1] = z.imag();
+    }
+  if (nv > 0)
+    OCTHIP_HIP(hipMemcpyAsync(coef, host.data(), sizeof(double) * 2 * ncol * nv, hipMemcpyHostToDevice, s));
+  OCTHIP_HIP(hipMemcpyAsync(dscale, host.data() + 2 * (size_t)ncol * nv, sizeof(double) * 2 * ncol,
+                            hipMemcpyHostToDevice, s));
   OCTHIP_HIP(hipStreamSynchronize(s));  // the host vector goes out of scope
   return OCTHIP_SUCCESS;
 }
@@ -209,6 +223,8 @@ void drop_krylov(octhip_hamiltonian_s* h, hipStream_t s, bool all) {
     if (all || h->krylov[i].s == s) {
       dfree(h->krylov[i].vec);
       dfree(h->krylov[i].small);
+      if (h->krylov[i].host) (void)hipHostFree(h->krylov[i].host);
+      if (h->krylov[i].ready) (void)hipEventDestroy(h->krylov[i].ready);
       h->krylov.erase(h->krylov.begin() + (long)i);
     } else {
       ++i;
@@ -236,100 +252,100 @@ extern "C" int octhip_exponential_lanczos_batch(octhip_hamiltonian_t h, double* 
   const cplx dt = imag_time ? cplx(0.0, deltat) : cplx(deltat, 0.0);
   const cplx pp = cplx(-0.0, -1.0) * dt;  // -i deltat
   const double eps = 2.220446049250313e-16;
+  const double tiny = 1e4 * eps;
+  const size_t cb = sizeof(double) * ncol;
+  double* const norm = kb.res + 4 * (size_t)ncol;     // behind the overlaps with two vectors
+  auto kept = [&](int k) { return kb.kept + (size_t)(k & 1) * ncol; };
+  auto fetch = [&]() -> int {  // a step's overlaps and norms to the host, an event behind them
+    OCTHIP_HIP(hipMemcpyAsync(kb.host, kb.res, 5 * cb, hipMemcpyDeviceToHost, s));
+    OCTHIP_HIP(hipEventRecord(kb.ready, s));
+    return OCTHIP_SUCCESS;
+  };
+  // The Krylov vectors are kept unnormalised, W_k = n_k vb(k + 1): the factors 1/n_k go into
+  // the next step's overlaps and update, so no pass only scales a vector.  A step is the
+  // H-apply, one pass for the overlaps with the two latest vectors, one pass that subtracts
+  // them and sums the norm, and one copy of the results to the host; the next H-apply is
+  // queued before the host waits for them, so that it runs while the projected problems are
+  // solved.  (137,065 points, 16 states, 12 steps: 8.4 -> 1.7 ms against a pass per dot product,
+  // subtraction and scaling, each with a copy and a wait.)
   // vb(1) = inh or psi (inner rows), beta = |vb(1)|
-  OCTHIP_HIP(hipMemcpyAsync(V(0), inh ? inh : psi, sizeof(double) * (size_t)np * L, hipMemcpyDeviceToDevice, s));
-  std::vector<cplx> d;
-  rc = dots(V(0), V(0), L, np, vol, kb.dots, s, nst, d);
+  rc = launch_gs_update(V(0), inh ? inh : psi, nullptr, 0, L, np, nullptr, nullptr, kb.part, s);
+  if (!rc) rc = launch_gs_norms(kb.part, L, np, nst, vol, 0.0, norm, kept(0), nullptr, s);
+  if (!rc) rc = fetch();
   if (rc) return rc;
+  OCTHIP_HIP(hipEventSynchronize(kb.ready));
   std::vector<double> beta(nst);
   bool all_null = true;
   for (int i = 0; i < nst; ++i) {
-    beta[i] = std::sqrt(d[i].real());
+    beta[i] = kb.host[4 * (size_t)ncol + i];
     if (std::fabs(beta[i]) > 1e-12) all_null = false;
   }
   if (iterations) *iterations = 0;
   if (residual) *residual = 0.0;
   if (all_null) return OCTHIP_SUCCESS;
-  std::vector<cplx> c(nst);
-  for (int i = 0; i < nst; ++i) c[i] = cplx(1.0 / beta[i], 0.0);
-  rc = upload_coefs(kb.coef, c, ncol, 1.0, s);
-  if (!rc) rc = launch_scal_cols(V(0), L, np, 1, kb.coef, s);
-  if (rc) return rc;
   const int M = order + 1;  // hamilt(1:M, 1:M) per state, column-major
   std::vector<cplx> hamilt((size_t)nst * M * M, 0.0), expo((size_t)nst * M, 0.0);
   auto H = [&](int st, int i, int j) -> cplx& { return hamilt[(size_t)st * M * M + i + (size_t)j * M]; };
-  std::vector<double> res(nst, 0.0);
+  std::vector<double> res(nst, 0.0), nk((size_t)M * nst, 1.0);  // nk: the norm of every vector kept
+  for (int st = 0; st < nst; ++st) nk[st] = beta[st];
   int iter = 1;
+  rc = propagator_apply(h, V(0), V(1), ldf, s);
+  if (rc) return rc;
   for (; iter <= order; ++iter) {
-    rc = propagator_apply(h, V(iter - 1), V(iter), ldf, s);
-    if (rc) return rc;
     // classical Gram-Schmidt against vb(l..iter), l = max(1, iter - 1) (Hermitian H):
     // every overlap first, then the subtractions (mesh_batch_inc.F90:1218-1231)
-    const int l = std::max(1, iter - 1);
-    std::vector<std::vector<cplx>> ss;
-    for (int j = l; j <= iter; ++j) {
-      std::vector<cplx> o;
-      rc = dots(V(j - 1), V(iter), L, np, vol, kb.dots, s, nst, o);
-      if (rc) return rc;
-      for (int st = 0; st < nst; ++st) H(st, j - 1, iter - 1) = o[st];
-      ss.push_back(o);
-    }
-    for (int j = l; j <= iter; ++j) {
-      for (int st = 0; st < nst; ++st) c[st] = -ss[j - l][st];
-      rc = upload_coefs(kb.coef, c, ncol, 0.0, s);
-      if (!rc) rc = launch_axpy_cols(V(iter), V(j - 1), L, np, 1, kb.coef, s);
-      if (rc) return rc;
-    }
-    rc = dots(V(iter), V(iter), L, np, vol, kb.dots, s, nst, d);
+    const int l = std::max(1, iter - 1), nv = iter - l + 1;
+    const double* x[2] = {V(l - 1), V(iter - 1)};
+    // the kept norms of the vectors in the order of x: those of an even and an odd vector lie
+    // side by side, so an odd-even pair takes the vectors the other way round
+    const bool swap = nv == 2 && ((l - 1) & 1);
+    if (swap) std::swap(x[0], x[1]);
+    rc = launch_gs_dots(x, nv, V(iter), L, np, nst, vol, nv == 2 ? kb.kept : kept(iter - 1), kept(iter - 1), kb.part,
+                        kb.res, kb.coef, kb.scale, s);
+    if (!rc) rc = launch_gs_update(V(iter), nullptr, x, nv, L, np, kb.scale, kb.coef, kb.part, s);
+    if (!rc) rc = launch_gs_norms(kb.part, L, np, nst, vol, tiny, norm, kept(iter), nullptr, s);
+    if (!rc) rc = fetch();
+    if (!rc && iter < order) rc = propagator_apply(h, V(iter), V(iter + 1), ldf, s);
     if (rc) return rc;
+    OCTHIP_HIP(hipEventSynchronize(kb.ready));
     bool happy = true;
     for (int st = 0; st < nst; ++st) {
-      const double nrm = std::sqrt(d[st].real());
+      for (int j = l; j <= iter; ++j) {
+        const int v = swap ? 1 - (j - l) : j - l;
+        H(st, j - 1, iter - 1) = cplx(kb.host[2 * ((size_t)v * ncol + st)], kb.host[2 * ((size_t)v * ncol + st) + 1]);
+      }
+      const double nrm = kb.host[4 * (size_t)ncol + st];
       H(st, iter, iter - 1) = nrm;
+      nk[(size_t)iter * nst + st] = nrm >= tiny ? nrm : 1.0;
       if (!krylov_function(iter, &H(st, 0, 0), M, pp, inh != nullptr, &expo[(size_t)st * M]))
         return fail(OCTHIP_ERR_HIP, "Lanczos: the projected eigenproblem did not converge");
       res[st] = std::abs(H(st, iter, iter - 1) * std::abs(expo[(size_t)st * M + iter - 1]));
-      if (std::abs(H(st, iter, iter - 1)) >= 1e4 * eps) happy = false;
+      if (std::abs(H(st, iter, iter - 1)) >= tiny) happy = false;
     }
     if (happy) break;  // happy breakdown
-    for (int st = 0; st < nst; ++st) {
-      const double a = std::abs(H(st, iter, iter - 1));
-      c[st] = a >= 1e4 * eps ? cplx(1.0 / a, 0.0) : cplx(1.0, 0.0);
-    }
-    rc = upload_coefs(kb.coef, c, ncol, 1.0, s);
-    if (!rc) rc = launch_scal_cols(V(iter), L, np, 1, kb.coef, s);
-    if (rc) return rc;
     if (iter > 3 && *std::max_element(res.begin(), res.end()) < lanczos_tol) break;
   }
   const int used = std::min(iter, order);  // a completed loop adds vb(order+1) with factor 0
   if (iterations) *iterations = used;
   if (residual) *residual = *std::max_element(res.begin(), res.end());
-  if (inh) {
-    // psi += deltat nrm V expo(:, 1)  (exponential.F90:883-887)
-    for (int ii = 1; ii <= used; ++ii) {
+  // inh: psi += deltat nrm V expo(:, 1)  (exponential.F90:883-887); else psi = expo(1,1) psi +
+  // sum_{ii >= 2} beta expo(ii,1) vb(ii)  (888-896); GS_MAX vectors per pass
+  for (int ii = inh ? 1 : 2; ii <= used || (!inh && ii == 2); ii += GS_MAX) {
+    const int nv = std::max(0, std::min(GS_MAX, used - ii + 1));
+    std::vector<cplx> c((size_t)nv * nst), first(nst);
+    const double* x[GS_MAX] = {};
+    for (int v = 0; v < nv; ++v) {
+      x[v] = V(ii + v - 1);
       for (int st = 0; st < nst; ++st) {
-        const double rb = dt.real() * beta[st];
-        const cplx ex = expo[(size_t)st * M + ii - 1];
-        c[st] = cplx(rb * ex.real(), rb * ex.imag());
+        const double rb = (inh ? dt.real() * beta[st] : beta[st]) / nk[(size_t)(ii + v - 1) * nst + st];
+        const cplx ex = expo[(size_t)st * M + ii + v - 1];
+        c[(size_t)v * nst + st] = cplx(rb * ex.real(), rb * ex.imag());
       }
-      rc = upload_coefs(kb.coef, c, ncol, 0.0, s);
-      if (!rc) rc = launch_axpy_cols(psi, V(ii - 1), L, np, 1, kb.coef, s);
-      if (rc) return rc;
     }
-    return OCTHIP_SUCCESS;
-  }
-  // psi = expo(1,1) psi + sum_{ii >= 2} beta expo(ii,1) vb(ii)  (exponential.F90:888-896)
-  for (int st = 0; st < nst; ++st) c[st] = expo[(size_t)st * M];
-  rc = upload_coefs(kb.coef, c, ncol, 1.0, s);
-  if (!rc) rc = launch_scal_cols(psi, L, np, 1, kb.coef, s);
-  if (rc) return rc;
-  for (int ii = 2; ii <= used; ++ii) {
-    for (int st = 0; st < nst; ++st) {
-      const cplx ex = expo[(size_t)st * M + ii - 1];
-      c[st] = cplx(beta[st] * ex.real(), beta[st] * ex.imag());
-    }
-    rc = upload_coefs(kb.coef, c, ncol, 0.0, s);
-    if (!rc) rc = launch_axpy_cols(psi, V(ii - 1), L, np, 1, kb.coef, s);
+    const bool scaled = !inh && ii == 2;
+    for (int st = 0; st < nst; ++st) first[st] = expo[(size_t)st * M];
+    rc = upload_factors(c, nv, nst, ncol, scaled ? &first : nullptr, kb.coef, kb.scale, s);
+    if (!rc) rc = launch_gs_update(psi, nullptr, x, nv, L, np, scaled ? kb.scale : nullptr, kb.coef, nullptr, s);
     if (rc) return rc;
   }
   return OCTHIP_SUCCESS;
@@ -402,42 +418,49 @@ extern "C" int octhip_mesh_batch_orthogonalization(int nvec, const double* const
   const int L = 1 << ldf, ncol = L / 2;
   OCTHIP_REQUIRE(nst >= 1 && nst <= ncol && np >= 0, "bad sizes nst=%d np=%d", nst, np);
   hipStream_t s = (hipStream_t)stream;
-  double *scratch = nullptr, *coef = nullptr;
-  int rc = dalloc((void**)&scratch, dotp_scratch_bytes(L, 1));
-  if (!rc) rc = dalloc((void**)&coef, sizeof(double) * 2 * ncol);
-  // classical Gram-Schmidt: every overlap <psi_k|phi> first, then phi -= sum_k <psi_k|phi> psi_k
-  std::vector<std::vector<cplx>> ss(nvec);
-  for (int k = 0; k < nvec && !rc; ++k) rc = dots(psi[k], phi, L, np, vol, scratch, s, nst, ss[k]);
-  std::vector<cplx> c(nst);
-  for (int k = 0; k < nvec && !rc; ++k) {
-    for (int st = 0; st < nst; ++st) c[st] = -ss[k][st];
-    rc = upload_coefs(coef, c, ncol, 0.0, s);
-    if (!rc) rc = launch_axpy_cols(phi, psi[k], L, np, 1, coef, s);
+  // one block: overlaps (nvec), factors of a pass, scaling, norms, partial sums
+  const size_t col2 = 2 * (size_t)ncol;
+  Scratch buf;
+  int rc = buf.get(sizeof(double) * (col2 * (nvec + GS_MAX + 2)) + gs_scratch_bytes(L));
+  if (rc) return rc;
+  double* const ov = static_cast<double*>(buf.ptr());
+  double* const dnorm = ov + col2 * nvec;             // behind the overlaps: one copy to the host
+  double* const coef = dnorm + col2;
+  double* const scale = coef + col2 * GS_MAX;
+  double* const part = scale + col2;
+  // Classical Gram-Schmidt: every overlap <psi_k|phi> first, GS_MAX vectors per pass over phi,
+  // then phi -= sum_k <psi_k|phi> psi_k, GS_MAX vectors per pass, the last pass summing the norm.
+  // (155,331 points, 32 states, 4 vectors with the H-apply before: 1253 -> 343 us.)
+  for (int k = 0; k < nvec && !rc; k += GS_MAX) {
+    const int nv = std::min(GS_MAX, nvec - k);
+    rc = launch_gs_dots(psi + k, nv, phi, L, np, nst, vol, nullptr, nullptr, part, ov + col2 * k, coef, nullptr, s);
   }
-  if (!rc && overlap)  // overlap(k, st) = <psi_k|phi_st>, column-major (nvec x nst)
+  const bool with_norm = norm || normalize;
+  for (int k = 0; k < std::max(nvec, 1) && !rc; k += GS_MAX) {
+    const int nv = std::min(GS_MAX, nvec - k);
+    const bool last = k + GS_MAX >= nvec;
+    if (nv == 0 && !with_norm) break;
+    // the factors of the last pass are still in coef; earlier ones are formed from the overlaps
+    if (nvec > GS_MAX) rc = launch_gs_factors(ov + col2 * k, nv, ncol, nst, coef, s);
+    if (!rc) rc = launch_gs_update(phi, nullptr, psi + k, nv, L, np, nullptr, coef, last && with_norm ? part : nullptr, s);
+  }
+  if (!rc && with_norm) rc = launch_gs_norms(part, L, np, nst, vol, 0.0, dnorm, nullptr, scale, s);
+  if (!rc && normalize) rc = launch_gs_update(phi, nullptr, nullptr, 0, L, np, scale, nullptr, nullptr, s);
+  std::vector<double> host(col2 * (nvec + 1));
+  if (!rc && (overlap || norm)) {
+    const hipError_t e = hipMemcpyAsync(host.data(), ov, sizeof(double) * host.size(), hipMemcpyDeviceToHost, s);
+    if (e != hipSuccess) rc = fail(OCTHIP_ERR_HIP, "orthogonalization: %s", hipGetErrorString(e));
+  }
+  const hipError_t e = hipStreamSynchronize(s);  // results on the host, scratch out of use
+  if (rc) return rc;
+  if (e != hipSuccess) return fail(OCTHIP_ERR_HIP, "orthogonalization: %s", hipGetErrorString(e));
+  if (overlap)  // overlap(k, st) = <psi_k|phi_st>, column-major (nvec x nst)
     for (int k = 0; k < nvec; ++k)
       for (int st = 0; st < nst; ++st) {
-        overlap[2 * ((size_t)k + (size_t)st * nvec)] = ss[k][st].real();
-        overlap[2 * ((size_t)k + (size_t)st * nvec) + 1] = ss[k][st].imag();
+        overlap[2 * ((size_t)k + (size_t)st * nvec)] = host[col2 * k + 2 * st];
+        overlap[2 * ((size_t)k + (size_t)st * nvec) + 1] = host[col2 * k + 2 * st + 1];
       }
-  if (!rc && (norm || normalize)) {
-    std::vector<cplx> d;
-    rc = dots(phi, phi, L, np, vol, scratch, s, nst, d);
-    for (int st = 0; st < nst && !rc; ++st) {
-      const double nr = std::sqrt(d[st].real());
-      if (norm) norm[st] = nr;
-      c[st] = cplx(1.0 / nr, 0.0);
-    }
-    if (!rc && normalize) {
-      rc = upload_coefs(coef, c, ncol, 1.0, s);
-      if (!rc) rc = launch_scal_cols(phi, L, np, 1, coef, s);
-      if (!rc) {
-        hipError_t e = hipStreamSynchronize(s);
-        if (e != hipSuccess) rc = fail(OCTHIP_ERR_HIP, "orthogonalization: %s", hipGetErrorString(e));
-      }
-    }
-  }
-  dfree(scratch);
-  dfree(coef);
-  return rc;
+  if (norm)
+    for (int st = 0; st < nst; ++st) norm[st] = host[col2 * nvec + st];
+  return OCTHIP_SUCCESS;
 }

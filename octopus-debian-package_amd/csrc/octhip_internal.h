@@ -52,6 +52,28 @@ const double* zero_row();
 int dalloc(void** p, size_t bytes);
 void dfree(void* p);
 
+// A device scratch buffer of a call that has no handle to keep it: taken from a pool of the
+// library and given back when the call ends (hipMalloc and hipFree cost about 100 us, and
+// hipFree waits for the device).  The caller synchronises its stream first.  The pool keeps at
+// most SCRATCH_KEEP buffers, of at most SCRATCH_MAX bytes each, until octhip_finalize; it is
+// safe with several threads and streams (a buffer has one user at a time).
+class Scratch {
+ public:
+  Scratch() = default;
+  Scratch(const Scratch&) = delete;
+  Scratch& operator=(const Scratch&) = delete;
+  ~Scratch();
+  int get(size_t bytes);
+  void* ptr() const { return p_; }
+
+ private:
+  void* p_ = nullptr;
+  size_t bytes_ = 0;
+};
+constexpr int SCRATCH_KEEP = 4;
+constexpr size_t SCRATCH_MAX = (size_t)16 << 20;
+void scratch_clear();
+
 template <typename T>
 int upload(T** dst, const T* src, size_t count, hipStream_t s) {
   *dst = nullptr;
@@ -216,6 +238,8 @@ struct octhip_hamiltonian_s {
     double* vec;
     size_t bytes;
     double* small;
+    double* host;                // pinned copy of a step's overlaps and norms
+    hipEvent_t ready;            // ... recorded behind that copy
   };
   std::vector<KrylovSet> krylov;
   // periodic boundaries: boundary row np+b takes inner row bnd_src[b]

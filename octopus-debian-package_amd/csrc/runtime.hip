@@ -3,6 +3,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
+#include <utility>
 #include <vector>
 
 #include <rocprofiler-sdk-roctx/roctx.h>
@@ -52,6 +54,53 @@ int dalloc(void** p, size_t bytes) {
 
 void dfree(void* p) {
   if (p) (void)hipFree(p);
+}
+
+namespace {
+std::mutex g_scratch_mu;
+std::vector<std::pair<void*, size_t>> g_scratch;  // buffers nobody uses
+}  // namespace
+
+int Scratch::get(size_t bytes) {
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    for (size_t i = 0; i < g_scratch.size(); ++i)
+      if (g_scratch[i].second >= bytes) {
+        p_ = g_scratch[i].first;
+        bytes_ = g_scratch[i].second;
+        g_scratch.erase(g_scratch.begin() + (long)i);
+        return OCTHIP_SUCCESS;
+      }
+  }
+  const int rc = dalloc(&p_, bytes);
+  if (!rc) bytes_ = bytes;
+  return rc;
+}
+
+Scratch::~Scratch() {
+  if (!p_) return;
+  void* old = p_;
+  if (bytes_ <= SCRATCH_MAX) {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    if ((int)g_scratch.size() < SCRATCH_KEEP) {
+      g_scratch.push_back({p_, bytes_});
+      old = nullptr;
+    } else {  // keep the larger buffers
+      for (auto& e : g_scratch)
+        if (e.second < bytes_) {
+          old = e.first;
+          e = {p_, bytes_};
+          break;
+        }
+    }
+  }
+  dfree(old);
+}
+
+void scratch_clear() {
+  std::lock_guard<std::mutex> lock(g_scratch_mu);
+  for (auto& e : g_scratch) dfree(e.first);
+  g_scratch.clear();
 }
 
 // ------------------------------------------------------------- profiling --
@@ -168,6 +217,7 @@ extern "C" int octhip_init(int device) {
 extern "C" int octhip_finalize(void) {
   if (!g_init) return OCTHIP_SUCCESS;
   OCTHIP_HIP(hipDeviceSynchronize());
+  scratch_clear();
   dfree(g_zero_row);
   g_zero_row = nullptr;
   g_init = false;

@@ -3,11 +3,10 @@
 // The reference runs the Taylor propagator batch by batch and system by system
 // (src/td/propagation_ops_elec.F90:232-249 over batches, one propagation per system),
 // each H-apply being ~5 kernel launches.  Here every kernel kind of one Taylor order runs
-// once for all pairs: the boundary clear, the projector bra, its reduction, the ket and
-// the multi-sphere sums go through multi-segment launches (a block finds its pair from a
-// block-offset table), and the fused stencil + local + ket + Taylor-epilogue pass is one
+// once for all pairs: the boundary clear, the projector bra, its reduction and the ket go through multi-segment launches (a block finds its pair
+// from a block-offset table), and the fused stencil + local + ket + Taylor-epilogue pass is one
 // z-march launch over a (pair, tile segment, lane chunk) work list, cut into 8
-// contiguous parts for the 8 XCDs.  A Taylor step is then 1 + 5 * order launches
+// contiguous parts for the 8 XCDs.  A Taylor step is then 1 + 4 * order launches
 // whatever the number of systems and batches.  Every pair has its own work buffers;
 // results are bit-identical to per-pair octhip_exponential_taylor_batch /
 // octhip_hamiltonian_apply_batch calls (same kernel bodies on the same data).
@@ -86,7 +85,7 @@ struct octhip_batched_s {
   bool mfma = true, nl = false;
   int lc = 16, lpt = 2;
   std::complex<double> zf[33];
-  Seg zero, reduce, ket, ksum;
+  Seg zero, reduce, ket;
   std::vector<Seg> bra;                 // [0] H-apply input psi, [k] Taylor order k input
   std::vector<ZArgs*> zdesc;            // [0] H-apply (store to hpsi), [k] Taylor order k
   int4* sched[2] = {nullptr, nullptr};  // per plan: blockIdx -> {first record, planes, lane chunk, pair}
@@ -107,7 +106,6 @@ void destroy(octhip_batched_s* b) {
   free_seg(b->zero);
   free_seg(b->reduce);
   free_seg(b->ket);
-  free_seg(b->ksum);
   for (auto& s : b->bra) free_seg(s);
   for (auto* z : b->zdesc) dfree(z);
   dfree(b->sched[0]);
@@ -230,7 +228,6 @@ int run_bra(octhip_batched_s* b, const Seg& bra, hipStream_t s) {
   if (!rc) rc = launch_multi(MULTI_BRA_REDUCE, b->reduce.args, b->reduce.off, b->reduce.nseg, b->reduce.nblocks, s);
   if (!rc) rc = launch_multi(b->mfma ? MULTI_KET_MFMA : MULTI_KET_PLAIN, b->ket.args, b->ket.off, b->ket.nseg,
                              b->ket.nblocks, s);
-  if (!rc) rc = launch_multi(MULTI_KET_SUM, b->ksum.args, b->ksum.off, b->ksum.nseg, b->ksum.nblocks, s);
   return rc;
 }
 
@@ -290,8 +287,8 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
     const size_t L = (size_t)p.L;
     if (b->nl) {
       rc = dalloc((void**)&p.partial, sizeof(double) * h->nchunk * h->max_nprojs * L);
-      if (!rc) rc = dalloc((void**)&p.proj, sizeof(double) * h->full_projection_size * L);
-      if (!rc) rc = dalloc((void**)&p.ksum, sizeof(double) * ((size_t)h->total_points + h->nmulti) * L);
+      if (!rc) rc = dalloc((void**)&p.proj, sizeof(double) * h->nprow * L);
+      if (!rc) rc = dalloc((void**)&p.ksum, sizeof(double) * h->nslot * L);
     }
     if (!rc) rc = dalloc((void**)&p.y[0], sizeof(double) * h->np * L);
     if (!rc) rc = dalloc((void**)&p.y[1], sizeof(double) * h->np * L);
@@ -323,12 +320,12 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
       p.plan[plan] = pl;
     }
   }
-  // boundary clear, reduce, ket, ket sums
+  // boundary clear, reduce, ket
   if (!rc) {
     std::vector<ZeroArgs> za;
     std::vector<BraReduceArgs> ra;
     std::vector<KetArgs> ka;
-    std::vector<int> zb, rb, kb, sb;
+    std::vector<int> zb, rb, kb;
     for (const Pair& p : b->pairs) {
       const octhip_hamiltonian_s* h = p.h;
       const int np = h->kin->np, np_part = h->kin->np_part;
@@ -337,33 +334,19 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
       BraReduceArgs r;
       std::memset(&r, 0, sizeof(r));
       r.partial = p.partial;
-      r.proj_mat = h->d_proj_mat;
-      r.mat_pbase = h->d_mat_pbase;
-      r.mat_chunk0 = h->d_mat_chunk0;
+      r.row = h->d_prow;
       r.scals = h->d_scals;
       r.proj = p.proj;
       r.L = p.L;
       r.pjmax = h->max_nprojs;
-      r.nproj = b->nl ? h->full_projection_size : 0;
+      r.nrow = b->nl ? h->nprow : 0;
       ra.push_back(r);
-      rb.push_back(blocks_for((size_t)r.nproj * p.L, 4096));
+      rb.push_back(blocks_for((size_t)r.nrow * p.L, 4096));
       KetArgs k;
-      std::memset(&k, 0, sizeof(k));
-      k.chunks = h->d_chunks;
-      k.mat_info = h->d_mat_info;
-      k.mat_pbase = h->d_mat_pbase;
-      k.pt = h->d_pt;
-      k.pjs = h->pjs;
-      k.proj = p.proj;
-      k.kbuf = p.ksum;
-      k.L = p.L;
-      k.multi_pos = h->d_multi_pos;
-      k.multi_g = h->d_multi_g;
-      k.nmulti = b->nl ? h->nmulti : 0;
-      k.total_points = h->total_points;
+      ket_args(h, p.L, p.partial, p.proj, p.ksum, false, k);
+      k.pphase = nullptr;  // finite systems
       ka.push_back(k);
-      kb.push_back(b->nl ? h->nchunk * (b->mfma ? mfma_lane_tiles(p.L) : 1) : 0);
-      sb.push_back(blocks_for((size_t)k.nmulti * ((p.L & 1) ? p.L : p.L / 2), 8192));
+      kb.push_back(b->nl ? ket_blocks(h->nkgrp) * (b->mfma ? mfma_lane_tiles(p.L) : 1) : 0);
     }
     for (size_t i = 0; i < b->pairs.size() && b->nl && !rc; ++i)
       if (!(ra[i].partial && ra[i].proj && ka[i].proj && ka[i].kbuf))
@@ -371,7 +354,6 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
     if (!rc) rc = make_seg(za, zb, b->zero);
     if (!rc) rc = make_seg(ra, rb, b->reduce);
     if (!rc) rc = make_seg(ka, kb, b->ket);
-    if (!rc) rc = make_seg(ka, sb, b->ksum);
   }
   // bra tables and z-march descriptors: [0] H-apply, [k] Taylor order k
   for (int k = 0; k <= order && !rc; ++k) {

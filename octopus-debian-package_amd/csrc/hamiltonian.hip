@@ -53,8 +53,8 @@ int ensure_work(octhip_hamiltonian_s* h, int ldf, hipStream_t s) {
     int rc = OCTHIP_SUCCESS;
     if (h->nmat > 0) {
       rc = dalloc((void**)&w.partial, sizeof(double) * h->nchunk * h->max_nprojs * L);
-      if (!rc) rc = dalloc((void**)&w.proj, sizeof(double) * h->full_projection_size * L);
-      if (!rc) rc = dalloc((void**)&w.ksum, sizeof(double) * ((size_t)h->total_points + h->nmulti) * L);
+      if (!rc) rc = dalloc((void**)&w.proj, sizeof(double) * h->nprow * L);
+      if (!rc) rc = dalloc((void**)&w.ksum, sizeof(double) * std::max(h->nslot, 1) * L);
     }
     if (rc) return rc;
     w.work_ldf = ldf;
@@ -81,7 +81,7 @@ int ensure_taylor(octhip_hamiltonian_s* h, int ldf, hipStream_t s) {
   return OCTHIP_SUCCESS;
 }
 
-// projections of batch f (L lanes) into h->d_proj; zero_bc (optional) = a batch whose
+// projections of batch f (L lanes) and their ket rows into h->d_ksum; zero_bc (optional) = a batch whose
 // boundary rows are cleared on the way (fused into the bra launch when it can be)
 int run_bra(octhip_hamiltonian_s* h, const double* f, int L, hipStream_t s, double* zero_bc = nullptr) {
   const int np = h->kin->np, np_part = h->kin->np_part;
@@ -106,41 +106,20 @@ int run_bra(octhip_hamiltonian_s* h, const double* f, int L, hipStream_t s, doub
                                   (size_t)(np_part - np) * L)
                 : launch_bra(b, h->nchunk, false, s);
   if (rc) return rc;
-  // with the MFMA ket, each ket workgroup sums the partials of its matrix itself
-  const bool fuse = mfma && h->max_nprojs <= KET_FUSE_PJMAX;
+  const bool sums = mfma && ket_sums_partials(h, L);
   BraReduceArgs r;
   r.partial = h->d_partial;
-  r.proj_mat = h->d_proj_mat;
-  r.mat_pbase = h->d_mat_pbase;
-  r.mat_chunk0 = h->d_mat_chunk0;
+  r.row = h->d_prow;
   r.scals = h->d_scals;
   r.proj = h->d_proj;
   r.L = L;
   r.pjmax = h->max_nprojs;
-  r.nproj = h->full_projection_size;
-  if (!fuse) rc = launch_bra_reduce(r, s);
+  r.nrow = h->nprow;
+  if (!sums) rc = launch_bra_reduce(r, s);
   if (rc) return rc;
   KetArgs k;
-  if (fuse) {
-    k.partial = h->d_partial;
-    k.mat_chunk0 = h->d_mat_chunk0;
-    k.scals = h->d_scals;
-    k.pjmax = h->max_nprojs;
-  }
-  k.chunks = h->d_chunks;
-  k.mat_info = h->d_mat_info;
-  k.mat_pbase = h->d_mat_pbase;
-  k.pt = h->d_pt;
-  k.pjs = h->pjs;
-  k.proj = h->d_proj;
-  k.kbuf = h->d_ksum;
-  k.L = L;
-  k.multi_pos = h->d_multi_pos;
-  k.multi_g = h->d_multi_g;
-  k.nmulti = h->nmulti;
-  k.total_points = h->total_points;
-  k.pphase = h->has_kpoint ? h->d_pphase : nullptr;
-  return launch_ket(k, h->nchunk, h->use_mfma, s);
+  ket_args(h, L, h->d_partial, h->d_proj, h->d_ksum, sums, k);
+  return launch_ket(k, h->use_mfma, s);
 }
 
 // v_eff(p) = v(p) + (f0 x + f1 y + f2 z): the dipole term of laser_potential
@@ -154,6 +133,34 @@ __global__ void k_veff(double* __restrict__ veff, const double* __restrict__ v,
 }  // namespace
 
 namespace octhip {
+bool ket_sums_partials(const octhip_hamiltonian_s* h, int L) {
+  const int tiles = mfma_lane_tiles(L);
+  return h->ket_sums * (L / tiles) <= KET_SUMS && ket_blocks(h->nkgrp) * tiles <= KET_SUM_BLOCKS;
+}
+
+void ket_args(const octhip_hamiltonian_s* h, int L, const double* partial, const double* proj, double* kbuf,
+              bool sums, KetArgs& k) {
+  k = KetArgs();
+  if (sums) {
+    k.partial = partial;
+    k.sum = h->d_ksumrow;
+    k.scals = h->d_scals;
+    k.pjmax = h->max_nprojs;
+  }
+  k.grp = h->d_kgrp;
+  k.ngrp = h->nkgrp;
+  k.step = h->d_kstep;
+  k.blk = h->d_kblk;
+  k.pt = h->d_kpt;
+  k.proj = proj;
+  k.kbuf = kbuf;
+  k.L = L;
+  if (h->has_kpoint) {
+    k.pphase = h->d_pphase;
+    k.kg = h->d_kg;
+  }
+}
+
 int zero_boundary(double* f, int np, int np_part, int L, hipStream_t s) {
   const size_t count = (size_t)(np_part - np) * L;
   if (count == 0) return OCTHIP_SUCCESS;
@@ -207,7 +214,7 @@ void fill_terms(const octhip_hamiltonian_s* h, int terms, ApplyArgs& a) {
   if ((terms & OCTHIP_TERM_NON_LOCAL_POTENTIAL) && h->nmat > 0 && h->nslot > 0) {
     a.kslot = h->d_kslot;
     a.ksum = h->d_ksum;
-    a.nk = h->total_points + h->nmulti;
+    a.nk = h->nslot;
   }
 }
 
@@ -272,6 +279,103 @@ int periodic_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, 
   if (!rc && set_phase) rc = launch_phase(hpsi, hpsi, h->d_phase, np, L, true, s);
   return rc;
 }
+// Ket tables of a handle (KetArgs, BraReduceArgs::row).
+struct KetTables {
+  std::vector<int> slot, g;
+  std::vector<KetGroup> grp;
+  std::vector<int4> step, sum, prow;
+  std::vector<int2> blk;
+  std::vector<double> pt;
+  std::vector<int> matrix;  // matrix of each step
+};
+
+int padded_projs(const octhip_hamiltonian_s* h, int a) { return (h->offsets[6 * (size_t)a + O_PROJS] + 3) / 4 * 4; }
+
+// the sums of each workgroup: the projection rows (from prow0[a]) of its groups' matrices,
+// each once; returns the largest number
+int ket_sums(const octhip_hamiltonian_s* h, const std::vector<int>& prow0, KetTables& t) {
+  int most = 0;
+  std::vector<int> row(h->nmat, -1), open;  // first sum of the matrices of the workgroup
+  for (size_t g0 = 0; g0 < t.grp.size(); g0 += KET_GROUPS) {
+    for (int a : open) row[a] = -1;
+    open.clear();
+    int2 b = make_int2((int)t.sum.size(), 0);
+    const KetGroup& last = t.grp[std::min(g0 + KET_GROUPS, t.grp.size()) - 1];
+    for (int q = t.grp[g0].step; q < last.step + last.steps; ++q) {
+      const int a = t.matrix[q];
+      if (row[a] < 0) {
+        row[a] = b.y;
+        open.push_back(a);
+        for (int j = 0; j < padded_projs(h, a); ++j, ++b.y) t.sum.push_back(t.prow[prow0[a] + j]);
+      }
+      t.step[q].x = row[a] + (t.step[q].y - prow0[a]);
+    }
+    most = std::max(most, b.y);
+    t.blk.push_back(b);
+  }
+  return most;
+}
+
+// pos, ent: CSR over the mesh points of their sphere points {map index, matrix}, matrix order
+void build_ket(octhip_hamiltonian_s* h, const double* matrices, const std::vector<int>& pos,
+               const std::vector<int2>& ent, const std::vector<int>& chunk0, KetTables& t) {
+  std::vector<int> prow0(h->nmat);
+  for (int a = 0; a < h->nmat; ++a) {
+    const int* o = h->offsets.data() + 6 * (size_t)a;
+    prow0[a] = (int)t.prow.size();
+    for (int j = 0; j < padded_projs(h, a); ++j)
+      t.prow.push_back(make_int4(chunk0[a], chunk0[a + 1], j, j < o[O_PROJS] ? o[O_SCAL] + j : -1));
+  }
+  h->nprow = (int)t.prow.size();
+  // mesh points inside a sphere, by their set of matrices, mesh order within a set
+  std::vector<int> pts;
+  for (int p = 0; p < h->np; ++p)
+    if (pos[p + 1] > pos[p]) pts.push_back(p);
+  auto cmp = [&](int p, int q) {  // -1, 0, 1: order of the two points' sets
+    for (int i = pos[p], j = pos[q];; ++i, ++j) {
+      if (i == pos[p + 1] || j == pos[q + 1]) return (i < pos[p + 1]) - (j < pos[q + 1]);
+      if (ent[i].y != ent[j].y) return ent[i].y < ent[j].y ? -1 : 1;
+    }
+  };
+  std::stable_sort(pts.begin(), pts.end(), [&](int p, int q) { return cmp(p, q) < 0; });
+  h->nslot = (int)pts.size();
+  t.slot.assign(h->np, 0);
+  for (size_t i = 0, e; i < pts.size(); i = e) {
+    for (e = i + 1; e < pts.size() && e < i + 16 && cmp(pts[i], pts[e]) == 0;) ++e;
+    const int p0 = pos[pts[i]], ne = pos[pts[i] + 1] - p0, n = (int)(e - i);
+    const int step0 = (int)t.step.size(), line0 = (int)(t.pt.size() / 4);
+    for (int k = 0; k < ne; ++k) {
+      const int a = ent[p0 + k].y;
+      const int* o = h->offsets.data() + 6 * (size_t)a;
+      const int entry = (int)t.g.size();
+      for (size_t r = i; r < e; ++r) t.g.push_back(ent[pos[pts[r]] + k].x);
+      for (int j = 0; j < o[O_PROJS]; j += 4) {
+        t.step.push_back(make_int4(0, prow0[a] + j, j == 0 ? entry : -1, 0));
+        t.matrix.push_back(a);
+        for (int r = 0; r < n; ++r)
+          for (int c = j; c < j + 4; ++c)
+            t.pt.push_back(c < o[O_PROJS] ? matrices[o[O_MATRIX] + (size_t)c * o[O_POINTS] + (t.g[entry + r] - o[O_MAP])]
+                                          : 0.0);
+      }
+    }
+    KetGroup g = {};
+    g.row = (int)i;
+    g.rows = n;
+    g.steps = (int)t.step.size() - step0;
+    g.step = step0;
+    g.line = line0;
+    t.grp.push_back(g);
+    for (size_t r = i; r < e; ++r) t.slot[pts[r]] = (int)r + 1;
+  }
+  h->nkgrp = (int)t.grp.size();
+  h->ket_sums = ket_sums(h, prow0, t);
+  for (KetGroup& g : t.grp)
+    for (int u = 0; u < KET_AHEAD; ++u) {
+      const int4 q = t.step[g.step + std::min(u, g.steps - 1)];
+      g.ahead[u] = make_int2(q.x, q.y);
+    }
+}
+
 }  // namespace
 
 extern "C" int octhip_hamiltonian_create(octhip_nl_operator_t kinetic, double mass, const double* vlocal,
@@ -306,7 +410,6 @@ extern "C" int octhip_hamiltonian_create(octhip_nl_operator_t kinetic, double ma
   h->np = np;
   h->nmat = nmat;
   h->max_nprojs = max_nprojs;
-  h->full_projection_size = (int)nproj;
   h->total_points = (int)total_points;
   h->pjs = max_nprojs;
   h->offsets.assign(offsets ? offsets : nullptr, offsets ? offsets + 6 * (size_t)nmat : nullptr);
@@ -315,15 +418,12 @@ extern "C" int octhip_hamiltonian_create(octhip_nl_operator_t kinetic, double ma
   if (vlocal) rc = upload(&h->d_v, vlocal, (size_t)np, s);
   if (!rc && nmat > 0) {
     std::vector<double> pt(total_points * (size_t)h->pjs, 0.0);
-    std::vector<int> cnt(np + 1, 0), pbase(nmat), npj(nmat), proj_mat(nproj, 0), chunk0(nmat + 1);
+    std::vector<int> cnt(np + 1, 0), chunk0(nmat + 1);
     std::vector<int4> info(nmat), chunks;
     for (int a = 0; a < nmat; ++a) {
       const int* o = offsets + 6 * (size_t)a;
       const int npt = o[O_POINTS], nj = o[O_PROJS];
-      pbase[a] = o[O_SCAL];
-      npj[a] = nj;
       info[a] = make_int4(npt, nj, o[O_MATRIX], o[O_MAP]);
-      for (int j = 0; j < nj; ++j) proj_mat[o[O_SCAL] + j] = a;
       for (int q = 0; q < npt; ++q) {
         for (int j = 0; j < nj; ++j)
           pt[(size_t)(o[O_MAP] + q) * h->pjs + j] = matrices[o[O_MATRIX] + (size_t)j * npt + q];
@@ -347,36 +447,24 @@ extern "C" int octhip_hamiltonian_create(octhip_nl_operator_t kinetic, double ma
       }
     }
     h->nchunk = (int)chunks.size();
-    // ket row per mesh point: its sphere point if it lies in one sphere, else a summed row
-    std::vector<int> kslot(np, 0), multi_pos(1, 0), multi_g;
-    int nslot = 0;
-    for (int p = 0; p < np; ++p) {
-      const int ne = pos[p + 1] - pos[p];
-      if (ne == 0) continue;
-      ++nslot;
-      if (ne == 1) {
-        kslot[p] = ent[pos[p]].x + 1;
-      } else {
-        kslot[p] = (int)total_points + (int)multi_pos.size();
-        for (int e = pos[p]; e < pos[p + 1]; ++e) multi_g.push_back(ent[e].x);
-        multi_pos.push_back((int)multi_g.size());
-      }
+    KetTables kt;
+    build_ket(h, matrices, pos, ent, chunk0, kt);
+    rc = upload(&h->d_kslot, kt.slot.data(), kt.slot.size(), s);
+    if (!rc && !kt.grp.empty()) {
+      rc = upload(&h->d_kgrp, kt.grp.data(), kt.grp.size(), s);
+      if (!rc) rc = upload(&h->d_kstep, kt.step.data(), kt.step.size(), s);
+      if (!rc) rc = upload(&h->d_kpt, kt.pt.data(), kt.pt.size(), s);
+      if (!rc) rc = upload(&h->d_kg, kt.g.data(), kt.g.size(), s);
+      if (!rc) rc = upload(&h->d_kblk, kt.blk.data(), kt.blk.size(), s);
+      if (!rc) rc = upload(&h->d_ksumrow, kt.sum.data(), kt.sum.size(), s);
     }
-    h->nslot = nslot;
-    h->nmulti = (int)multi_pos.size() - 1;
-    rc = upload(&h->d_kslot, kslot.data(), kslot.size(), s);
-    if (!rc) rc = upload(&h->d_multi_pos, multi_pos.data(), multi_pos.size(), s);
-    if (!rc && !multi_g.empty()) rc = upload(&h->d_multi_g, multi_g.data(), multi_g.size(), s);
     if (!rc) rc = upload(&h->d_matrices, matrices, matrix_size, s);
     if (!rc) rc = upload(&h->d_maps, maps, total_points, s);
     if (!rc) rc = upload(&h->d_scals, scals, nproj, s);
     if (!rc) rc = upload(&h->d_pt, pt.data(), pt.size(), s);
-    if (!rc) rc = upload(&h->d_mat_pbase, pbase.data(), pbase.size(), s);
-    if (!rc) rc = upload(&h->d_mat_npj, npj.data(), npj.size(), s);
     if (!rc) rc = upload(&h->d_chunks, chunks.data(), chunks.size(), s);
-    if (!rc) rc = upload(&h->d_mat_chunk0, chunk0.data(), chunk0.size(), s);
     if (!rc) rc = upload(&h->d_mat_info, info.data(), info.size(), s);
-    if (!rc) rc = upload(&h->d_proj_mat, proj_mat.data(), proj_mat.size(), s);
+    if (!rc) rc = upload(&h->d_prow, kt.prow.data(), kt.prow.size(), s);
   }
   if (rc) {
     octhip_hamiltonian_destroy(h);
@@ -390,10 +478,14 @@ extern "C" int octhip_hamiltonian_destroy(octhip_hamiltonian_t h) {
   if (!h) return OCTHIP_SUCCESS;
   (void)hipDeviceSynchronize();
   dfree(h->d_mat_info);
-  dfree(h->d_proj_mat);
   dfree(h->d_kslot);
-  dfree(h->d_multi_pos);
-  dfree(h->d_multi_g);
+  dfree(h->d_kgrp);
+  dfree(h->d_kstep);
+  dfree(h->d_prow);
+  dfree(h->d_kblk);
+  dfree(h->d_ksumrow);
+  dfree(h->d_kpt);
+  dfree(h->d_kg);
   dfree(h->d_v);
   dfree(h->d_xyz);
   dfree(h->d_veff);
@@ -401,10 +493,7 @@ extern "C" int octhip_hamiltonian_destroy(octhip_hamiltonian_t h) {
   dfree(h->d_maps);
   dfree(h->d_scals);
   dfree(h->d_pt);
-  dfree(h->d_mat_pbase);
-  dfree(h->d_mat_npj);
   dfree(h->d_chunks);
-  dfree(h->d_mat_chunk0);
   for (auto& w : h->sets)
     for (void* p : {(void*)w.partial, (void*)w.proj, (void*)w.ksum, (void*)w.y0, (void*)w.y1, (void*)w.y2,
                     (void*)w.dpart, (void*)w.dw, (void*)w.ephase})
@@ -490,9 +579,10 @@ extern "C" int octhip_hamiltonian_memory(octhip_hamiltonian_t h, size_t* bytes) 
   for (const void* p : {(const void*)h->d_v, (const void*)h->d_xyz, (const void*)h->d_veff,
                         (const void*)h->d_matrices, (const void*)h->d_maps, (const void*)h->d_scals,
                         (const void*)h->d_pt,
-                        (const void*)h->d_mat_pbase, (const void*)h->d_mat_npj, (const void*)h->d_chunks,
-                        (const void*)h->d_mat_chunk0, (const void*)h->d_mat_info, (const void*)h->d_proj_mat,
-                        (const void*)h->d_kslot, (const void*)h->d_multi_pos, (const void*)h->d_multi_g,
+                        (const void*)h->d_chunks, (const void*)h->d_mat_info, (const void*)h->d_prow,
+                        (const void*)h->d_kslot, (const void*)h->d_kgrp, (const void*)h->d_kstep,
+                        (const void*)h->d_kblk, (const void*)h->d_ksumrow, (const void*)h->d_kpt,
+                        (const void*)h->d_kg,
                         (const void*)h->d_bnd_src, (const void*)h->d_phase, (const void*)h->d_phase_corr,
                         (const void*)h->d_pphase})
     data += dev_bytes(p);

@@ -330,50 +330,62 @@ struct BraArgs {
   const double* __restrict__ pphase = nullptr;
 };
 
+// Projections of a matrix occupy 4 ceil(nprojs / 4) rows, the last ones zero, so that the
+// ket's steps of 4 projectors need no masks.
 struct BraReduceArgs {
   const double* __restrict__ partial;
-  const int* __restrict__ proj_mat;   // projection index -> matrix
-  const int* __restrict__ mat_pbase;
-  const int* __restrict__ mat_chunk0; // nmat+1
+  const int4* __restrict__ row;       // nrow: {first chunk, last chunk + 1, projector, scal or -1: a zero row}
   const double* __restrict__ scals;
-  double* __restrict__ proj;          // (full_projection_size, L)
-  int L, pjmax, nproj;
+  double* __restrict__ proj;          // (nrow, L)
+  int L, pjmax, nrow;
 };
 
+// groups of <= 16 rows per ket workgroup (one a wave), steps of a group loaded with it
+constexpr int KET_GROUPS = 4;
+constexpr int KET_AHEAD = 4;
+// Where the ket is a few hundred workgroups with few projections each, they sum the bra's
+// partials themselves (LDS of KET_SUMS doubles) and save a launch: radius-3 spheres at h =
+// 0.45 x 16 lanes, 69 workgroups of <= 8 projection rows, 5.1 us instead of 4.0 + 3.9 (bra
+// reduce).  Every workgroup waits for its sums, though: 566 workgroups of up to 64 rows take
+// 10.9 instead of 5.5 + 4.1, and 2480 of about 6 rows (R = 12 sphere x 64 lanes) 28.3
+// instead of 14.0 + 5.0.
+constexpr int KET_SUMS = 512;
+constexpr int KET_SUM_BLOCKS = 512;
+
 // Ket of X(hamiltonian_elec_base_nlocal_finish) (src/hamiltonian/hamiltonian_elec_base_inc.F90:
-// 914-943) in two passes:
-//  k_ket:     kbuf[g, l] = sum_j P[g, j] proj[pbase(g) + j, l] for every global sphere point g
-//             (matrix by matrix: a (npoints x nprojs) x (nprojs x L) product, FP64 MFMA);
-//  k_ket_sum: kbuf[total_points + m, l] = sum of the rows of the m-th mesh point that lies in
-//             several spheres, in matrix order.
-// A mesh point p then adds row kref[p] of kbuf (its single sphere row or its sum), or nothing.
+// 914-943) in one pass over the mesh points that lie in at least one sphere:
+//   kbuf[r, l] = sum_a sum_j P_a[r, j] proj[a, j, l],  a in matrix order.
+// The ket rows are sorted by the set of matrices of their point and cut into groups of <= 16
+// rows with one set, so a group is one FP64 MFMA product over steps of 4 projectors and no
+// row takes part in a matrix it does not belong to (an infinity in one projection stays in
+// its own sphere).  Mesh point p then adds row kslot[p] - 1 of kbuf, or nothing.
+struct KetGroup {
+  int row, rows, steps, step;         // first ket row, rows, steps, first step
+  int line, pad[3];                   // first line of pt
+  int2 ahead[KET_AHEAD];              // the first steps' (sum, proj) again: one load fetches a group
+};
 struct KetArgs {
-  const int4* __restrict__ chunks;    // bra chunks {matrix, q0, q1, -}
-  const int4* __restrict__ mat_info;  // {npoints, nprojs, matrix offset, map offset}
-  const int* __restrict__ mat_pbase;
-  const double* __restrict__ pt;      // transposed projector rows, stride pjs
-  int pjs;
+  const KetGroup* __restrict__ grp;
+  int ngrp;                           // workgroup b owns groups KET_GROUPS b ..
+  const int4* __restrict__ step;      // {row of the block's sums, row of proj, first kg entry or -1: same matrix, -}
+  const int2* __restrict__ blk;       // {first sum, sums} of a workgroup
+  const double* __restrict__ pt;      // lines of 4 projector values: line + step * rows + row
   const double* __restrict__ proj;
   double* __restrict__ kbuf;
   int L;
-  // multi-sphere sums
-  const int* __restrict__ multi_pos;  // nmulti+1 CSR into multi_g
-  const int* __restrict__ multi_g;    // global sphere points, matrix order
-  int nmulti, total_points;
   // optional (MFMA form only): the bra's chunk partials instead of proj; each workgroup
-  // then forms the projections of its matrix and lane tile itself, summed and scaled as
+  // then forms the projections of its groups and lane tile itself, summed and scaled as
   // k_bra_reduce does (so bit-identical), and k_bra_reduce is not launched
   const double* __restrict__ partial = nullptr;
-  const int* __restrict__ mat_chunk0 = nullptr;  // nmat+1
+  const int4* __restrict__ sum = nullptr;  // as BraReduceArgs::row
   const double* __restrict__ scals = nullptr;
   int pjmax = 0;
-  // Bloch phases of the sphere points: the ket row of point q is multiplied by
-  // conj(pphase[q]) (hamiltonian_elec_base_inc.F90:955-966); null: none
+  // Bloch phases: the term of a matrix is multiplied by conj(pphase[kg[entry + row]])
+  // (hamiltonian_elec_base_inc.F90:955-966); null: none
   const double* __restrict__ pphase = nullptr;
+  const int* __restrict__ kg = nullptr;
 };
 
-// largest projector count per matrix for which the ket forms its projections itself
-constexpr int KET_FUSE_PJMAX = 32;
 
 struct BraMfmaArgs {
   BraArgs b;
@@ -392,12 +404,18 @@ struct ZeroArgs {
 
 // kernels of a multi-segment launch (several systems/batches in one grid)
 enum { MULTI_BRA_MFMA = 1, MULTI_BRA_PLAIN, MULTI_BRA_REDUCE, MULTI_KET_MFMA, MULTI_KET_PLAIN,
-       MULTI_KET_SUM, MULTI_ZERO };
+       MULTI_ZERO };
 // args: device array of nseg argument blocks; off: device array of nseg+1 block offsets
 int launch_multi(int kind, const void* args, const int* off, int nseg, int nblocks, hipStream_t s);
 
 int launch_bra(const BraArgs& b, int nchunk, bool mfma, hipStream_t s);
-int launch_ket(const KetArgs& k, int nchunk, bool mfma, hipStream_t s);
+// whether the ket of h sums the partials itself at this row length, and its arguments then
+// (sums) or from proj
+bool ket_sums_partials(const octhip_hamiltonian_s* h, int L);
+void ket_args(const octhip_hamiltonian_s* h, int L, const double* partial, const double* proj, double* kbuf,
+              bool sums, KetArgs& k);
+inline int ket_blocks(int ngrp) { return (ngrp + KET_GROUPS - 1) / KET_GROUPS; }
+int launch_ket(const KetArgs& k, bool mfma, hipStream_t s);
 // lane tiles of the MFMA bra and ket over rows of L lanes (L >= 16): 32-lane tiles (two
 // columns per lane) when 32 divides L, else 16-lane tiles
 __host__ __device__ inline int mfma_lane_tiles(int L) { return (L & 31) == 0 ? L >> 5 : L >> 4; }

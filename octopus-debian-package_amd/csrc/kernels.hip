@@ -228,27 +228,29 @@ __global__ __launch_bounds__(BLOCK) void k_bra_mfma(const BraMfmaArgs m) {
   }
 }
 
-// proj[i, l] = scal[i] * sum_{chunks of matrix(i)} partial[chunk, i - pbase, l]
+// one projection: scal * sum of its matrix's partials (one per chunk of <= 256 sphere
+// points: 29 for a radius-3 sphere at h = 0.25), loaded together with clamped indices, then
+// added in chunk order
+__device__ __forceinline__ double proj_sum(const double* __restrict__ partial, const double* __restrict__ scals,
+                                           int4 w, int pjmax, int L, int l) {
+  if (w.w < 0) return 0.0;
+  double s = 0.0;
+  for (int c = w.x; c < w.y; c += 32) {
+    double v[32];
+#pragma unroll
+    for (int u = 0; u < 32; ++u) v[u] = partial[((size_t)min(c + u, w.y - 1) * pjmax + w.z) * L + l];
+#pragma unroll
+    for (int u = 0; u < 32; ++u)
+      if (c + u < w.y) s += v[u];
+  }
+  return s * scals[w.w];
+}
+
 __device__ __forceinline__ void bra_reduce_body(const BraReduceArgs& r, int bid, int nblk) {
-  const size_t total = (size_t)r.nproj * r.L;
+  const size_t total = (size_t)r.nrow * r.L;
   for (size_t t = bid * (size_t)BLOCK + threadIdx.x; t < total; t += (size_t)nblk * BLOCK) {
     const int i = (int)(t / r.L);
-    const int l = (int)(t - (size_t)i * r.L);
-    const int a = r.proj_mat[i];
-    const int j = i - r.mat_pbase[a];
-    double s = 0.0;
-    const int c0 = r.mat_chunk0[a], c1 = r.mat_chunk0[a + 1];
-    // a matrix's partials (one per chunk of <= 256 sphere points: 29 for a radius-3
-    // sphere at h = 0.25) are loaded together, clamped indices, then added in chunk order
-    for (int c = c0; c < c1; c += 32) {
-      double v[32];
-#pragma unroll
-      for (int u = 0; u < 32; ++u) v[u] = r.partial[((size_t)min(c + u, c1 - 1) * r.pjmax + j) * r.L + l];
-#pragma unroll
-      for (int u = 0; u < 32; ++u)
-        if (c + u < c1) s += v[u];
-    }
-    r.proj[t] = s * r.scals[i];
+    r.proj[t] = proj_sum(r.partial, r.scals, r.row[i], r.pjmax, r.L, (int)(t - (size_t)i * r.L));
   }
 }
 
@@ -283,200 +285,171 @@ int launch_bra_mfma(const BraArgs& b, const double* pt, int pjs, int nchunk, hip
   return OCTHIP_SUCCESS;
 }
 
-// One workgroup per bra chunk (<= BRA_CHUNK sphere points of one matrix).  MFMA form:
-// D(16 points x 16 lanes) = A(16 points x 4 projectors) B(4 projectors x 16 lanes); lane
-// (kk, ii) supplies A[ii][kk] = P[q0+ii, jb+kk] and B[kk][ii] = proj[pbase+jb+kk, col];
-// accumulator element r of lane (kk, ii) is D[4r+kk][ii].
-// One workgroup per (chunk, lane tile of 16 TW lanes); the 4 waves take the chunk's groups
-// of 16 sphere points in turn.  Loads are unconditional (clamped indices, zero operands).
+// One workgroup per (KET_GROUPS groups, lane tile of 16 TW lanes), a group per wave.  MFMA form: D(16 rows x 16 lanes) = A(16 rows x 4
+// projectors) B(4 projectors x 16 lanes); lane (kk, ii) supplies A[ii][kk] = P[row ii, kk]
+// and B[kk][ii] = proj[kk, col] of the step; accumulator element r of lane (kk, ii) is
+// D[4r+kk][ii].  Operands past a group's rows are clamped: their D rows are not stored.
 // TW = 2: 32-lane tiles, lane ii computes columns 2ii and 2ii+1 with two MFMAs that share
 // the projector operand and stores them as one 16-byte piece (one complex value); each
 // column's sum is the TW = 1 sum, in the same order.
-template <int TW>
-__device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int c, int lt, double* sproj) {
-  const int4 ch = k.chunks[c];
-  const int4 mi = k.mat_info[ch.x];
-  const int npj = mi.y, mapoff = mi.w;
-  const int pb = k.mat_pbase[ch.x];
-  const int wave = threadIdx.x >> 6, ln = threadIdx.x & 63;
+// A wave's loads are a chain of round trips (group, then its operands), which is what
+// bounds this kernel: a group's record holds its first KET_AHEAD steps, whose operands are
+// loaded together, and a wave has one group.
+template <int TW, bool PHASE, bool SUMS>
+__device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt, double* sproj) {
+  constexpr int TL = 16 * TW;                 // lanes of the tile
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+  const int g = b * KET_GROUPS + wave;
   const int kk = ln >> 4, ii = ln & 15;
-  constexpr int TL = 16 * TW;               // lanes of the tile
-  const int col = lt * TL + ii * TW;        // first column of this lane
-  const int ngrp = (ch.z - ch.y + 15) >> 4;  // <= 16: each wave takes at most 4 groups
-  static_assert(BRA_CHUNK <= 256, "4 groups of 16 sphere points per wave");
-  // projector values of the first 4 projectors of this wave's groups, loaded before the
-  // projections are formed so that both sets of loads are in flight together
-  double apre[4];
+  const int col = lt * TL + ii * TW;          // first column of this lane
+  const KetGroup gr = k.grp[min(g, k.ngrp - 1)];
+  const int n = gr.rows, ns = gr.steps;
+  const double* const pt = k.pt + 4 * ((size_t)gr.line + min(ii, n - 1)) + kk;
+  const double* const pj = SUMS ? sproj + kk * TL + ii * TW : k.proj + (size_t)kk * k.L + col;
+  const size_t ldp = SUMS ? TL : k.L;
+  double av[KET_AHEAD];
+  Vec<TW> bv[KET_AHEAD];
 #pragma unroll
-  for (int gi = 0; gi < 4; ++gi) {
-    const int q = ch.y + (wave + 4 * gi) * 16 + ii;
-    apre[gi] = k.pt[(size_t)(mapoff + (q < ch.z ? q : ch.y)) * k.pjs + (kk < npj ? kk : npj - 1)];
-  }
-  if (k.partial) {
-    // proj[pb + j, lt * TL + i] for j < npj, i < TL: the bra_reduce_body sum, same order
-    const int c0 = k.mat_chunk0[ch.x], c1 = k.mat_chunk0[ch.x + 1];
-    for (int t = threadIdx.x; t < npj * TL; t += BLOCK) {
-      const int j = t / TL, l = lt * TL + (t % TL);
-      double s = 0.0;
-      for (int c = c0; c < c1; c += 32) {
-        double v[32];
-#pragma unroll
-        for (int u = 0; u < 32; ++u) v[u] = k.partial[((size_t)min(c + u, c1 - 1) * k.pjmax + j) * k.L + l];
-#pragma unroll
-        for (int u = 0; u < 32; ++u)
-          if (c + u < c1) s += v[u];
-      }
-      sproj[t] = s * k.scals[pb + j];
-    }
+  for (int u = 0; u < KET_AHEAD; ++u) av[u] = pt[4 * (size_t)(min(u, ns - 1) * n)];
+  if constexpr (SUMS) {
+    const int2 bl = k.blk[b];
+    for (int t = threadIdx.x; t < bl.y * TL; t += BLOCK)
+      sproj[t] = proj_sum(k.partial, k.scals, k.sum[bl.x + t / TL], k.pjmax, k.L, lt * TL + (t % TL));
     __syncthreads();
   }
+  if (g >= k.ngrp) return;
+  d4 acc[TW], tot[TW];
 #pragma unroll
-  for (int gi = 0; gi < 4; ++gi) {
-    const int g = wave + 4 * gi;
-    if (g >= ngrp) break;
-    const int pt0 = ch.y + g * 16;
-    const int q = pt0 + ii;
-    const int qs = q < ch.z ? q : ch.y;
-    d4 acc[TW];
-#pragma unroll
-    for (int w = 0; w < TW; ++w) acc[w] = d4{0.0, 0.0, 0.0, 0.0};
-    for (int jb = 0; jb < npj; jb += 4) {
-      const bool jok = jb + kk < npj;
-      const int jj = jok ? jb + kk : npj - 1;
-      const double a = jb == 0 ? apre[gi] : k.pt[(size_t)(mapoff + qs) * k.pjs + jj];
-      const Vec<TW> bb = k.partial ? ldv<TW>(sproj + jj * TL + ii * TW) : ldv<TW>(k.proj + (size_t)(pb + jj) * k.L + col);
-#pragma unroll
-      for (int w = 0; w < TW; ++w)
-        acc[w] = __builtin_amdgcn_mfma_f64_16x16x4f64((q < ch.z && jok) ? a : 0.0, jok ? bb.v[w] : 0.0, acc[w], 0, 0, 0);
-    }
-    if (k.pphase) {
-      // ket row of point qo times conj(its Bloch phase): with TW = 2 the lane holds the
-      // (re, im) pair, otherwise lanes ii ^ 1 hold the pair
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int qo = pt0 + 4 * r + kk;
-        const size_t pi2 = 2 * (size_t)(mapoff + (qo < ch.z ? qo : ch.y));
-        if constexpr (TW == 2) {
-          const double re = zmul_lane(k.pphase[pi2], -k.pphase[pi2 + 1], acc[0][r], acc[1][r], false);
-          const double im = zmul_lane(k.pphase[pi2], -k.pphase[pi2 + 1], acc[1][r], acc[0][r], true);
-          acc[0][r] = re;
-          acc[1][r] = im;
-        } else {
-          const double xq = __shfl_xor(acc[0][r], 1);
-          acc[0][r] = zmul_lane(k.pphase[pi2], -k.pphase[pi2 + 1], acc[0][r], xq, (col & 1) != 0);
-        }
-      }
-    }
+  for (int w = 0; w < TW; ++w) acc[w] = tot[w] = d4{0.0, 0.0, 0.0, 0.0};
+  int ent = 0;                                // PHASE: first entry of the matrix in acc
+  const auto flush = [&]() {
+    // tot += the matrix's term of row 4r+kk times conj(its Bloch phase): with TW = 2 the
+    // lane holds the (re, im) pair, otherwise lanes ii ^ 1 hold the pair
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int qo = pt0 + 4 * r + kk;
-      if (qo < ch.z) {
-        Vec<TW> o;
-#pragma unroll
-        for (int w = 0; w < TW; ++w) o.v[w] = acc[w][r];
-        stv<TW>(k.kbuf + (size_t)(mapoff + qo) * k.L + col, o);
+      const size_t pi2 = 2 * (size_t)k.kg[ent + min(4 * r + kk, n - 1)];
+      const double pr = k.pphase[pi2], pi = -k.pphase[pi2 + 1];
+      if constexpr (TW == 2) {
+        tot[0][r] += zmul_lane(pr, pi, acc[0][r], acc[1][r], false);
+        tot[1][r] += zmul_lane(pr, pi, acc[1][r], acc[0][r], true);
+      } else {
+        tot[0][r] += zmul_lane(pr, pi, acc[0][r], __shfl_xor(acc[0][r], 1), (col & 1) != 0);
       }
     }
-  }
-}
-
-__global__ __launch_bounds__(BLOCK) void k_ket_mfma(const KetArgs k) {
-  __shared__ double2 sproj2[KET_FUSE_PJMAX * 16];  // 16-byte aligned: read as lane pairs
-  double* const sproj = reinterpret_cast<double*>(sproj2);
-  if ((k.L & 31) == 0) {
-    const int nlt = k.L >> 5;
-    ket_mfma_body<2>(k, blockIdx.x / nlt, blockIdx.x % nlt, sproj);
-  } else {
-    const int nlt = k.L >> 4;
-    ket_mfma_body<1>(k, blockIdx.x / nlt, blockIdx.x % nlt, sproj);
-  }
-}
-
-// plain form, any row length: one thread per (sphere point, lane)
-__device__ __forceinline__ void ket_plain_body(const KetArgs& k, int c) {
-  const int4 ch = k.chunks[c];
-  const int4 mi = k.mat_info[ch.x];
-  const int npj = mi.y, mapoff = mi.w;
-  const int pb = k.mat_pbase[ch.x];
-  const int total = (ch.z - ch.y) * k.L;
-  for (int t = threadIdx.x; t < total; t += BLOCK) {
-    const int q = ch.y + t / k.L, l = t % k.L;
-    const double* prow = k.pt + (size_t)(mapoff + q) * k.pjs;
-    double acc = 0.0;
-    for (int jj = 0; jj < npj; ++jj) acc = fma(prow[jj], k.proj[(size_t)(pb + jj) * k.L + l], acc);
-    if (k.pphase) {
-      double accq = 0.0;  // the other lane of the (re, im) pair
-      for (int jj = 0; jj < npj; ++jj) accq = fma(prow[jj], k.proj[(size_t)(pb + jj) * k.L + (l ^ 1)], accq);
-      const size_t pi2 = 2 * (size_t)(mapoff + q);
-      acc = zmul_lane(k.pphase[pi2], -k.pphase[pi2 + 1], acc, accq, (l & 1) != 0);
+  };
+  for (int q0 = 0; q0 < ns; q0 += KET_AHEAD) {
+    if (q0 > 0) {
+#pragma unroll
+      for (int u = 0; u < KET_AHEAD; ++u) av[u] = pt[4 * (size_t)(min(q0 + u, ns - 1) * n)];
     }
-    k.kbuf[(size_t)(mapoff + q) * k.L + l] = acc;
-  }
-}
-
-// one thread per (multi-sphere mesh point, LPT consecutive lanes of its row)
-template <int LPT>
-__device__ __forceinline__ void ket_sum_lanes(const KetArgs& k, int bid, int nblk) {
-  const int lp = k.L / LPT;
-  const size_t total = (size_t)k.nmulti * lp;
-  for (size_t t = bid * (size_t)BLOCK + threadIdx.x; t < total; t += (size_t)nblk * BLOCK) {
-    const int m = (int)(t / lp);
-    const int l = (int)(t - (size_t)m * lp) * LPT;
-    Vec<LPT> s;
 #pragma unroll
-    for (int q = 0; q < LPT; ++q) s.v[q] = 0.0;
-    const int e0 = k.multi_pos[m], e1 = k.multi_pos[m + 1];
-    // rows in groups of 4 loaded together (clamped indices), added in entry order
-    for (int e = e0; e < e1; e += 4) {
-      Vec<LPT> v[4];
+    for (int u = 0; u < KET_AHEAD; ++u) {
+      const int2 q = q0 == 0 ? gr.ahead[u] : *reinterpret_cast<const int2*>(k.step + gr.step + min(q0 + u, ns - 1));
+      bv[u] = ldv<TW>(pj + (SUMS ? q.x : q.y) * ldp);
+    }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = ldv<LPT>(k.kbuf + (size_t)k.multi_g[min(e + u, e1 - 1)] * k.L + l);
+    for (int u = 0; u < KET_AHEAD; ++u) {
+      if (q0 + u >= ns) break;
+      if constexpr (PHASE) {
+        const int z = k.step[gr.step + q0 + u].z;
+        if (z >= 0) {
+          if (q0 + u > 0) flush();
+          ent = z;
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (e + u < e1) {
-#pragma unroll
-          for (int q = 0; q < LPT; ++q) s.v[q] = s.v[q] + v[u].v[q];
+          for (int w = 0; w < TW; ++w) acc[w] = d4{0.0, 0.0, 0.0, 0.0};
         }
+      }
+#pragma unroll
+      for (int w = 0; w < TW; ++w) acc[w] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], bv[u].v[w], acc[w], 0, 0, 0);
     }
-    stv<LPT>(k.kbuf + ((size_t)k.total_points + m) * k.L + l, s);
+  }
+  if constexpr (PHASE) {
+    flush();
+#pragma unroll
+    for (int w = 0; w < TW; ++w) acc[w] = tot[w];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (4 * r + kk < n) {
+      Vec<TW> o;
+#pragma unroll
+      for (int w = 0; w < TW; ++w) o.v[w] = acc[w][r];
+      stv<TW>(k.kbuf + (size_t)(gr.row + 4 * r + kk) * k.L + col, o);
+    }
   }
 }
 
-__device__ __forceinline__ void ket_sum_body(const KetArgs& k, int bid, int nblk) {
-  if (k.L & 1) ket_sum_lanes<1>(k, bid, nblk);
-  else ket_sum_lanes<2>(k, bid, nblk);
+template <bool PHASE, bool SUMS>
+__device__ __forceinline__ void ket_mfma(const KetArgs& k, int b) {
+  __shared__ double2 sproj2[SUMS ? KET_SUMS / 2 : 1];  // 16-byte aligned: read as lane pairs
+  double* const sproj = reinterpret_cast<double*>(sproj2);
+  const int nlt = mfma_lane_tiles(k.L);
+  if ((k.L & 31) == 0) ket_mfma_body<2, PHASE, SUMS>(k, b / nlt, b % nlt, sproj);
+  else ket_mfma_body<1, PHASE, SUMS>(k, b / nlt, b % nlt, sproj);
 }
 
+// plain form, any row length: a wave per group, one thread per (row, lane)
+__device__ __forceinline__ void ket_plain_body(const KetArgs& k, int b) {
+  static_assert(KET_GROUPS == BLOCK / 64, "a group per wave");
+  const int g = b * KET_GROUPS + (threadIdx.x >> 6);
+  if (g < k.ngrp) {
+    const KetGroup& gr = k.grp[g];
+    const int n = gr.rows, ns = gr.steps;
+    for (int t = threadIdx.x & 63; t < n * k.L; t += 64) {
+      const int r = t / k.L, l = t - r * k.L;
+      double tot = 0.0, acc = 0.0, accq = 0.0;  // accq: the other lane of the (re, im) pair
+      int ent = 0;
+      for (int q = 0; q <= ns; ++q) {
+        const int4 s = q < ns ? k.step[gr.step + q] : make_int4(0, 0, 0, 0);
+        if (k.pphase && q > 0 && s.z >= 0) {
+          const size_t pi2 = 2 * (size_t)k.kg[ent + r];
+          tot += zmul_lane(k.pphase[pi2], -k.pphase[pi2 + 1], acc, accq, (l & 1) != 0);
+          acc = accq = 0.0;
+        }
+        if (q == ns) break;
+        if (s.z >= 0) ent = s.z;
+        const double* a = k.pt + 4 * (size_t)(gr.line + q * n + r);
+        const double* pj = k.proj + (size_t)s.y * k.L;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = fma(a[j], pj[(size_t)j * k.L + l], acc);
+        if (k.pphase) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) accq = fma(a[j], pj[(size_t)j * k.L + (l ^ 1)], accq);
+        }
+      }
+      k.kbuf[(size_t)(gr.row + r) * k.L + l] = k.pphase ? tot : acc;
+    }
+  }
+}
+
+template <bool PHASE, bool SUMS>
+__global__ __launch_bounds__(BLOCK) void k_ket_mfma(const KetArgs k) { ket_mfma<PHASE, SUMS>(k, blockIdx.x); }
 __global__ __launch_bounds__(BLOCK) void k_ket_plain(const KetArgs k) { ket_plain_body(k, blockIdx.x); }
-__global__ __launch_bounds__(BLOCK) void k_ket_sum(const KetArgs k) { ket_sum_body(k, blockIdx.x, gridDim.x); }
 
-int launch_ket(const KetArgs& k, int nchunk, bool mfma, hipStream_t s) {
-  if (nchunk <= 0) return OCTHIP_SUCCESS;
-  if (k.partial && !(mfma && k.L >= 16 && k.pjmax <= KET_FUSE_PJMAX))
-    return fail(OCTHIP_ERR_INVALID, "k_ket: projections from partials need the MFMA form and <= %d projectors",
-                KET_FUSE_PJMAX);
-  {
-    ProfScope prof("k_ket", s);
-    if (mfma && k.L >= 16)  // 32-lane tiles when the row length allows, else 16-lane tiles
-      hipLaunchKernelGGL(k_ket_mfma, dim3(nchunk * mfma_lane_tiles(k.L)), dim3(BLOCK), 0, s, k);
-    else
-      hipLaunchKernelGGL(k_ket_plain, dim3(nchunk), dim3(BLOCK), 0, s, k);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(OCTHIP_ERR_HIP, "k_ket launch: %s", hipGetErrorString(e));
-  }
-  // one thread per lane pair of each multi-sphere point (per lane for odd row lengths)
-  const size_t total = (size_t)k.nmulti * ((k.L & 1) ? k.L : k.L / 2);
-  if (total == 0) return OCTHIP_SUCCESS;
-  const int grid = (int)std::min<size_t>((total + BLOCK - 1) / BLOCK, 8192);
-  ProfScope prof("k_ket_sum", s);
-  hipLaunchKernelGGL(k_ket_sum, dim3(grid), dim3(BLOCK), 0, s, k);
+int launch_ket(const KetArgs& k, bool mfma, hipStream_t s) {
+  const int nblock = ket_blocks(k.ngrp);
+  if (nblock <= 0) return OCTHIP_SUCCESS;
+  mfma = mfma && k.L >= 16;
+  if (k.partial && !mfma) return fail(OCTHIP_ERR_INVALID, "k_ket: projections from partials need the MFMA form");
+  ProfScope prof("k_ket", s);
+  const dim3 tiles(nblock * mfma_lane_tiles(k.L));  // 32-lane tiles when the row length allows, else 16
+  if (mfma && k.pphase && k.partial)
+    hipLaunchKernelGGL((k_ket_mfma<true, true>), tiles, dim3(BLOCK), 0, s, k);
+  else if (mfma && k.pphase)
+    hipLaunchKernelGGL((k_ket_mfma<true, false>), tiles, dim3(BLOCK), 0, s, k);
+  else if (mfma && k.partial)
+    hipLaunchKernelGGL((k_ket_mfma<false, true>), tiles, dim3(BLOCK), 0, s, k);
+  else if (mfma)
+    hipLaunchKernelGGL((k_ket_mfma<false, false>), tiles, dim3(BLOCK), 0, s, k);
+  else
+    hipLaunchKernelGGL(k_ket_plain, dim3(nblock), dim3(BLOCK), 0, s, k);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(OCTHIP_ERR_HIP, "k_ket_sum launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return fail(OCTHIP_ERR_HIP, "k_ket launch: %s", hipGetErrorString(e));
   return OCTHIP_SUCCESS;
 }
 
 int launch_bra_reduce(const BraReduceArgs& r, hipStream_t s) {
-  const size_t total = (size_t)r.nproj * r.L;
+  const size_t total = (size_t)r.nrow * r.L;
   if (total == 0) return OCTHIP_SUCCESS;
   int grid = (int)((total + BLOCK - 1) / BLOCK);
   if (grid > 4096) grid = 4096;
@@ -527,21 +500,13 @@ __global__ __launch_bounds__(BLOCK) void k_bra_reduce_multi(const BraReduceArgs*
 __global__ __launch_bounds__(BLOCK) void k_ket_mfma_multi(const KetArgs* __restrict__ a,
                                                           const int* __restrict__ off, int nseg) {
   const int i = segment_of(off, nseg, blockIdx.x);
-  __shared__ double2 sproj2[KET_FUSE_PJMAX * 16];  // 16-byte aligned: read as lane pairs
-  double* const sproj = reinterpret_cast<double*>(sproj2);
-  const int b = blockIdx.x - off[i], nlt = mfma_lane_tiles(a[i].L);
-  if ((a[i].L & 31) == 0) ket_mfma_body<2>(a[i], b / nlt, b % nlt, sproj);
-  else ket_mfma_body<1>(a[i], b / nlt, b % nlt, sproj);
+  const KetArgs k = a[i];
+  ket_mfma<false, false>(k, blockIdx.x - off[i]);
 }
 __global__ __launch_bounds__(BLOCK) void k_ket_plain_multi(const KetArgs* __restrict__ a,
                                                            const int* __restrict__ off, int nseg) {
   const int i = segment_of(off, nseg, blockIdx.x);
   ket_plain_body(a[i], blockIdx.x - off[i]);
-}
-__global__ __launch_bounds__(BLOCK) void k_ket_sum_multi(const KetArgs* __restrict__ a,
-                                                         const int* __restrict__ off, int nseg) {
-  const int i = segment_of(off, nseg, blockIdx.x);
-  ket_sum_body(a[i], blockIdx.x - off[i], off[i + 1] - off[i]);
 }
 __global__ __launch_bounds__(BLOCK) void k_zero_multi(const ZeroArgs* __restrict__ a,
                                                       const int* __restrict__ off, int nseg) {
@@ -565,12 +530,12 @@ int launch_multi(int kind, const void* args, const int* off, int nseg, int nbloc
   switch (kind) {
     case MULTI_BRA_MFMA: {
       ProfScope prof("k_bra", s);
-      hipLaunchKernelGGL(k_bra_mfma_multi, g, b, 0, s, (const BraMfmaArgs*)args, off, nseg);
+      hipLaunchKernelGGL(k_bra_mfma_multi, g, dim3(BLOCK), 0, s, (const BraMfmaArgs*)args, off, nseg);
       return check_launch("k_bra_mfma_multi");
     }
     case MULTI_BRA_PLAIN: {
       ProfScope prof("k_bra", s);
-      hipLaunchKernelGGL(k_bra_plain_multi, g, b, 0, s, (const BraMfmaArgs*)args, off, nseg);
+      hipLaunchKernelGGL(k_bra_plain_multi, g, dim3(BLOCK), 0, s, (const BraMfmaArgs*)args, off, nseg);
       return check_launch("k_bra_plain_multi");
     }
     case MULTI_BRA_REDUCE: {
@@ -587,11 +552,6 @@ int launch_multi(int kind, const void* args, const int* off, int nseg, int nbloc
       ProfScope prof("k_ket", s);
       hipLaunchKernelGGL(k_ket_plain_multi, g, b, 0, s, (const KetArgs*)args, off, nseg);
       return check_launch("k_ket_plain_multi");
-    }
-    case MULTI_KET_SUM: {
-      ProfScope prof("k_ket_sum", s);
-      hipLaunchKernelGGL(k_ket_sum_multi, g, b, 0, s, (const KetArgs*)args, off, nseg);
-      return check_launch("k_ket_sum_multi");
     }
     case MULTI_ZERO: {
       ProfScope prof("k_zero_rows", s);

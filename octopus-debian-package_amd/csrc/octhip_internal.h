@@ -169,6 +169,9 @@ struct octhip_nl_operator_s {
   std::deque<ZPlan> plans;               // a deque: callers keep references
 };
 
+namespace octhip {
+struct KetGroup;
+}
 struct octhip_hamiltonian_s {
   octhip_nl_operator_t kin = nullptr;
   double mass = 1.0;
@@ -181,7 +184,6 @@ struct octhip_hamiltonian_s {
   // projectors
   int nmat = 0;
   int max_nprojs = 0;
-  int full_projection_size = 0;
   int total_points = 0;
   int pjs = 0;                  // row stride of the transposed projector table
   std::vector<int> offsets;     // 6*nmat host copy
@@ -189,19 +191,23 @@ struct octhip_hamiltonian_s {
   int* d_maps = nullptr;        // 1-based
   double* d_scals = nullptr;
   double* d_pt = nullptr;       // total_points x pjs (row-major, transposed blocks)
-  int* d_mat_pbase = nullptr;   // nmat: offset of the matrix's projections
-  int* d_mat_npj = nullptr;     // nmat: nprojs
   // bra chunking: chunk c = (matrix, first sphere point, last+1)
   int nchunk = 0;
   int4* d_chunks = nullptr;     // {matrix, q0, q1, 0}
-  int* d_mat_chunk0 = nullptr;  // nmat+1 first chunk of each matrix
   int4* d_mat_info = nullptr;   // nmat: {npoints, nprojs, matrix offset, map offset}
-  int* d_proj_mat = nullptr;    // projection index -> matrix
   int nslot = 0;                // mesh points inside at least one sphere
-  int nmulti = 0;               // mesh points inside several spheres
   int* d_kslot = nullptr;       // np: row of the ket buffer of each mesh point + 1, or 0
-  int* d_multi_pos = nullptr;   // nmulti+1
-  int* d_multi_g = nullptr;     // sphere points of the multi-sphere mesh points
+  // ket tables (KetArgs): groups of rows with one set of matrices, blocks of groups
+  int nkgrp = 0;
+  int ket_sums = 0;             // most projection rows of the groups of one ket workgroup
+  octhip::KetGroup* d_kgrp = nullptr;
+  int4* d_kstep = nullptr;
+  int2* d_kblk = nullptr;
+  int4* d_ksumrow = nullptr;
+  double* d_kpt = nullptr;      // lines of 4 projector values
+  int* d_kg = nullptr;          // sphere point of each (group, matrix, row)
+  int nprow = 0;                // projection rows: 4 ceil(nprojs / 4) a matrix
+  int4* d_prow = nullptr;       // BraReduceArgs::row
   // Work buffers, one set per stream: applies on different streams (Octopus gives every
   // batch its own stream, accel_set_stream) may run concurrently.  The set of the stream
   // of the current call is mirrored in the fields below; sets captured into a graph are
@@ -225,8 +231,8 @@ struct octhip_hamiltonian_s {
   std::vector<octhip_taylor_graph_t> graphs;
   int work_ldf = -1;
   double* d_partial = nullptr;  // nchunk * max_nprojs * L
-  double* d_proj = nullptr;     // full_projection_size * L
-  double* d_ksum = nullptr;     // (total_points + nmulti) * L ket rows
+  double* d_proj = nullptr;     // nprow * L
+  double* d_ksum = nullptr;     // nslot * L ket rows
   double* d_y[3] = {nullptr, nullptr, nullptr};  // Taylor powers H^k psi, np rows each
   int y_ldf = -1;
   std::vector<void*> retired;   // work buffers outgrown by a larger ldf, freed at destroy

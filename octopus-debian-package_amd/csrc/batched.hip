@@ -83,6 +83,8 @@ struct octhip_batched_s {
   int order = 4;
   double dt = 0.0;
   bool mfma = true, nl = false;
+  int bra_kind = MULTI_BRA_PLAIN;
+  size_t bra_lds = 0;                   // of the widest pair
   int lc = 16, lpt = 2;
   std::complex<double> zf[33];
   Seg zero, reduce, ket;
@@ -125,23 +127,16 @@ int build_bra(octhip_batched_s* b, const std::vector<const double*>& in, Seg& ou
     const Pair& p = b->pairs[i];
     const octhip_hamiltonian_s* h = p.h;
     BraMfmaArgs m;
-    std::memset(&m, 0, sizeof(m));
+    bra_mfma_args(h, p.L, p.partial, m);
     m.b.psi = in[i];
-    m.b.L = p.L;
-    m.b.chunks = h->d_chunks;
-    m.b.mat_info = h->d_mat_info;
-    m.b.mats = h->d_matrices;
-    m.b.maps = h->d_maps;
-    m.b.partial = p.partial;
-    m.b.pjmax = h->max_nprojs;
-    m.pt = h->d_pt;
-    m.pjs = h->pjs;
+    m.b.pphase = m.set.phase = nullptr;  // finite systems
+    if (!b->mfma) m.b.pjmax = h->max_nprojs;
     if (b->nl && !(m.b.psi && m.b.partial && m.b.chunks && m.b.maps && m.pt))
       return fail(OCTHIP_ERR_STATE, "batched: incomplete bra arguments for pair %zu", i);
     args.push_back(m);
-    // MFMA bra: one block per (chunk, lane tile of 32, or of 16 when 32 does not divide
-    // the row); plain bra: one per chunk
-    blocks.push_back(h->nmat > 0 ? h->nchunk * (b->mfma ? mfma_lane_tiles(p.L) : 1) : 0);
+    // MFMA bra: one block per (chunk or block of groups, lane tile of 32, or of 16 when 32
+    // does not divide the row); plain bra: one per chunk
+    blocks.push_back(h->nmat == 0 ? 0 : b->mfma ? bra_mfma_blocks(h, p.L) : h->nchunk);
   }
   return make_seg(args, blocks, out);
 }
@@ -224,7 +219,7 @@ int build_zdesc(octhip_batched_s* b, int k, ZArgs** out) {
 
 int run_bra(octhip_batched_s* b, const Seg& bra, hipStream_t s) {
   if (!b->nl) return OCTHIP_SUCCESS;
-  int rc = launch_multi(b->mfma ? MULTI_BRA_MFMA : MULTI_BRA_PLAIN, bra.args, bra.off, bra.nseg, bra.nblocks, s);
+  int rc = launch_multi(b->bra_kind, bra.args, bra.off, bra.nseg, bra.nblocks, s, b->bra_lds);
   if (!rc) rc = launch_multi(MULTI_BRA_REDUCE, b->reduce.args, b->reduce.off, b->reduce.nseg, b->reduce.nblocks, s);
   if (!rc) rc = launch_multi(b->mfma ? MULTI_KET_MFMA : MULTI_KET_PLAIN, b->ket.args, b->ket.off, b->ket.nseg,
                              b->ket.nblocks, s);
@@ -272,6 +267,9 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
   b->lpt = 2;
   b->mfma = minL >= 16;
   for (int i = 0; i < npairs; ++i) b->mfma = b->mfma && hms[i]->use_mfma;
+  if (b->mfma) b->bra_kind = MULTI_BRA_SETS;
+  for (int i = 0; i < npairs; ++i)
+    if (b->mfma && !bra_by_sets(hms[i])) b->bra_kind = MULTI_BRA_MFMA;
   taylor_coefs(deltat, 0, order, b->zf);
   const int resident[2] = {zmarch_resident(b->lc, b->lpt, EPI_STORE, b->nl, true),
                            zmarch_resident(b->lc, b->lpt, EPI_TAYLOR, b->nl, true)};
@@ -286,7 +284,7 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
     const octhip_hamiltonian_s* h = p.h;
     const size_t L = (size_t)p.L;
     if (b->nl) {
-      rc = dalloc((void**)&p.partial, sizeof(double) * h->nchunk * h->max_nprojs * L);
+      rc = dalloc((void**)&p.partial, sizeof(double) * partial_doubles(h, L));
       if (!rc) rc = dalloc((void**)&p.proj, sizeof(double) * h->nprow * L);
       if (!rc) rc = dalloc((void**)&p.ksum, sizeof(double) * h->nslot * L);
     }
@@ -338,13 +336,15 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
       r.scals = h->d_scals;
       r.proj = p.proj;
       r.L = p.L;
-      r.pjmax = h->max_nprojs;
+      r.sets = b->mfma && bra_by_sets(h);
+      r.pjmax = r.sets ? (h->max_nprojs + 3) / 4 * 4 : h->max_nprojs;
+      if (b->mfma) b->bra_lds = std::max(b->bra_lds, bra_mfma_lds(h, p.L));
       r.nrow = b->nl ? h->nprow : 0;
       ra.push_back(r);
-      rb.push_back(blocks_for((size_t)r.nrow * p.L, 4096));
+      rb.push_back(bra_reduce_blocks(r));
       KetArgs k;
-      ket_args(h, p.L, p.partial, p.proj, p.ksum, false, k);
-      k.pphase = nullptr;  // finite systems
+      ket_args(h, p.L, p.proj, p.ksum, k);
+      k.phase = nullptr;  // finite systems
       ka.push_back(k);
       kb.push_back(b->nl ? ket_blocks(h->nkgrp) * (b->mfma ? mfma_lane_tiles(p.L) : 1) : 0);
     }

@@ -10,8 +10,7 @@ using namespace octhip;
 
 namespace octhip {
 void stencil_args(const octhip_nl_operator_s* op, double factor, ApplyArgs& a);
-int launch_bra_mfma(const BraArgs& b, const double* pt, int pjs, int nchunk, hipStream_t s, double* zf = nullptr,
-                    size_t zfirst = 0, size_t zcount = 0);
+int launch_bra_mfma(BraMfmaArgs& m, size_t lds, hipStream_t s);
 int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t s);
 int prepare_operator(octhip_nl_operator_s* op, int L, bool nl);
 }  // namespace octhip
@@ -52,7 +51,7 @@ int ensure_work(octhip_hamiltonian_s* h, int ldf, hipStream_t s) {
     const size_t L = (size_t)1 << ldf;
     int rc = OCTHIP_SUCCESS;
     if (h->nmat > 0) {
-      rc = dalloc((void**)&w.partial, sizeof(double) * h->nchunk * h->max_nprojs * L);
+      rc = dalloc((void**)&w.partial, sizeof(double) * partial_doubles(h, L));
       if (!rc) rc = dalloc((void**)&w.proj, sizeof(double) * h->nprow * L);
       if (!rc) rc = dalloc((void**)&w.ksum, sizeof(double) * std::max(h->nslot, 1) * L);
     }
@@ -85,40 +84,40 @@ int ensure_taylor(octhip_hamiltonian_s* h, int ldf, hipStream_t s) {
 // boundary rows are cleared on the way (fused into the bra launch when it can be)
 int run_bra(octhip_hamiltonian_s* h, const double* f, int L, hipStream_t s, double* zero_bc = nullptr) {
   const int np = h->kin->np, np_part = h->kin->np_part;
-  if (h->nmat == 0) return zero_bc ? zero_boundary(zero_bc, np, np_part, L, s) : OCTHIP_SUCCESS;
+  if (h->nchunk == 0) return zero_bc ? zero_boundary(zero_bc, np, np_part, L, s) : OCTHIP_SUCCESS;
   const bool mfma = h->use_mfma && L >= 16;
   if (zero_bc && !mfma) {
     int rc = zero_boundary(zero_bc, np, np_part, L, s);
     if (rc) return rc;
     zero_bc = nullptr;
   }
-  BraArgs b;
-  b.psi = f;
-  b.L = L;
-  b.chunks = h->d_chunks;
-  b.mat_info = h->d_mat_info;
-  b.mats = h->d_matrices;
-  b.maps = h->d_maps;
-  b.partial = h->d_partial;
-  b.pjmax = h->max_nprojs;
-  b.pphase = h->has_kpoint ? h->d_pphase : nullptr;
-  int rc = mfma ? launch_bra_mfma(b, h->d_pt, h->pjs, h->nchunk, s, zero_bc, (size_t)np * L,
-                                  (size_t)(np_part - np) * L)
-                : launch_bra(b, h->nchunk, false, s);
+  BraMfmaArgs m;
+  bra_mfma_args(h, L, h->d_partial, m);
+  m.b.psi = f;
+  m.zf = zero_bc;
+  m.zfirst = (size_t)np * L;
+  m.zcount = zero_bc ? (size_t)(np_part - np) * L : 0;
+  int rc;
+  if (mfma) {
+    rc = launch_bra_mfma(m, bra_mfma_lds(h, L), s);
+  } else {
+    m.b.pjmax = h->max_nprojs;
+    rc = launch_bra(m.b, h->nchunk, false, s);
+  }
   if (rc) return rc;
-  const bool sums = mfma && ket_sums_partials(h, L);
   BraReduceArgs r;
   r.partial = h->d_partial;
   r.row = h->d_prow;
   r.scals = h->d_scals;
   r.proj = h->d_proj;
   r.L = L;
-  r.pjmax = h->max_nprojs;
+  r.pjmax = m.b.pjmax;
   r.nrow = h->nprow;
-  if (!sums) rc = launch_bra_reduce(r, s);
+  r.sets = mfma && m.sets;
+  rc = launch_bra_reduce(r, s);
   if (rc) return rc;
   KetArgs k;
-  ket_args(h, L, h->d_partial, h->d_proj, h->d_ksum, sums, k);
+  ket_args(h, L, h->d_proj, h->d_ksum, k);
   return launch_ket(k, h->use_mfma, s);
 }
 
@@ -133,32 +132,58 @@ __global__ void k_veff(double* __restrict__ veff, const double* __restrict__ v,
 }  // namespace
 
 namespace octhip {
-bool ket_sums_partials(const octhip_hamiltonian_s* h, int L) {
-  const int tiles = mfma_lane_tiles(L);
-  return h->ket_sums * (L / tiles) <= KET_SUMS && ket_blocks(h->nkgrp) * tiles <= KET_SUM_BLOCKS;
+namespace {
+int padded(int nprojs) { return (nprojs + 3) / 4 * 4; }
+}  // namespace
+
+bool bra_by_sets(const octhip_hamiltonian_s* h) { return h->nsblk > 0; }
+
+size_t partial_doubles(const octhip_hamiltonian_s* h, size_t L) {
+  return std::max((size_t)h->nchunk * h->max_nprojs, (size_t)h->set_parts * padded(h->max_nprojs)) * L;
 }
 
-void ket_args(const octhip_hamiltonian_s* h, int L, const double* partial, const double* proj, double* kbuf,
-              bool sums, KetArgs& k) {
+int bra_mfma_blocks(const octhip_hamiltonian_s* h, int L) {
+  return (bra_by_sets(h) ? h->nsblk : h->nchunk) * mfma_lane_tiles(L);
+}
+
+size_t bra_mfma_lds(const octhip_hamiltonian_s* h, int L) {
+  const size_t lanes = L / mfma_lane_tiles(L);
+  return sizeof(double) * 4 * lanes * (bra_by_sets(h) ? h->set_sums : 16);
+}
+
+void bra_mfma_args(const octhip_hamiltonian_s* h, int L, double* partial, BraMfmaArgs& m) {
+  m = BraMfmaArgs();
+  m.sets = bra_by_sets(h);
+  m.b.L = L;
+  m.b.chunks = h->d_chunks;
+  m.b.mat_info = h->d_mat_info;
+  m.b.mats = h->d_matrices;
+  m.b.maps = h->d_maps;
+  m.b.partial = partial;
+  m.b.pjmax = m.sets ? padded(h->max_nprojs) : h->max_nprojs;
+  m.b.pphase = h->has_kpoint ? h->d_pphase : nullptr;
+  m.set.grp = h->d_kgrp;
+  m.set.step = h->d_kstep;
+  m.set.pt = h->d_kpt;
+  m.set.point = h->d_kpoint;
+  m.set.blk = h->d_sblk;
+  m.set.part = h->d_spart;
+  m.set.phase = h->has_kpoint ? h->d_kphase : nullptr;
+  m.pt = h->d_pt;
+  m.pjs = h->pjs;
+  m.nbra = L >= 16 ? bra_mfma_blocks(h, L) : 0;
+}
+
+void ket_args(const octhip_hamiltonian_s* h, int L, const double* proj, double* kbuf, KetArgs& k) {
   k = KetArgs();
-  if (sums) {
-    k.partial = partial;
-    k.sum = h->d_ksumrow;
-    k.scals = h->d_scals;
-    k.pjmax = h->max_nprojs;
-  }
   k.grp = h->d_kgrp;
   k.ngrp = h->nkgrp;
   k.step = h->d_kstep;
-  k.blk = h->d_kblk;
   k.pt = h->d_kpt;
   k.proj = proj;
   k.kbuf = kbuf;
   k.L = L;
-  if (h->has_kpoint) {
-    k.pphase = h->d_pphase;
-    k.kg = h->d_kg;
-  }
+  k.phase = h->has_kpoint ? h->d_kphase : nullptr;
 }
 
 int zero_boundary(double* f, int np, int np_part, int L, hipStream_t s) {
@@ -283,37 +308,53 @@ int periodic_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, 
 struct KetTables {
   std::vector<int> slot, g;
   std::vector<KetGroup> grp;
-  std::vector<int4> step, sum, prow;
-  std::vector<int2> blk;
+  std::vector<int4> step, sblk;
+  std::vector<ProjRow> prow;
+  std::vector<int> point, spart;
   std::vector<double> pt;
   std::vector<int> matrix;  // matrix of each step
 };
 
 int padded_projs(const octhip_hamiltonian_s* h, int a) { return (h->offsets[6 * (size_t)a + O_PROJS] + 3) / 4 * 4; }
 
-// the sums of each workgroup: the projection rows (from prow0[a]) of its groups' matrices,
-// each once; returns the largest number
-int ket_sums(const octhip_hamiltonian_s* h, const std::vector<int>& prow0, KetTables& t) {
-  int most = 0;
-  std::vector<int> row(h->nmat, -1), open;  // first sum of the matrices of the workgroup
-  for (size_t g0 = 0; g0 < t.grp.size(); g0 += KET_GROUPS) {
-    for (int a : open) row[a] = -1;
-    open.clear();
-    int2 b = make_int2((int)t.sum.size(), 0);
-    const KetGroup& last = t.grp[std::min(g0 + KET_GROUPS, t.grp.size()) - 1];
-    for (int q = t.grp[g0].step; q < last.step + last.steps; ++q) {
-      const int a = t.matrix[q];
-      if (row[a] < 0) {
-        row[a] = b.y;
-        open.push_back(a);
-        for (int j = 0; j < padded_projs(h, a); ++j, ++b.y) t.sum.push_back(t.prow[prow0[a] + j]);
-      }
-      t.step[q].x = row[a] + (t.step[q].y - prow0[a]);
+// blocks of the bra by sets: <= BRA_SET_GROUPS groups and `most` rows of sums
+void set_blocks(octhip_hamiltonian_s* h, int most, KetTables& t) {
+  const int pj = (h->max_nprojs + 3) / 4 * 4;
+  std::vector<int> slot(h->nmat, -1), count(h->nmat, 0), matrix;
+  int first_matrix = 0;
+  for (size_t i = 0; i < t.grp.size(); ++i) {
+    const int s0 = t.grp[i].step, s1 = s0 + t.grp[i].steps;
+    int add = 0;
+    for (int q = s0; q < s1; ++q) add += t.step[q].w && slot[t.matrix[q]] < 0;
+    if (t.sblk.empty() || t.sblk.back().y == BRA_SET_GROUPS || (t.sblk.back().w + add) * pj > most) {
+      for (size_t k = first_matrix; k < matrix.size(); ++k) slot[matrix[k]] = -1;
+      first_matrix = (int)matrix.size();
+      t.sblk.push_back(make_int4((int)i, 0, first_matrix, 0));
     }
-    most = std::max(most, b.y);
-    t.blk.push_back(b);
+    int4& b = t.sblk.back();
+    ++b.y;
+    int j = 0;
+    for (int q = s0; q < s1; ++q) {
+      const int a = t.matrix[q];
+      if (slot[a] < 0) {
+        slot[a] = b.w++;
+        matrix.push_back(a);
+        ++count[a];
+      }
+      j = t.step[q].w ? 0 : j + 4;
+      t.step[q].y = slot[a] * pj + j;
+    }
+    h->set_sums = std::max(h->set_sums, b.w * pj);
   }
-  return most;
+  // the parts of one matrix are consecutive, in block order
+  std::vector<int> first(h->nmat + 1, 0);
+  for (int a = 0; a < h->nmat; ++a) first[a + 1] = first[a] + count[a];
+  h->set_parts = first[h->nmat];
+  size_t row = 0;
+  for (int a = 0; a < h->nmat; ++a)
+    for (int j = 0; j < padded_projs(h, a); ++j) t.prow[row++].part[1] = make_int2(first[a], first[a + 1]);
+  for (int a : matrix) t.spart.push_back(first[a]++);
+  h->nsblk = (int)t.sblk.size();
 }
 
 // pos, ent: CSR over the mesh points of their sphere points {map index, matrix}, matrix order
@@ -324,7 +365,8 @@ void build_ket(octhip_hamiltonian_s* h, const double* matrices, const std::vecto
     const int* o = h->offsets.data() + 6 * (size_t)a;
     prow0[a] = (int)t.prow.size();
     for (int j = 0; j < padded_projs(h, a); ++j)
-      t.prow.push_back(make_int4(chunk0[a], chunk0[a + 1], j, j < o[O_PROJS] ? o[O_SCAL] + j : -1));
+      t.prow.push_back(ProjRow{{make_int2(chunk0[a], chunk0[a + 1]), make_int2(0, 0)}, j,
+                               j < o[O_PROJS] ? o[O_SCAL] + j : -1});
   }
   h->nprow = (int)t.prow.size();
   // mesh points inside a sphere, by their set of matrices, mesh order within a set
@@ -340,17 +382,20 @@ void build_ket(octhip_hamiltonian_s* h, const double* matrices, const std::vecto
   std::stable_sort(pts.begin(), pts.end(), [&](int p, int q) { return cmp(p, q) < 0; });
   h->nslot = (int)pts.size();
   t.slot.assign(h->np, 0);
+  int set = 0, widest = 0;  // most slots of a set
   for (size_t i = 0, e; i < pts.size(); i = e) {
     for (e = i + 1; e < pts.size() && e < i + 16 && cmp(pts[i], pts[e]) == 0;) ++e;
     const int p0 = pos[pts[i]], ne = pos[pts[i] + 1] - p0, n = (int)(e - i);
     const int step0 = (int)t.step.size(), line0 = (int)(t.pt.size() / 4);
+    if (i > 0 && cmp(pts[i - 1], pts[i]) != 0) ++set;
+    widest = std::max(widest, ne);
     for (int k = 0; k < ne; ++k) {
       const int a = ent[p0 + k].y;
       const int* o = h->offsets.data() + 6 * (size_t)a;
       const int entry = (int)t.g.size();
       for (size_t r = i; r < e; ++r) t.g.push_back(ent[pos[pts[r]] + k].x);
       for (int j = 0; j < o[O_PROJS]; j += 4) {
-        t.step.push_back(make_int4(0, prow0[a] + j, j == 0 ? entry : -1, 0));
+        t.step.push_back(make_int4(prow0[a] + j, 0, entry, j == 0));
         t.matrix.push_back(a);
         for (int r = 0; r < n; ++r)
           for (int c = j; c < j + 4; ++c)
@@ -364,15 +409,29 @@ void build_ket(octhip_hamiltonian_s* h, const double* matrices, const std::vecto
     g.steps = (int)t.step.size() - step0;
     g.step = step0;
     g.line = line0;
+    g.set = set;
     t.grp.push_back(g);
     for (size_t r = i; r < e; ++r) t.slot[pts[r]] = (int)r + 1;
   }
   h->nkgrp = (int)t.grp.size();
-  h->ket_sums = ket_sums(h, prow0, t);
+  t.point = pts;
+  // Bra by sets where a set's sums fit a block, unless the rows it reads (groups padded to 16
+  // points) with its parts written and read clearly exceed those of the bra by spheres (sets
+  // of a few points each).  Without any overlap it reads a tenth more and is still faster
+  // (R = 12 sphere x 64 lanes, 16 spheres of radius 1.5 / 4 of them: 14.5 / 13.5 us against
+  // 18.0 / 16.1; R = 8 x 16 lanes, 6 spheres: 6.9 against 9.6): more, smaller waves.
+  const int pj = (h->max_nprojs + 3) / 4 * 4;
+  if (widest * pj <= BRA_SET_ROWS) {
+    set_blocks(h, widest * pj <= BRA_SET_ROWS / 2 ? BRA_SET_ROWS / 2 : BRA_SET_ROWS, t);
+    const size_t by_sets = 16 * (size_t)h->nkgrp + 2 * (size_t)h->set_parts * pj;
+    const size_t by_spheres = ent.size() + 2 * (size_t)h->nchunk * h->max_nprojs;
+    if (4 * by_sets >= 5 * by_spheres) h->nsblk = h->set_parts = h->set_sums = 0;
+  }
   for (KetGroup& g : t.grp)
     for (int u = 0; u < KET_AHEAD; ++u) {
       const int4 q = t.step[g.step + std::min(u, g.steps - 1)];
-      g.ahead[u] = make_int2(q.x, q.y);
+      g.proj[u] = q.x;
+      g.sum[u] = q.y;
     }
 }
 
@@ -454,9 +513,12 @@ extern "C" int octhip_hamiltonian_create(octhip_nl_operator_t kinetic, double ma
       rc = upload(&h->d_kgrp, kt.grp.data(), kt.grp.size(), s);
       if (!rc) rc = upload(&h->d_kstep, kt.step.data(), kt.step.size(), s);
       if (!rc) rc = upload(&h->d_kpt, kt.pt.data(), kt.pt.size(), s);
-      if (!rc) rc = upload(&h->d_kg, kt.g.data(), kt.g.size(), s);
-      if (!rc) rc = upload(&h->d_kblk, kt.blk.data(), kt.blk.size(), s);
-      if (!rc) rc = upload(&h->d_ksumrow, kt.sum.data(), kt.sum.size(), s);
+      h->kg = std::move(kt.g);
+      if (!rc && h->nsblk > 0) {
+        rc = upload(&h->d_sblk, kt.sblk.data(), kt.sblk.size(), s);
+        if (!rc) rc = upload(&h->d_spart, kt.spart.data(), kt.spart.size(), s);
+        if (!rc) rc = upload(&h->d_kpoint, kt.point.data(), kt.point.size(), s);
+      }
     }
     if (!rc) rc = upload(&h->d_matrices, matrices, matrix_size, s);
     if (!rc) rc = upload(&h->d_maps, maps, total_points, s);
@@ -482,10 +544,11 @@ extern "C" int octhip_hamiltonian_destroy(octhip_hamiltonian_t h) {
   dfree(h->d_kgrp);
   dfree(h->d_kstep);
   dfree(h->d_prow);
-  dfree(h->d_kblk);
-  dfree(h->d_ksumrow);
+  dfree(h->d_kphase);
+  dfree(h->d_sblk);
+  dfree(h->d_spart);
+  dfree(h->d_kpoint);
   dfree(h->d_kpt);
-  dfree(h->d_kg);
   dfree(h->d_v);
   dfree(h->d_xyz);
   dfree(h->d_veff);
@@ -581,8 +644,8 @@ extern "C" int octhip_hamiltonian_memory(octhip_hamiltonian_t h, size_t* bytes) 
                         (const void*)h->d_pt,
                         (const void*)h->d_chunks, (const void*)h->d_mat_info, (const void*)h->d_prow,
                         (const void*)h->d_kslot, (const void*)h->d_kgrp, (const void*)h->d_kstep,
-                        (const void*)h->d_kblk, (const void*)h->d_ksumrow, (const void*)h->d_kpt,
-                        (const void*)h->d_kg,
+                        (const void*)h->d_kpt, (const void*)h->d_kphase,
+                        (const void*)h->d_sblk, (const void*)h->d_spart, (const void*)h->d_kpoint,
                         (const void*)h->d_bnd_src, (const void*)h->d_phase, (const void*)h->d_phase_corr,
                         (const void*)h->d_pphase})
     data += dev_bytes(p);
@@ -1370,7 +1433,7 @@ extern "C" int octhip_hamiltonian_set_phases(octhip_hamiltonian_t h, const doubl
   OCTHIP_REQUIRE(h->graphs.empty(), "destroy the Taylor graphs of this Hamiltonian before setting Bloch phases");
   const int np_part = h->kin->np_part, nb = np_part - h->np;
   (void)hipDeviceSynchronize();
-  for (double** p : {&h->d_phase, &h->d_phase_corr, &h->d_pphase}) {
+  for (double** p : {&h->d_phase, &h->d_phase_corr, &h->d_pphase, &h->d_kphase}) {
     dfree(*p);
     *p = nullptr;
   }
@@ -1381,6 +1444,10 @@ extern "C" int octhip_hamiltonian_set_phases(octhip_hamiltonian_t h, const doubl
   int rc = upload(&h->d_phase, phase, 2 * (size_t)np_part, nullptr);
   if (!rc && nb > 0) rc = upload(&h->d_phase_corr, phase_corr, 2 * (size_t)nb, nullptr);
   if (!rc && h->nmat > 0) rc = upload(&h->d_pphase, projector_phases, 2 * (size_t)h->total_points, nullptr);
+  std::vector<double> by_entry(2 * h->kg.size());
+  for (size_t e = 0; e < h->kg.size(); ++e)
+    for (int c = 0; c < 2; ++c) by_entry[2 * e + c] = projector_phases[2 * (size_t)h->kg[e] + c];
+  if (!rc) rc = upload(&h->d_kphase, by_entry.data(), by_entry.size(), nullptr);
   if (rc) return rc;
   h->has_kpoint = true;
   return OCTHIP_SUCCESS;

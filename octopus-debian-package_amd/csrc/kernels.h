@@ -7,6 +7,8 @@
 // covers 64 consecutive doubles of one or more rows (512 B when L >= 64).
 #pragma once
 
+#include <algorithm>
+
 #include "octhip_internal.h"
 
 namespace octhip {
@@ -322,7 +324,7 @@ struct BraArgs {
   const int4* __restrict__ mat_info;  // {npoints, nprojs, matrix offset, map offset}
   const double* __restrict__ mats;    // column-major blocks
   const int* __restrict__ maps;       // 1-based
-  double* __restrict__ partial;       // (chunk, pjmax, L)
+  double* __restrict__ partial;       // (part, pjmax, L): a part is a chunk or a block's matrix
   int pjmax;
   // Bloch phases of the sphere points (complex pairs, indexed like the maps; complex rows
   // only): the gathered values are multiplied by them (hamiltonian_elec_base_inc.F90:
@@ -330,71 +332,83 @@ struct BraArgs {
   const double* __restrict__ pphase = nullptr;
 };
 
-// Projections of a matrix occupy 4 ceil(nprojs / 4) rows, the last ones zero, so that the
-// ket's steps of 4 projectors need no masks.
+// Row of the projections: a matrix has 4 ceil(nprojs / 4) rows, the last ones zero, so that
+// the ket's steps of 4 projectors need no masks.  It is the scaled sum of its matrix's parts,
+// parts [part[m].x, part[m].y) with m = 0 for the bra by spheres, 1 for the bra by sets.
+struct ProjRow {
+  int2 part[2];
+  int j, scal;                        // projector of the matrix, its scal or -1: a zero row
+};
+
 struct BraReduceArgs {
   const double* __restrict__ partial;
-  const int4* __restrict__ row;       // nrow: {first chunk, last chunk + 1, projector, scal or -1: a zero row}
+  const ProjRow* __restrict__ row;    // nrow
   const double* __restrict__ scals;
   double* __restrict__ proj;          // (nrow, L)
-  int L, pjmax, nrow;
+  int L, pjmax, nrow, sets;           // sets: the parts to sum
 };
 
 // groups of <= 16 rows per ket workgroup (one a wave), steps of a group loaded with it
 constexpr int KET_GROUPS = 4;
 constexpr int KET_AHEAD = 4;
-// Where the ket is a few hundred workgroups with few projections each, they sum the bra's
-// partials themselves (LDS of KET_SUMS doubles) and save a launch: radius-3 spheres at h =
-// 0.45 x 16 lanes, 69 workgroups of <= 8 projection rows, 5.1 us instead of 4.0 + 3.9 (bra
-// reduce).  Every workgroup waits for its sums, though: 566 workgroups of up to 64 rows take
-// 10.9 instead of 5.5 + 4.1, and 2480 of about 6 rows (R = 12 sphere x 64 lanes) 28.3
-// instead of 14.0 + 5.0.
-constexpr int KET_SUMS = 512;
-constexpr int KET_SUM_BLOCKS = 512;
-
 // Ket of X(hamiltonian_elec_base_nlocal_finish) (src/hamiltonian/hamiltonian_elec_base_inc.F90:
 // 914-943) in one pass over the mesh points that lie in at least one sphere:
 //   kbuf[r, l] = sum_a sum_j P_a[r, j] proj[a, j, l],  a in matrix order.
 // The ket rows are sorted by the set of matrices of their point and cut into groups of <= 16
 // rows with one set, so a group is one FP64 MFMA product over steps of 4 projectors and no
 // row takes part in a matrix it does not belong to (an infinity in one projection stays in
-// its own sphere).  Mesh point p then adds row kslot[p] - 1 of kbuf, or nothing.
+// its own sphere).  Mesh point p then adds row kslot[p] - 1 of kbuf, or nothing.  R = 12
+// sphere x 64 lanes: 10.7 us, 40 MB written (one row per sphere point and a pass that summed
+// those of shared mesh points: 15 + 8 us); R = 10 x 128 lanes 6.5 (10.5 + 6.4).
 struct KetGroup {
   int row, rows, steps, step;         // first ket row, rows, steps, first step
-  int line, pad[3];                   // first line of pt
-  int2 ahead[KET_AHEAD];              // the first steps' (sum, proj) again: one load fetches a group
+  int line, set, pad[2];              // first line of pt, number of the group's set
+  int proj[KET_AHEAD];                // the first steps again: one load fetches a group
+  int sum[KET_AHEAD];
 };
 struct KetArgs {
   const KetGroup* __restrict__ grp;
   int ngrp;                           // workgroup b owns groups KET_GROUPS b ..
-  const int4* __restrict__ step;      // {row of the block's sums, row of proj, first kg entry or -1: same matrix, -}
-  const int2* __restrict__ blk;       // {first sum, sums} of a workgroup
+  const int4* __restrict__ step;      // {row of proj, row of the bra block's sums, first entry, 1: new matrix}
   const double* __restrict__ pt;      // lines of 4 projector values: line + step * rows + row
   const double* __restrict__ proj;
   double* __restrict__ kbuf;
   int L;
-  // optional (MFMA form only): the bra's chunk partials instead of proj; each workgroup
-  // then forms the projections of its groups and lane tile itself, summed and scaled as
-  // k_bra_reduce does (so bit-identical), and k_bra_reduce is not launched
-  const double* __restrict__ partial = nullptr;
-  const int4* __restrict__ sum = nullptr;  // as BraReduceArgs::row
-  const double* __restrict__ scals = nullptr;
-  int pjmax = 0;
-  // Bloch phases: the term of a matrix is multiplied by conj(pphase[kg[entry + row]])
-  // (hamiltonian_elec_base_inc.F90:955-966); null: none
-  const double* __restrict__ pphase = nullptr;
-  const int* __restrict__ kg = nullptr;
+  // Bloch phases by entry (conjugated and multiplied onto the terms of a matrix, entry + row;
+  // hamiltonian_elec_base_inc.F90:955-966); null: none
+  const double* __restrict__ phase = nullptr;
 };
 
 
+// Bra by sets: the same groups as the ket's, so the row of a mesh point inside several
+// spheres is read once and feeds the projectors of all of them, 16 projector rows at a time
+// (16 overlapping radius-3 spheres, R = 12 x 64 lanes: 78636 rows instead of 115833, 30 ->
+// 22.5 us with the boundary rows cleared alongside; R = 10 x 128 lanes 13.5 -> 8.2; R = 6 x
+// 16 lanes 9.4 -> 6.6).
+// Block b owns <= BRA_SET_GROUPS groups, one a wave; its sums (slots x pjmax projector rows x lanes, for each wave)
+// are in LDS and leave as one part per matrix (slot).
+struct BraSetArgs {
+  const KetGroup* __restrict__ grp;
+  const int4* __restrict__ step;
+  const double* __restrict__ pt;
+  const int* __restrict__ point;      // mesh row of each ket row
+  const int4* __restrict__ blk;       // {first group, groups, first slot, slots}
+  const int* __restrict__ part;       // part of each slot
+  const double* __restrict__ phase;   // Bloch phases by entry; null: none
+};
+constexpr int BRA_SET_GROUPS = 4;
+constexpr int BRA_SET_ROWS = 64;      // sums of a block: 4 waves x 64 rows x 32 lanes, 64 KB LDS
+
 struct BraMfmaArgs {
   BraArgs b;
+  BraSetArgs set;
+  int sets;                       // the bra by sets (else by spheres)
   const double* __restrict__ pt;  // total_points x pjs
   int pjs;
   // optional: rows [zfirst, zfirst + zcount) of zf cleared by blocks nbra.. of the launch
   double* zf;
   size_t zfirst, zcount;
-  int nbra;                       // blocks doing the bra: chunks x 16-lane tiles
+  int nbra;                       // blocks doing the bra: chunks (blocks) x lane tiles
 };
 
 struct ZeroArgs {
@@ -403,22 +417,31 @@ struct ZeroArgs {
 };
 
 // kernels of a multi-segment launch (several systems/batches in one grid)
-enum { MULTI_BRA_MFMA = 1, MULTI_BRA_PLAIN, MULTI_BRA_REDUCE, MULTI_KET_MFMA, MULTI_KET_PLAIN,
+enum { MULTI_BRA_MFMA = 1, MULTI_BRA_SETS, MULTI_BRA_PLAIN, MULTI_BRA_REDUCE, MULTI_KET_MFMA, MULTI_KET_PLAIN,
        MULTI_ZERO };
 // args: device array of nseg argument blocks; off: device array of nseg+1 block offsets
-int launch_multi(int kind, const void* args, const int* off, int nseg, int nblocks, hipStream_t s);
+int launch_multi(int kind, const void* args, const int* off, int nseg, int nblocks, hipStream_t s, size_t lds = 0);
 
 int launch_bra(const BraArgs& b, int nchunk, bool mfma, hipStream_t s);
-// whether the ket of h sums the partials itself at this row length, and its arguments then
-// (sums) or from proj
-bool ket_sums_partials(const octhip_hamiltonian_s* h, int L);
-void ket_args(const octhip_hamiltonian_s* h, int L, const double* partial, const double* proj, double* kbuf,
-              bool sums, KetArgs& k);
+// whether the MFMA bra of h goes by sets
+bool bra_by_sets(const octhip_hamiltonian_s* h);
+// MFMA bra arguments (psi and the cleared rows are left to the caller), its blocks and its
+// dynamic LDS at rows of L lanes
+void bra_mfma_args(const octhip_hamiltonian_s* h, int L, double* partial, BraMfmaArgs& m);
+int bra_mfma_blocks(const octhip_hamiltonian_s* h, int L);
+size_t bra_mfma_lds(const octhip_hamiltonian_s* h, int L);
+// doubles of a partial buffer for rows of L lanes
+size_t partial_doubles(const octhip_hamiltonian_s* h, size_t L);
+// ket arguments of h for rows of L lanes
+void ket_args(const octhip_hamiltonian_s* h, int L, const double* proj, double* kbuf, KetArgs& k);
 inline int ket_blocks(int ngrp) { return (ngrp + KET_GROUPS - 1) / KET_GROUPS; }
 int launch_ket(const KetArgs& k, bool mfma, hipStream_t s);
 // lane tiles of the MFMA bra and ket over rows of L lanes (L >= 16): 32-lane tiles (two
 // columns per lane) when 32 divides L, else 16-lane tiles
 __host__ __device__ inline int mfma_lane_tiles(int L) { return (L & 31) == 0 ? L >> 5 : L >> 4; }
+inline int bra_reduce_blocks(const BraReduceArgs& r) {
+  return std::min((r.nrow * ((r.L + 15) / 16) + BLOCK / 64 - 1) / (BLOCK / 64), 4096);
+}
 int launch_bra_reduce(const BraReduceArgs& r, hipStream_t s);
 
 // sphere points per bra chunk

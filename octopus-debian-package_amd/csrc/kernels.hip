@@ -129,7 +129,7 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 // each column's sum is the TW = 1 sum, in the same order.
 constexpr int BRA_RED = 4 * 16 * 16;  // LDS doubles per accumulator of the wave reduction
 template <int TW>
-__device__ __forceinline__ void bra_mfma_body(const BraMfmaArgs& m, int c, int lt, double (*red)[BRA_RED]) {
+__device__ __forceinline__ void bra_mfma_body(const BraMfmaArgs& m, int c, int lt, double* red) {
   constexpr int KB = 16;                    // MFMA steps (4 sphere points each) per load block
   const BraArgs& b = m.b;
   const int4 ch = b.chunks[c];
@@ -190,7 +190,7 @@ __device__ __forceinline__ void bra_mfma_body(const BraMfmaArgs& m, int c, int l
 #pragma unroll
     for (int w = 0; w < TW; ++w)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[w][(wave * 16 + 4 * r + kk) * 16 + ii] = acc[w][r];
+      for (int r = 0; r < 4; ++r) red[w * BRA_RED + (wave * 16 + 4 * r + kk) * 16 + ii] = acc[w][r];
     __syncthreads();
     if (wave == 0) {
 #pragma unroll
@@ -198,8 +198,8 @@ __device__ __forceinline__ void bra_mfma_body(const BraMfmaArgs& m, int c, int l
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int jl = 4 * r + kk;
-          const double t = (red[w][(0 * 16 + jl) * 16 + ii] + red[w][(1 * 16 + jl) * 16 + ii]) +
-                           (red[w][(2 * 16 + jl) * 16 + ii] + red[w][(3 * 16 + jl) * 16 + ii]);
+          const double t = (red[w * BRA_RED + (0 * 16 + jl) * 16 + ii] + red[w * BRA_RED + (1 * 16 + jl) * 16 + ii]) +
+                           (red[w * BRA_RED + (2 * 16 + jl) * 16 + ii] + red[w * BRA_RED + (3 * 16 + jl) * 16 + ii]);
           const int j = jb + jl;
           if (j < npj) b.partial[((size_t)c * b.pjmax + j) * b.L + col + w] = t;
         }
@@ -207,6 +207,120 @@ __device__ __forceinline__ void bra_mfma_body(const BraMfmaArgs& m, int c, int l
   }
 }
 
+// Bra by sets.  A wave takes one group of <= 16 mesh points: its 4 state loads and the
+// projector loads of its first 32 projector rows are in flight together, and a product
+// A(16 projector rows x 4 points) B(4 points x 16 lanes) serves up to 4 matrices of 4
+// projectors.  Lane (kk, ii) supplies A[ii][kk] = P[row ii, point kk] from line step(ii/4) of
+// the group (32-byte runs) and gets D[4r+kk][ii]: rows 4r .. 4r+3 are those of step r.  The
+// sums go to the wave's part of LDS and the 4 waves are added in a fixed order.  No row of a
+// group takes part in a matrix it does not belong to, and operands past its points are zero.
+// PHASE: the states times the Bloch phases of (point, matrix), which differ by matrix: a
+// product per step, of which D rows 4r .. 4r+3 are kept.
+template <int TW, bool PHASE>
+__device__ __forceinline__ void bra_set_body(const BraMfmaArgs& m, int bl, int lt, double* red) {
+  constexpr int TL = 16 * TW;
+  static_assert(BRA_SET_GROUPS == BLOCK / 64, "a group per wave");
+  const BraArgs& b = m.b;
+  const BraSetArgs& a = m.set;
+  const int4 blk = a.blk[bl];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+  const int kk = ln >> 4, ii = ln & 15;
+  const int col = lt * TL + ii * TW;
+  const int sums = blk.w * b.pjmax * TL;      // LDS doubles of a wave
+  double* const mine = red + (size_t)wave * sums;
+  const KetGroup gr = a.grp[blk.x + min(wave, blk.y - 1)];
+  const int n = gr.rows, ns = gr.steps;
+  int p[4], row[4];
+  double av[2][4];                            // projector rows 0 .. 15 and 16 .. 31
+  Vec<TW> bv[4];
+  const double* const pt = a.pt + 4 * (size_t)gr.line + (ii & 3);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    p[k] = min(4 * k + kk, n - 1);
+    row[k] = a.point[gr.row + p[k]];
+    av[0][k] = pt[4 * (size_t)(min(ii >> 2, ns - 1) * n + p[k])];
+  }
+  if (ns > 4)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) av[1][k] = pt[4 * (size_t)(min(4 + (ii >> 2), ns - 1) * n + p[k])];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) bv[k] = ldv<TW>(b.psi + (size_t)row[k] * b.L + col);
+  for (int t = ln; t < sums; t += 64) mine[t] = 0.0;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (wave < blk.y) {
+    for (int t0 = 0; t0 < ns; t0 += 4) {      // 16 projector rows at a time
+      double x[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        x[k] = t0 == 0   ? av[0][k]
+               : t0 == 4 ? av[1][k]
+                         : pt[4 * (size_t)(min(t0 + (ii >> 2), ns - 1) * n + p[k])];
+        x[k] = 4 * k + kk < n ? x[k] : 0.0;
+      }
+      d4 acc[TW];
+      const auto product = [&](const Vec<TW>* v) {
+#pragma unroll
+        for (int w = 0; w < TW; ++w) acc[w] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int w = 0; w < TW; ++w)
+            acc[w] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[k], 4 * k + kk < n ? v[k].v[w] : 0.0, acc[w], 0, 0, 0);
+      };
+      if constexpr (!PHASE) product(bv);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (t0 + r >= ns) break;
+        if constexpr (PHASE) {
+          const size_t ent = a.step[gr.step + t0 + r].z;
+          Vec<TW> ph[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const double pr = a.phase[2 * (ent + p[k])], pi = a.phase[2 * (ent + p[k]) + 1];
+            if constexpr (TW == 2) {
+              ph[k].v[0] = zmul_lane(pr, pi, bv[k].v[0], bv[k].v[1], false);
+              ph[k].v[1] = zmul_lane(pr, pi, bv[k].v[1], bv[k].v[0], true);
+            } else {
+              ph[k].v[0] = zmul_lane(pr, pi, bv[k].v[0], __shfl_xor(bv[k].v[0], 1), (col & 1) != 0);
+            }
+          }
+          product(ph);
+        }
+        // a matrix that holds the point twice adds to its rows twice
+        const int sum = t0 == 0 ? gr.sum[r] : a.step[gr.step + t0 + r].y;
+        double* const d = mine + (sum + kk) * TL + ii * TW;
+        Vec<TW> v = ldv<TW>(d);
+#pragma unroll
+        for (int w = 0; w < TW; ++w) v.v[w] += acc[w][r];
+        stv<TW>(d, v);
+      }
+    }
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < sums; t += BLOCK) {
+    const int q = t / TL, slot = q / b.pjmax;
+    const double v = (red[t] + red[t + sums]) + (red[t + 2 * (size_t)sums] + red[t + 3 * (size_t)sums]);
+    b.partial[((size_t)a.part[blk.z + slot] * b.pjmax + (q - slot * b.pjmax)) * b.L + lt * TL + (t - q * TL)] = v;
+  }
+}
+
+extern __shared__ double2 bra_lds[];
+template <bool SETS, bool PHASE>
+__device__ __forceinline__ void bra_mfma(const BraMfmaArgs& m, int b) {
+  double* const red = reinterpret_cast<double*>(bra_lds);
+  const int nlt = mfma_lane_tiles(m.b.L);
+  const bool wide = (m.b.L & 31) == 0;
+  if constexpr (SETS) {
+    if (wide) bra_set_body<2, PHASE>(m, b / nlt, b % nlt, red);
+    else bra_set_body<1, PHASE>(m, b / nlt, b % nlt, red);
+  } else {
+    if (wide) bra_mfma_body<2>(m, b / nlt, b % nlt, red);
+    else bra_mfma_body<1>(m, b / nlt, b % nlt, red);
+  }
+}
+
+template <bool SETS, bool PHASE>
 __global__ __launch_bounds__(BLOCK) void k_bra_mfma(const BraMfmaArgs m) {
   const int nz = (int)gridDim.x - m.nbra;
   if ((int)blockIdx.x < nz) {
@@ -217,40 +331,34 @@ __global__ __launch_bounds__(BLOCK) void k_bra_mfma(const BraMfmaArgs m) {
       m.zf[m.zfirst + t] = 0.0;
     return;
   }
-  __shared__ double red[2][BRA_RED];
-  const int b = (int)blockIdx.x - nz;
-  if ((m.b.L & 31) == 0) {
-    const int nlt = m.b.L >> 5;
-    bra_mfma_body<2>(m, b / nlt, b % nlt, red);
-  } else {
-    const int nlt = m.b.L >> 4;
-    bra_mfma_body<1>(m, b / nlt, b % nlt, red);
-  }
+  bra_mfma<SETS, PHASE>(m, (int)blockIdx.x - nz);
 }
 
-// one projection: scal * sum of its matrix's partials (one per chunk of <= 256 sphere
-// points: 29 for a radius-3 sphere at h = 0.25), loaded together with clamped indices, then
-// added in chunk order
-__device__ __forceinline__ double proj_sum(const double* __restrict__ partial, const double* __restrict__ scals,
-                                           int4 w, int pjmax, int L, int l) {
-  if (w.w < 0) return 0.0;
-  double s = 0.0;
-  for (int c = w.x; c < w.y; c += 32) {
-    double v[32];
-#pragma unroll
-    for (int u = 0; u < 32; ++u) v[u] = partial[((size_t)min(c + u, w.y - 1) * pjmax + w.z) * L + l];
-#pragma unroll
-    for (int u = 0; u < 32; ++u)
-      if (c + u < w.y) s += v[u];
-  }
-  return s * scals[w.w];
-}
-
+// Projection row i at 16 lanes, by one wave: scal * the sum of its matrix's parts as four
+// interleaved sums, (s0 + s1) + (s2 + s3): lanes 16 q .. 16 q + 15 add parts first + q,
+// first + q + 4, ..., loaded together with clamped indices.  (A radius-3 sphere at h = 0.25
+// has 29 parts by spheres and about 120 by sets; four sums keep either at one or two round
+// trips, so the launch is 4 to 5 us at all sizes.)
 __device__ __forceinline__ void bra_reduce_body(const BraReduceArgs& r, int bid, int nblk) {
-  const size_t total = (size_t)r.nrow * r.L;
-  for (size_t t = bid * (size_t)BLOCK + threadIdx.x; t < total; t += (size_t)nblk * BLOCK) {
-    const int i = (int)(t / r.L);
-    r.proj[t] = proj_sum(r.partial, r.scals, r.row[i], r.pjmax, r.L, (int)(t - (size_t)i * r.L));
+  constexpr int N = 16;
+  const int ln = threadIdx.x & 63, tiles = (r.L + 15) / 16;
+  for (int t = bid * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t < r.nrow * tiles;
+       t += nblk * (BLOCK / 64)) {
+    const int i = t / tiles, l0 = (t - i * tiles) * 16, l = min(l0 + (ln & 15), r.L - 1);
+    const ProjRow w = r.row[i];
+    const int2 p = r.sets ? w.part[1] : w.part[0];
+    double s = 0.0;
+    for (int c = p.x + (ln >> 4); c < p.y && w.scal >= 0; c += 4 * N) {
+      double v[N];
+#pragma unroll
+      for (int u = 0; u < N; ++u) v[u] = r.partial[((size_t)min(c + 4 * u, p.y - 1) * r.pjmax + w.j) * r.L + l];
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+        if (c + 4 * u < p.y) s += v[u];
+    }
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    if (ln < 16 && l0 + ln < r.L) r.proj[(size_t)i * r.L + l] = w.scal < 0 ? 0.0 : s * r.scals[w.scal];
   }
 }
 
@@ -272,14 +380,16 @@ int launch_bra(const BraArgs& b, int nchunk, bool mfma, hipStream_t s) {
   return OCTHIP_SUCCESS;
 }
 
-int launch_bra_mfma(const BraArgs& b, const double* pt, int pjs, int nchunk, hipStream_t s, double* zf,
-                    size_t zfirst, size_t zcount) {
-  if (nchunk <= 0) return OCTHIP_SUCCESS;
-  // 32-lane tiles (two columns per lane) when the row length allows, else 16-lane tiles
-  BraMfmaArgs m{b, pt, pjs, zf, zfirst, zf ? zcount : 0, nchunk * mfma_lane_tiles(b.L)};
-  const int zblocks = zf ? (int)std::min<size_t>((zcount + BLOCK - 1) / BLOCK, 2048) : 0;
+int launch_bra_mfma(BraMfmaArgs& m, size_t lds, hipStream_t s) {
+  if (m.nbra <= 0) return OCTHIP_SUCCESS;
+  const int zblocks = m.zf ? (int)std::min<size_t>((m.zcount + BLOCK - 1) / BLOCK, 2048) : 0;
   ProfScope prof("k_bra", s);
-  hipLaunchKernelGGL(k_bra_mfma, dim3(m.nbra + zblocks), dim3(BLOCK), 0, s, m);
+  if (m.sets && m.set.phase)
+    hipLaunchKernelGGL((k_bra_mfma<true, true>), dim3(m.nbra + zblocks), dim3(BLOCK), lds, s, m);
+  else if (m.sets)
+    hipLaunchKernelGGL((k_bra_mfma<true, false>), dim3(m.nbra + zblocks), dim3(BLOCK), lds, s, m);
+  else
+    hipLaunchKernelGGL((k_bra_mfma<false, false>), dim3(m.nbra + zblocks), dim3(BLOCK), lds, s, m);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(OCTHIP_ERR_HIP, "k_bra_mfma launch: %s", hipGetErrorString(e));
   return OCTHIP_SUCCESS;
@@ -295,29 +405,18 @@ int launch_bra_mfma(const BraArgs& b, const double* pt, int pjs, int nchunk, hip
 // A wave's loads are a chain of round trips (group, then its operands), which is what
 // bounds this kernel: a group's record holds its first KET_AHEAD steps, whose operands are
 // loaded together, and a wave has one group.
-template <int TW, bool PHASE, bool SUMS>
-__device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt, double* sproj) {
+template <int TW, bool PHASE>
+__device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
   constexpr int TL = 16 * TW;                 // lanes of the tile
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
   const int g = b * KET_GROUPS + wave;
   const int kk = ln >> 4, ii = ln & 15;
   const int col = lt * TL + ii * TW;          // first column of this lane
-  const KetGroup gr = k.grp[min(g, k.ngrp - 1)];
+  if (g >= k.ngrp) return;
+  const KetGroup gr = k.grp[g];
   const int n = gr.rows, ns = gr.steps;
   const double* const pt = k.pt + 4 * ((size_t)gr.line + min(ii, n - 1)) + kk;
-  const double* const pj = SUMS ? sproj + kk * TL + ii * TW : k.proj + (size_t)kk * k.L + col;
-  const size_t ldp = SUMS ? TL : k.L;
-  double av[KET_AHEAD];
-  Vec<TW> bv[KET_AHEAD];
-#pragma unroll
-  for (int u = 0; u < KET_AHEAD; ++u) av[u] = pt[4 * (size_t)(min(u, ns - 1) * n)];
-  if constexpr (SUMS) {
-    const int2 bl = k.blk[b];
-    for (int t = threadIdx.x; t < bl.y * TL; t += BLOCK)
-      sproj[t] = proj_sum(k.partial, k.scals, k.sum[bl.x + t / TL], k.pjmax, k.L, lt * TL + (t % TL));
-    __syncthreads();
-  }
-  if (g >= k.ngrp) return;
+  const double* const pj = k.proj + (size_t)kk * k.L + col;
   d4 acc[TW], tot[TW];
 #pragma unroll
   for (int w = 0; w < TW; ++w) acc[w] = tot[w] = d4{0.0, 0.0, 0.0, 0.0};
@@ -327,8 +426,8 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt, d
     // lane holds the (re, im) pair, otherwise lanes ii ^ 1 hold the pair
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const size_t pi2 = 2 * (size_t)k.kg[ent + min(4 * r + kk, n - 1)];
-      const double pr = k.pphase[pi2], pi = -k.pphase[pi2 + 1];
+      const size_t pi2 = 2 * (size_t)(ent + min(4 * r + kk, n - 1));
+      const double pr = k.phase[pi2], pi = -k.phase[pi2 + 1];
       if constexpr (TW == 2) {
         tot[0][r] += zmul_lane(pr, pi, acc[0][r], acc[1][r], false);
         tot[1][r] += zmul_lane(pr, pi, acc[1][r], acc[0][r], true);
@@ -338,23 +437,22 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt, d
     }
   };
   for (int q0 = 0; q0 < ns; q0 += KET_AHEAD) {
-    if (q0 > 0) {
-#pragma unroll
-      for (int u = 0; u < KET_AHEAD; ++u) av[u] = pt[4 * (size_t)(min(q0 + u, ns - 1) * n)];
-    }
+    double av[KET_AHEAD];
+    Vec<TW> bv[KET_AHEAD];
 #pragma unroll
     for (int u = 0; u < KET_AHEAD; ++u) {
-      const int2 q = q0 == 0 ? gr.ahead[u] : *reinterpret_cast<const int2*>(k.step + gr.step + min(q0 + u, ns - 1));
-      bv[u] = ldv<TW>(pj + (SUMS ? q.x : q.y) * ldp);
+      const int q = min(q0 + u, ns - 1);
+      av[u] = pt[4 * (size_t)(q * n)];
+      bv[u] = ldv<TW>(pj + (size_t)(q0 == 0 ? gr.proj[u] : k.step[gr.step + q].x) * k.L);
     }
 #pragma unroll
     for (int u = 0; u < KET_AHEAD; ++u) {
       if (q0 + u >= ns) break;
       if constexpr (PHASE) {
-        const int z = k.step[gr.step + q0 + u].z;
-        if (z >= 0) {
+        const int4 st = k.step[gr.step + q0 + u];
+        if (st.w) {
           if (q0 + u > 0) flush();
-          ent = z;
+          ent = st.z;
 #pragma unroll
           for (int w = 0; w < TW; ++w) acc[w] = d4{0.0, 0.0, 0.0, 0.0};
         }
@@ -379,13 +477,11 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt, d
   }
 }
 
-template <bool PHASE, bool SUMS>
+template <bool PHASE>
 __device__ __forceinline__ void ket_mfma(const KetArgs& k, int b) {
-  __shared__ double2 sproj2[SUMS ? KET_SUMS / 2 : 1];  // 16-byte aligned: read as lane pairs
-  double* const sproj = reinterpret_cast<double*>(sproj2);
   const int nlt = mfma_lane_tiles(k.L);
-  if ((k.L & 31) == 0) ket_mfma_body<2, PHASE, SUMS>(k, b / nlt, b % nlt, sproj);
-  else ket_mfma_body<1, PHASE, SUMS>(k, b / nlt, b % nlt, sproj);
+  if ((k.L & 31) == 0) ket_mfma_body<2, PHASE>(k, b / nlt, b % nlt);
+  else ket_mfma_body<1, PHASE>(k, b / nlt, b % nlt);
 }
 
 // plain form, any row length: a wave per group, one thread per (row, lane)
@@ -400,47 +496,42 @@ __device__ __forceinline__ void ket_plain_body(const KetArgs& k, int b) {
       double tot = 0.0, acc = 0.0, accq = 0.0;  // accq: the other lane of the (re, im) pair
       int ent = 0;
       for (int q = 0; q <= ns; ++q) {
-        const int4 s = q < ns ? k.step[gr.step + q] : make_int4(0, 0, 0, 0);
-        if (k.pphase && q > 0 && s.z >= 0) {
-          const size_t pi2 = 2 * (size_t)k.kg[ent + r];
-          tot += zmul_lane(k.pphase[pi2], -k.pphase[pi2 + 1], acc, accq, (l & 1) != 0);
+        const int4 s = q < ns ? k.step[gr.step + q] : make_int4(0, 0, 0, 1);
+        if (k.phase && q > 0 && s.w) {
+          const size_t pi2 = 2 * (size_t)(ent + r);
+          tot += zmul_lane(k.phase[pi2], -k.phase[pi2 + 1], acc, accq, (l & 1) != 0);
           acc = accq = 0.0;
         }
         if (q == ns) break;
-        if (s.z >= 0) ent = s.z;
+        ent = s.z;
         const double* a = k.pt + 4 * (size_t)(gr.line + q * n + r);
-        const double* pj = k.proj + (size_t)s.y * k.L;
+        const double* pj = k.proj + (size_t)s.x * k.L;
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc = fma(a[j], pj[(size_t)j * k.L + l], acc);
-        if (k.pphase) {
+        if (k.phase) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) accq = fma(a[j], pj[(size_t)j * k.L + (l ^ 1)], accq);
         }
       }
-      k.kbuf[(size_t)(gr.row + r) * k.L + l] = k.pphase ? tot : acc;
+      k.kbuf[(size_t)(gr.row + r) * k.L + l] = k.phase ? tot : acc;
     }
   }
 }
 
-template <bool PHASE, bool SUMS>
-__global__ __launch_bounds__(BLOCK) void k_ket_mfma(const KetArgs k) { ket_mfma<PHASE, SUMS>(k, blockIdx.x); }
+template <bool PHASE>
+__global__ __launch_bounds__(BLOCK) void k_ket_mfma(const KetArgs k) { ket_mfma<PHASE>(k, blockIdx.x); }
 __global__ __launch_bounds__(BLOCK) void k_ket_plain(const KetArgs k) { ket_plain_body(k, blockIdx.x); }
 
 int launch_ket(const KetArgs& k, bool mfma, hipStream_t s) {
   const int nblock = ket_blocks(k.ngrp);
   if (nblock <= 0) return OCTHIP_SUCCESS;
   mfma = mfma && k.L >= 16;
-  if (k.partial && !mfma) return fail(OCTHIP_ERR_INVALID, "k_ket: projections from partials need the MFMA form");
   ProfScope prof("k_ket", s);
   const dim3 tiles(nblock * mfma_lane_tiles(k.L));  // 32-lane tiles when the row length allows, else 16
-  if (mfma && k.pphase && k.partial)
-    hipLaunchKernelGGL((k_ket_mfma<true, true>), tiles, dim3(BLOCK), 0, s, k);
-  else if (mfma && k.pphase)
-    hipLaunchKernelGGL((k_ket_mfma<true, false>), tiles, dim3(BLOCK), 0, s, k);
-  else if (mfma && k.partial)
-    hipLaunchKernelGGL((k_ket_mfma<false, true>), tiles, dim3(BLOCK), 0, s, k);
+  if (mfma && k.phase)
+    hipLaunchKernelGGL(k_ket_mfma<true>, tiles, dim3(BLOCK), 0, s, k);
   else if (mfma)
-    hipLaunchKernelGGL((k_ket_mfma<false, false>), tiles, dim3(BLOCK), 0, s, k);
+    hipLaunchKernelGGL(k_ket_mfma<false>, tiles, dim3(BLOCK), 0, s, k);
   else
     hipLaunchKernelGGL(k_ket_plain, dim3(nblock), dim3(BLOCK), 0, s, k);
   hipError_t e = hipGetLastError();
@@ -449,10 +540,8 @@ int launch_ket(const KetArgs& k, bool mfma, hipStream_t s) {
 }
 
 int launch_bra_reduce(const BraReduceArgs& r, hipStream_t s) {
-  const size_t total = (size_t)r.nrow * r.L;
-  if (total == 0) return OCTHIP_SUCCESS;
-  int grid = (int)((total + BLOCK - 1) / BLOCK);
-  if (grid > 4096) grid = 4096;
+  const int grid = bra_reduce_blocks(r);
+  if (grid == 0) return OCTHIP_SUCCESS;
   ProfScope prof("k_bra_reduce", s);
   hipLaunchKernelGGL(k_bra_reduce, dim3(grid), dim3(BLOCK), 0, s, r);
   hipError_t e = hipGetLastError();
@@ -479,13 +568,14 @@ __device__ __forceinline__ int segment_of(const int* __restrict__ off, int nseg,
   return lo;
 }
 
+// SETS: every pair's bra goes by sets (the other form takes more registers)
+template <bool SETS>
 __global__ __launch_bounds__(BLOCK) void k_bra_mfma_multi(const BraMfmaArgs* __restrict__ a,
                                                           const int* __restrict__ off, int nseg) {
   const int i = segment_of(off, nseg, blockIdx.x);
-  __shared__ double red[2][BRA_RED];
-  const int b = blockIdx.x - off[i], nlt = mfma_lane_tiles(a[i].b.L);
-  if ((a[i].b.L & 31) == 0) bra_mfma_body<2>(a[i], b / nlt, b % nlt, red);
-  else bra_mfma_body<1>(a[i], b / nlt, b % nlt, red);
+  const BraMfmaArgs m = a[i];
+  if (SETS || m.sets) bra_mfma<true, false>(m, blockIdx.x - off[i]);
+  else bra_mfma<false, false>(m, blockIdx.x - off[i]);
 }
 __global__ __launch_bounds__(BLOCK) void k_bra_plain_multi(const BraMfmaArgs* __restrict__ a,
                                                            const int* __restrict__ off, int nseg) {
@@ -501,7 +591,7 @@ __global__ __launch_bounds__(BLOCK) void k_ket_mfma_multi(const KetArgs* __restr
                                                           const int* __restrict__ off, int nseg) {
   const int i = segment_of(off, nseg, blockIdx.x);
   const KetArgs k = a[i];
-  ket_mfma<false, false>(k, blockIdx.x - off[i]);
+  ket_mfma<false>(k, blockIdx.x - off[i]);
 }
 __global__ __launch_bounds__(BLOCK) void k_ket_plain_multi(const KetArgs* __restrict__ a,
                                                            const int* __restrict__ off, int nseg) {
@@ -524,18 +614,23 @@ int check_launch(const char* what) {
 }
 }  // namespace
 
-int launch_multi(int kind, const void* args, const int* off, int nseg, int nblocks, hipStream_t s) {
+int launch_multi(int kind, const void* args, const int* off, int nseg, int nblocks, hipStream_t s, size_t lds) {
   if (nblocks <= 0) return OCTHIP_SUCCESS;
   const dim3 g(nblocks), b(BLOCK);
   switch (kind) {
     case MULTI_BRA_MFMA: {
       ProfScope prof("k_bra", s);
-      hipLaunchKernelGGL(k_bra_mfma_multi, g, dim3(BLOCK), 0, s, (const BraMfmaArgs*)args, off, nseg);
+      hipLaunchKernelGGL(k_bra_mfma_multi<false>, g, b, lds, s, (const BraMfmaArgs*)args, off, nseg);
+      return check_launch("k_bra_mfma_multi");
+    }
+    case MULTI_BRA_SETS: {
+      ProfScope prof("k_bra", s);
+      hipLaunchKernelGGL(k_bra_mfma_multi<true>, g, b, lds, s, (const BraMfmaArgs*)args, off, nseg);
       return check_launch("k_bra_mfma_multi");
     }
     case MULTI_BRA_PLAIN: {
       ProfScope prof("k_bra", s);
-      hipLaunchKernelGGL(k_bra_plain_multi, g, dim3(BLOCK), 0, s, (const BraMfmaArgs*)args, off, nseg);
+      hipLaunchKernelGGL(k_bra_plain_multi, g, b, 0, s, (const BraMfmaArgs*)args, off, nseg);
       return check_launch("k_bra_plain_multi");
     }
     case MULTI_BRA_REDUCE: {

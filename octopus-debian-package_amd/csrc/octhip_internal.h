@@ -171,6 +171,7 @@ struct octhip_nl_operator_s {
 
 namespace octhip {
 struct KetGroup;
+struct ProjRow;
 }
 struct octhip_hamiltonian_s {
   octhip_nl_operator_t kin = nullptr;
@@ -199,15 +200,18 @@ struct octhip_hamiltonian_s {
   int* d_kslot = nullptr;       // np: row of the ket buffer of each mesh point + 1, or 0
   // ket tables (KetArgs): groups of rows with one set of matrices, blocks of groups
   int nkgrp = 0;
-  int ket_sums = 0;             // most projection rows of the groups of one ket workgroup
   octhip::KetGroup* d_kgrp = nullptr;
   int4* d_kstep = nullptr;
-  int2* d_kblk = nullptr;
-  int4* d_ksumrow = nullptr;
+  // bra by sets (BraSetArgs): 0 blocks where the bra by spheres reads less
+  int nsblk = 0, set_parts = 0, set_sums = 0;  // blocks, parts, most sums (rows) of a block
+  int4* d_sblk = nullptr;
+  int* d_spart = nullptr;
+  int* d_kpoint = nullptr;
   double* d_kpt = nullptr;      // lines of 4 projector values
-  int* d_kg = nullptr;          // sphere point of each (group, matrix, row)
+  std::vector<int> kg;          // sphere point of each entry (group, matrix, row)
+  double* d_kphase = nullptr;   // Bloch phases by entry
   int nprow = 0;                // projection rows: 4 ceil(nprojs / 4) a matrix
-  int4* d_prow = nullptr;       // BraReduceArgs::row
+  octhip::ProjRow* d_prow = nullptr;
   // Work buffers, one set per stream: applies on different streams (Octopus gives every
   // batch its own stream, accel_set_stream) may run concurrently.  The set of the stream
   // of the current call is mirrored in the fields below; sets captured into a graph are

@@ -1,10 +1,10 @@
-"""Ket rows grouped by the set of projector matrices of their mesh point.
+"""Bra and ket over mesh points grouped by the set of projector matrices they belong to.
 
 Bar: max relative error <= 1e-12 per state against the oracle, as for every H-apply (the
-terms of one mesh point are short sums; the device only groups rows differently).  The
-sphere layouts take the group and block edges: one sphere, disjoint spheres, sets of two
-and three, a point set smaller than a group, and so many concentric spheres that one
-set has more projections than a ket workgroup sums itself.
+sums are the oracle's in another grouping).  The sphere layouts take the group and block
+edges: one sphere, a point set smaller than a group, disjoint spheres, sets of two and
+three, sets of more than 16 projector rows with mixed counts, and so many spheres on
+one point that its set no longer fits the sums of a bra workgroup.
 """
 import dataclasses
 
@@ -22,6 +22,8 @@ LAYOUTS = {
     "tiny": ([(0.0, 0.0, 0.0), (1.2, 0.0, 0.0)], 0.2, [3, 5]),
     "disjoint": ([(-1.5, 0.0, 0.0), (1.5, 0.0, 0.0)], 0.9, [4, 4]),
     "chain": ([(-1.4, 0.0, 0.0), (-0.5, 0.0, 0.0), (0.5, 0.1, 0.0), (1.4, 0.0, 0.2)], 1.0, [4, 1, 6, 4]),
+    "wide": ([(0.0, 0.0, 0.0), (0.4, 0.2, 0.0), (-0.3, 0.0, 0.5)], 1.3, [18, 7, 18]),
+    "stack": ([(0.06 * i, 0.0, -0.05 * i) for i in range(12)], 1.2, [4, 2, 4, 1, 4, 4, 3, 4, 4, 4, 4, 4]),
     "dense": ([(0.05 * i, 0.0, -0.04 * i) for i in range(24)], 1.2, [4] * 24),
 }
 

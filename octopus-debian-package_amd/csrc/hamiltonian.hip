@@ -274,20 +274,28 @@ int periodic_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, 
   if (h->has_kpoint && !is_complex) return fail(OCTHIP_ERR_INVALID, "Bloch phases need a complex batch");
   int rc = ensure_work(h, ldf, s);
   if (rc) return rc;
-  if (set_bc) {
-    rc = h->periodic ? launch_periodic_bc(psi, h->d_bnd_src, np, h->nbnd, L,
-                                          (has_phase && h->has_kpoint) ? h->d_phase_corr : nullptr, s)
-                     : zero_boundary(psi, np, np_part, L, s);
-    if (rc) return rc;
-  }
   const double* src = psi;
   const bool set_phase = h->has_kpoint && !has_phase;
+  double* e = nullptr;
   if (set_phase) {
-    double* e = nullptr;
     rc = ensure_ephase(h, ldf, s, &e);
-    if (!rc) rc = launch_phase(e, psi, h->d_phase, np_part, L, false, s);
     if (rc) return rc;
     src = e;
+  }
+  if (set_bc && h->periodic && set_phase) {
+    rc = launch_periodic_phase(e, psi, h->d_phase, h->d_bnd_src, np, np_part, L, s);
+    if (rc) return rc;
+  } else {
+    if (set_bc) {
+      rc = h->periodic ? launch_periodic_bc(psi, h->d_bnd_src, np, h->nbnd, L,
+                                            (has_phase && h->has_kpoint) ? h->d_phase_corr : nullptr, s)
+                       : zero_boundary(psi, np, np_part, L, s);
+      if (rc) return rc;
+    }
+    if (set_phase) {
+      rc = launch_phase(e, psi, h->d_phase, np_part, L, false, s);
+      if (rc) return rc;
+    }
   }
   if ((terms & OCTHIP_TERM_NON_LOCAL_POTENTIAL) && h->nmat > 0) {
     rc = run_bra(h, src, L, s, nullptr);
@@ -300,10 +308,10 @@ int periodic_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, 
   a.fo = hpsi;
   a.L = L;
   a.lim = np_part;  // boundary rows as set above (or by the caller)
-  rc = launch_operator(h->kin, a, EPI_STORE, s);
-  if (!rc && set_phase) rc = launch_phase(hpsi, hpsi, h->d_phase, np, L, true, s);
-  return rc;
+  a.out_phase = set_phase ? h->d_phase : nullptr;
+  return launch_operator(h->kin, a, EPI_STORE, s);
 }
+
 // Ket tables of a handle (KetArgs, BraReduceArgs::row).
 struct KetTables {
   std::vector<int> slot, g;

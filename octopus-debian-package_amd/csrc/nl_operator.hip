@@ -427,7 +427,11 @@ int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t
   if (!a.fi || !a.zrow || (a.kslot && !a.ksum) || (epi == EPI_STORE && !a.fo))
     return fail(OCTHIP_ERR_STATE, "apply: incomplete kernel arguments");
   const bool zm = op->zmarch_ok && op->kernel != 1 && a.n == 25 && zmarch_fits(op, a);
-  if (!zm) return launch_apply(a, op->lattice && a.n > 0, epi, s);
+  if (!zm) {
+    const int rc = launch_apply(a, op->lattice && a.n > 0, epi, s);
+    if (rc || !a.out_phase) return rc;
+    return launch_phase(a.fo, a.fo, a.out_phase, a.np, a.L, true, s);
+  }
   int lc, lpt;
   zmarch_shape(op, a.L, &lc, &lpt);
   const int zs = zmarch_zseg_for(op, a.L, epi, a.kslot != nullptr);
@@ -446,7 +450,8 @@ int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t
   z.a.nt = zmarch_nt(op, a);
   z.rec = op->d_rec;
   z.sched = sched;
-  return launch_zmarch(z, lc, lpt, epi, len, s);
+  // the phased store takes the plan of the plain one: it adds 16 bytes per row
+  return launch_zmarch(z, lc, lpt, a.out_phase ? EPI_PHASE : epi, len, s);
 }
 }  // namespace octhip
 

@@ -294,6 +294,8 @@ void drop_workset(octhip_hamiltonian_s* h, hipStream_t s);
 int propagator_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, hipStream_t s);
 inline bool is_periodic(const octhip_hamiltonian_s* h) { return h->periodic || h->has_kpoint; }
 int launch_periodic_bc(double* f, const int* src, int np, int nb, int L, const double* corr, hipStream_t s);
+int launch_periodic_phase(double* e, double* f, const double* phase, const int* src, int np, int np_part, int L,
+                          hipStream_t s);
 int launch_phase(double* dst, const double* src, const double* phase, int n, int L, bool conjugate, hipStream_t s);
 // nvec Krylov-style buffers of np_part rows of the stream's set (Lanczos, Chebyshev, and
 // the Taylor chain of periodic handles)

@@ -135,7 +135,7 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
   const int col = threadIdx.x / PAIRS;
   const int cx = col % ZTX, cy = col / ZTX;
   const int l = chunk * LC + kp * LPT;         // first lane of this thread
-  constexpr bool TAY = EPI != EPI_STORE;
+  constexpr bool TAY = EPI == EPI_TAYLOR || EPI == EPI_TAYLOR_X;
   const bool has_acc = TAY && a_acc != nullptr;
   // row q of an array starts at byte q << sh; arrays without a role here get no records
   const int sh = __builtin_ctz((unsigned)A.L) + 3;
@@ -145,7 +145,8 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
   const auto r_ks = zrsrc(A.kslot, NL ? (uint32_t)a_np * 4u : 0u);
   const auto r_k = zrsrc(A.ksum, NL ? (uint32_t)A.nk << sh : 0u);
   const auto r_ai = zrsrc(A.acc_in ? A.acc_in : a_acc, has_acc ? np_bytes : 0u);
-  const auto r_fo = zrsrc(A.fo, EPI == EPI_STORE ? np_bytes : 0u);
+  const auto r_fo = zrsrc(A.fo, TAY ? 0u : np_bytes);
+  const auto r_ph = zrsrc(A.out_phase, EPI == EPI_PHASE ? (uint32_t)a_np * 16u : 0u);
   const auto r_y = zrsrc(A.yout, (TAY && A.yout) ? np_bytes : 0u);
   const auto r_acc = zrsrc(a_acc, has_acc ? np_bytes : 0u);
   const auto r_ya = zrsrc(A.ya, (has_acc && A.ya) ? np_bytes : 0u);  // earlier powers, last order
@@ -183,6 +184,8 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
   Rec rec[4];
   double vr[4];
   uint32_t vd[4];  // QUAD: half of the potential per lane
+  Vec<2> ph[EPI == EPI_PHASE ? 4 : 1];  // Bloch phase, QUAD: a quarter of it per lane in pd
+  uint32_t pd[EPI == EPI_PHASE ? 4 : 1];
   Vec<LPT> kr[4], ar[TAY ? 4 : 1], ra[TAY ? 4 : 1], rb[TAY ? 4 : 1];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -274,6 +277,22 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
         }
         if constexpr (EPI == EPI_STORE) {
           bst<LPT>(r_fo, qo, s, a_nt);
+        } else if constexpr (EPI == EPI_PHASE) {
+          double pr = ph[kk & 3].v[0], pi = ph[kk & 3].v[1];
+          if constexpr (QUAD) {
+            const uint32_t d = pd[kk & 3];
+            pr = __builtin_bit_cast(double, (uint64_t)quad_bcast<1>(d) << 32 | quad_bcast<0>(d));
+            pi = __builtin_bit_cast(double, (uint64_t)quad_bcast<3>(d) << 32 | quad_bcast<2>(d));
+          }
+          pi = -pi;
+          Vec<LPT> o;
+          if constexpr (LPT == 2) {
+            o.v[0] = zmul_lane(pr, pi, s.v[0], s.v[1], false);
+            o.v[1] = zmul_lane(pr, pi, s.v[1], s.v[0], true);
+          } else {
+            o.v[0] = zmul_lane(pr, pi, s.v[0], __shfl_xor(s.v[0], 1), (l & 1) != 0);
+          }
+          bst<LPT>(r_fo, qo, o, a_nt);
         } else {
           bst<LPT>(r_y, qo, s, a_nt);  // dropped when there is no yout
           Vec<LPT> av = ar[kk & 3];
@@ -337,6 +356,11 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
         const uint32_t qv = in ? poff(qp, 3) : NONE;
         if constexpr (QUAD) vd[(kk + AD) & M] = __builtin_amdgcn_raw_buffer_load_b32(r_v, qv + (in ? (threadIdx.x & 1) * 4u : 0u), 0, 0);
         else vr[(kk + AD) & M] = bld<1>(r_v, qv).v[0];
+        if constexpr (EPI == EPI_PHASE) {
+          const uint32_t qh = in ? poff(qp, 4) : ~0u - 15u;
+          if constexpr (QUAD) pd[(kk + AD) & M] = __builtin_amdgcn_raw_buffer_load_b32(r_ph, qh + (in ? (threadIdx.x & 3) * 4u : 0u), 0, 0);
+          else ph[(kk + AD) & M] = bld<2>(r_ph, qh);
+        }
         if constexpr (NL) {
           // most waves have no ket row on a plane
           Vec<LPT> kv;

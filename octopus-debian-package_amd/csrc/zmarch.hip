@@ -21,6 +21,12 @@ int launch_nl(const ZArgs& z, int epi, int grid, size_t shmem, hipStream_t s) {
     } else {
       return fail(OCTHIP_ERR_INVALID, "z-march Taylor epilogue needs complex lane pairs");
     }
+  } else if (epi == EPI_PHASE) {
+    if constexpr (LC >= 2) {
+      hipLaunchKernelGGL((k_zmarch<LPT, LC, EPI_PHASE, NL>), dim3(grid), dim3(NT), shmem, s, z);
+    } else {
+      return fail(OCTHIP_ERR_INVALID, "z-march Bloch phases need complex lane pairs");
+    }
   } else {
     hipLaunchKernelGGL((k_zmarch<LPT, LC, EPI_STORE, NL>), dim3(grid), dim3(NT), shmem, s, z);
   }

@@ -385,8 +385,9 @@ int octhip_batched_destroy(octhip_batched_t batched);
  * discrete propagator: given chi_N with dJ = 2 Re <chi_N|d psi_N> (<a|b> = vol_pp sum
  * conj(a) b), backward returns dJ/d eps_s (host, nsteps) and dJ/dv(r) (device, np) and
  * leaves chi_0 = dJ/d psi_0* in chi.  Forward stores psi every checkpoint_every steps;
- * backward recomputes each segment from its checkpoint, the next segment on an internal
- * second stream while the current one runs backward, and accumulates the gradients on a
+ * backward takes the last two segments' states as forward left them (once, and if the
+ * potential is still the same) and recomputes every other segment from its checkpoint, the
+ * next segment on an internal second stream while the current one runs backward, and accumulates the gradients on a
  * third (memory: ceil(nsteps/K) checkpoints of np rows plus 2*(K+1) + 2*K*(order-1) +
  * 2*order + 2 batches of np rows; the Hamiltonian's work set for the second stream exists
  * only while backward runs).

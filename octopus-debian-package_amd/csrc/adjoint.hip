@@ -11,7 +11,11 @@
 // gradient (src/opt_control/propagation.F90:1016-1103, d_j = 2 Im <chi|x pol_j|psi>) is
 // its first-order-in-dt limit.  psi_s is restored from checkpoints every K steps
 // (oct_prop_init/oct_prop_check, propagation.F90:1108-1205, keep states at fixed
-// intervals) and recomputed forward inside each segment, keeping the H^k psi_s terms.
+// intervals) and recomputed forward inside each segment, keeping the H^k psi_s terms.  The
+// two buffer sets that the backward recomputes into are idle during the forward, which
+// leaves the states and terms of its last two segments there: they are not recomputed by
+// the backward that follows (R = 10 sphere, 32 states, 20 steps in segments of 10, forward
+// and backward: 17.2 ms instead of 24.8; 20 of 60 Taylor steps less).
 #include <algorithm>
 #include <cmath>
 #include <complex>
@@ -163,6 +167,8 @@ struct octhip_adjoint_s {
   hipEvent_t ev_chi[2] = {nullptr, nullptr}, ev_acc[2] = {nullptr, nullptr};
   int nckpt = 0;
   std::vector<double> eps;      // field of every step (set by forward)
+  int held[2] = {-1, -1};       // segment whose states the forward left in each set, or -1
+  long held_of = 0;             // ... with the Hamiltonian in this state
   bool forward_done = false;
 };
 
@@ -195,6 +201,19 @@ int step_field(octhip_adjoint_s* a, int s, hipStream_t st) {
 }
 
 size_t rows_bytes(size_t rows, int L) { return sizeof(double) * rows * (size_t)L; }
+
+// Step i of segment c: psi_s (the segment's checkpoint for i = 0) and, from index 1, the
+// terms H^k psi_s, in buffer set c & 1
+double* segment_psi(const octhip_adjoint_s* a, int c, int i) {
+  const size_t arr = (size_t)a->h->np * a->L;
+  return i == 0 ? a->d_ckpt + (size_t)c * arr : a->d_slot + ((size_t)(c & 1) * (a->K + 1) + i) * arr;
+}
+void segment_terms(const octhip_adjoint_s* a, int c, int i, double** ys) {
+  const size_t arr = (size_t)a->h->np * a->L;
+  ys[0] = segment_psi(a, c, i);
+  for (int k = 1; k < a->order; ++k)
+    ys[k] = a->d_seg + (((size_t)(c & 1) * a->K + i) * (a->order - 1) + (k - 1)) * arr;
+}
 
 }  // namespace
 
@@ -277,15 +296,30 @@ extern "C" int octhip_adjoint_forward(octhip_adjoint_t a, double* psi, const dou
   hipStream_t s = (hipStream_t)stream;
   const int np = a->h->np;
   for (int i = 0; i < a->nsteps; ++i) a->eps[i] = eps[i];
+  a->held[0] = a->held[1] = -1;
+  // in place up to the last two segments, then from buffer to buffer, psi_N into psi
+  const int first = std::max(a->nckpt - 2, 0) * a->K;
   for (int st = 0; st < a->nsteps; ++st) {
-    if (st % a->K == 0) {
-      OCTHIP_HIP(hipMemcpyAsync(a->d_ckpt + (size_t)(st / a->K) * np * a->L, psi, rows_bytes(np, a->L),
-                                hipMemcpyDeviceToDevice, s));
-    }
+    const int c = st / a->K, i = st % a->K;
+    if (i == 0 && st <= first)
+      OCTHIP_HIP(hipMemcpyAsync(segment_psi(a, c, 0), psi, rows_bytes(np, a->L), hipMemcpyDeviceToDevice, s));
     int rc = step_field(a, st, s);
-    if (!rc) rc = taylor_step(a->h, psi, a->ldf, a->dt, a->order, 0, nullptr, s);
+    if (rc) return rc;
+    if (st < first) {
+      rc = taylor_step(a->h, psi, a->ldf, a->dt, a->order, 0, nullptr, s);
+    } else {
+      double* ys[ADJ_MAX_ORDER];
+      segment_terms(a, c, i, ys);
+      double* out = st + 1 == a->nsteps ? psi : i + 1 == a->K ? segment_psi(a, c + 1, 0) : segment_psi(a, c, i + 1);
+      rc = taylor_step(a->h, out, a->ldf, a->dt, a->order, 0, ys, s, ys[0]);
+    }
     if (rc) return rc;
   }
+  // the steps in place clear psi's boundary rows
+  int rc = zero_boundary(psi, np, a->h->kin->np_part, a->L, s);
+  if (rc) return rc;
+  for (int c = std::max(a->nckpt - 2, 0); c < a->nckpt; ++c) a->held[c & 1] = c;
+  a->held_of = a->h->changes;
   a->forward_done = true;
   return OCTHIP_SUCCESS;
 }
@@ -337,7 +371,6 @@ int backward_run(octhip_adjoint_s* a, double* chi, double* dj_deps, double* dj_d
   // of segment c + 2 (the same set) to finish reading, and the backward of c waits for
   // recompute(c).  Each stream forms its own potential v + eps_s x (d_veff[0] recompute,
   // d_veff[1] backward) and has its own work buffers.
-  const size_t slot_set = (size_t)(a->K + 1) * arr, seg_set = (size_t)a->K * (order - 1) * arr;
   double* const vr = a->d_veff;
   double* const vb = a->d_veff + np;
   hipStream_t s2 = a->aux;
@@ -345,22 +378,26 @@ int backward_run(octhip_adjoint_s* a, double* chi, double* dj_deps, double* dj_d
     for (int d = 0; d < 3; ++d) f[d] = a->eps[st] * a->pol[d];
   };
   bool back_recorded[2] = {false, false};
+  // used once, and only with the potential of the forward: a further backward, or one after
+  // a new potential, recomputes every segment
+  const bool same = a->held_of == a->h->changes;
+  const int held[2] = {same ? a->held[0] : -1, same ? a->held[1] : -1};
+  a->held[0] = a->held[1] = -1;
   auto recompute = [&](int c) -> int {
     const int b = c & 1;
+    if (held[b] == c) return OCTHIP_SUCCESS;  // there already, queued on the caller's side of ev_fork
     if (back_recorded[b]) OCTHIP_HIP(hipStreamWaitEvent(s2, a->ev_back[b], 0));
-    double* slot = a->d_slot + b * slot_set;
-    double* seg = a->d_seg + b * seg_set;
     const int s0 = c * a->K, s1 = std::min(s0 + a->K, a->nsteps);
-    OCTHIP_HIP(hipMemcpyAsync(slot, a->d_ckpt + (size_t)c * np * L, rows_bytes(np, L), hipMemcpyDeviceToDevice, s2));
     double* ys[ADJ_MAX_ORDER];
     for (int st = s0; st < s1; ++st) {
       const int i = st - s0;
-      ys[0] = slot + (size_t)i * arr;
-      for (int k = 1; k < order; ++k) ys[k] = seg + ((size_t)i * (order - 1) + (k - 1)) * arr;
+      segment_terms(a, c, i, ys);
       double f[3];
       field_of(st, f);
       int rc = launch_veff(a->h, vr, f, s2);
-      if (!rc) rc = taylor_step(a->h, slot + (size_t)(i + 1) * arr, a->ldf, a->dt, order, 0, ys, s2, ys[0], vr);
+      if (!rc)
+        rc = taylor_step(a->h, a->d_slot + ((size_t)b * (a->K + 1) + i + 1) * arr, a->ldf, a->dt, order, 0, ys, s2,
+                         ys[0], vr);
       if (rc) return rc;
     }
     OCTHIP_HIP(hipEventRecord(a->ev_rec[b], s2));
@@ -378,9 +415,7 @@ int backward_run(octhip_adjoint_s* a, double* chi, double* dj_deps, double* dj_d
       rc = recompute(c - 1);
       if (rc) return rc;
     }
-    OCTHIP_HIP(hipStreamWaitEvent(s, a->ev_rec[b], 0));
-    double* slot = a->d_slot + b * slot_set;
-    double* seg = a->d_seg + b * seg_set;
+    if (held[b] != c) OCTHIP_HIP(hipStreamWaitEvent(s, a->ev_rec[b], 0));
     const int s0 = c * a->K, s1 = std::min(s0 + a->K, a->nsteps);
     // backward through the segment
     for (int st = s1 - 1; st >= s0; --st, ++t) {
@@ -399,8 +434,9 @@ int backward_run(octhip_adjoint_s* a, double* chi, double* dj_deps, double* dj_d
       if (rc) return rc;
       OCTHIP_HIP(hipEventRecord(a->ev_chi[u], s));
       OCTHIP_HIP(hipStreamWaitEvent(s3, a->ev_chi[u], 0));
-      acc.yp[0] = slot + (size_t)i * arr;
-      for (int k = 1; k < order; ++k) acc.yp[k] = seg + ((size_t)i * (order - 1) + (k - 1)) * arr;
+      double* yp[ADJ_MAX_ORDER];
+      segment_terms(a, c, i, yp);
+      for (int k = 0; k < order; ++k) acc.yp[k] = yp[k];
       acc.yc[0] = cur;
       for (int m = 1; m < order; ++m) acc.yc[m] = ychi + m * arr;
       {

@@ -598,6 +598,7 @@ extern "C" int octhip_hamiltonian_set_potential(octhip_hamiltonian_t h, const do
     int rc = dalloc((void**)&h->d_v, sizeof(double) * h->np);
     if (rc) return rc;
   }
+  ++h->changes;
   OCTHIP_HIP(hipMemcpyAsync(h->d_v, vlocal, sizeof(double) * h->np, hipMemcpyHostToDevice, s));
   OCTHIP_HIP(hipStreamSynchronize(s));
   return update_veff(h, s);
@@ -610,6 +611,7 @@ extern "C" int octhip_hamiltonian_set_dipole_field(octhip_hamiltonian_t h, const
   hipStream_t s = (hipStream_t)stream;
   if (positions) {
     // d_veff keeps its address (captured graphs read it); only the positions are replaced
+    ++h->changes;
     dfree(h->d_xyz);
     h->d_xyz = nullptr;
     int rc = upload(&h->d_xyz, positions, 3 * (size_t)h->np, s);

@@ -182,6 +182,7 @@ struct octhip_hamiltonian_s {
   double* d_veff = nullptr;     // np: v + field . x when a dipole field is set
   double field[3] = {0, 0, 0};
   bool has_field = false;
+  long changes = 0;             // uploads of the potential or the positions
   // projectors
   int nmat = 0;
   int max_nprojs = 0;

@@ -380,8 +380,10 @@ struct KetArgs {
   // Bloch phases by entry (conjugated and multiplied onto the terms of a matrix, entry + row;
   // hamiltonian_elec_base_inc.F90:955-966); null: none
   const double* __restrict__ phase = nullptr;
+  // with out: the rows are added to the mesh rows `point` of out instead (kbuf unused)
+  double* out = nullptr;
+  const int* __restrict__ point = nullptr;
 };
-
 
 // Bra by sets: the same groups as the ket's, so the row of a mesh point inside several
 // spheres is read once and feeds the projectors of all of them, 16 projector rows at a time

@@ -1,7 +1,7 @@
 // Kernel instances and launchers: fused apply, projector bra (FP64 MFMA and plain).
 #include <algorithm>
 
-#include "kernels.h"
+#include "bra.h"
 
 namespace octhip {
 
@@ -117,9 +117,6 @@ __global__ __launch_bounds__(BLOCK) void k_bra_plain(const BraArgs b) { bra_plai
 // A comes from the transposed projector table (16 lanes read consecutive doubles of one
 // sphere point's row), B from the state rows (16 lanes read 128 contiguous bytes, 256
 // with two columns per lane).
-typedef double d4 __attribute__((ext_vector_type(4)));
-
-
 // One workgroup per (chunk, lane tile of 16 TW lanes): grids of nchunk * L/(16 TW) blocks
 // keep every CU busy; the 4 waves take interleaved groups of 4 sphere points and are
 // summed through LDS in a fixed order.  Every load is issued unconditionally (clamped
@@ -207,104 +204,6 @@ __device__ __forceinline__ void bra_mfma_body(const BraMfmaArgs& m, int c, int l
   }
 }
 
-// Bra by sets.  A wave takes one group of <= 16 mesh points: its 4 state loads and the
-// projector loads of its first 32 projector rows are in flight together, and a product
-// A(16 projector rows x 4 points) B(4 points x 16 lanes) serves up to 4 matrices of 4
-// projectors.  Lane (kk, ii) supplies A[ii][kk] = P[row ii, point kk] from line step(ii/4) of
-// the group (32-byte runs) and gets D[4r+kk][ii]: rows 4r .. 4r+3 are those of step r.  The
-// sums go to the wave's part of LDS and the 4 waves are added in a fixed order.  No row of a
-// group takes part in a matrix it does not belong to, and operands past its points are zero.
-// PHASE: the states times the Bloch phases of (point, matrix), which differ by matrix: a
-// product per step, of which D rows 4r .. 4r+3 are kept.
-template <int TW, bool PHASE>
-__device__ __forceinline__ void bra_set_body(const BraMfmaArgs& m, int bl, int lt, double* red) {
-  constexpr int TL = 16 * TW;
-  static_assert(BRA_SET_GROUPS == BLOCK / 64, "a group per wave");
-  const BraArgs& b = m.b;
-  const BraSetArgs& a = m.set;
-  const int4 blk = a.blk[bl];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
-  const int kk = ln >> 4, ii = ln & 15;
-  const int col = lt * TL + ii * TW;
-  const int sums = blk.w * b.pjmax * TL;      // LDS doubles of a wave
-  double* const mine = red + (size_t)wave * sums;
-  const KetGroup gr = a.grp[blk.x + min(wave, blk.y - 1)];
-  const int n = gr.rows, ns = gr.steps;
-  int p[4], row[4];
-  double av[2][4];                            // projector rows 0 .. 15 and 16 .. 31
-  Vec<TW> bv[4];
-  const double* const pt = a.pt + 4 * (size_t)gr.line + (ii & 3);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    p[k] = min(4 * k + kk, n - 1);
-    row[k] = a.point[gr.row + p[k]];
-    av[0][k] = pt[4 * (size_t)(min(ii >> 2, ns - 1) * n + p[k])];
-  }
-  if (ns > 4)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) av[1][k] = pt[4 * (size_t)(min(4 + (ii >> 2), ns - 1) * n + p[k])];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) bv[k] = ldv<TW>(b.psi + (size_t)row[k] * b.L + col);
-  for (int t = ln; t < sums; t += 64) mine[t] = 0.0;
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  if (wave < blk.y) {
-    for (int t0 = 0; t0 < ns; t0 += 4) {      // 16 projector rows at a time
-      double x[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        x[k] = t0 == 0   ? av[0][k]
-               : t0 == 4 ? av[1][k]
-                         : pt[4 * (size_t)(min(t0 + (ii >> 2), ns - 1) * n + p[k])];
-        x[k] = 4 * k + kk < n ? x[k] : 0.0;
-      }
-      d4 acc[TW];
-      const auto product = [&](const Vec<TW>* v) {
-#pragma unroll
-        for (int w = 0; w < TW; ++w) acc[w] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-          for (int w = 0; w < TW; ++w)
-            acc[w] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[k], 4 * k + kk < n ? v[k].v[w] : 0.0, acc[w], 0, 0, 0);
-      };
-      if constexpr (!PHASE) product(bv);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (t0 + r >= ns) break;
-        if constexpr (PHASE) {
-          const size_t ent = a.step[gr.step + t0 + r].z;
-          Vec<TW> ph[4];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const double pr = a.phase[2 * (ent + p[k])], pi = a.phase[2 * (ent + p[k]) + 1];
-            if constexpr (TW == 2) {
-              ph[k].v[0] = zmul_lane(pr, pi, bv[k].v[0], bv[k].v[1], false);
-              ph[k].v[1] = zmul_lane(pr, pi, bv[k].v[1], bv[k].v[0], true);
-            } else {
-              ph[k].v[0] = zmul_lane(pr, pi, bv[k].v[0], __shfl_xor(bv[k].v[0], 1), (col & 1) != 0);
-            }
-          }
-          product(ph);
-        }
-        // a matrix that holds the point twice adds to its rows twice
-        const int sum = t0 == 0 ? gr.sum[r] : a.step[gr.step + t0 + r].y;
-        double* const d = mine + (sum + kk) * TL + ii * TW;
-        Vec<TW> v = ldv<TW>(d);
-#pragma unroll
-        for (int w = 0; w < TW; ++w) v.v[w] += acc[w][r];
-        stv<TW>(d, v);
-      }
-    }
-  }
-  __syncthreads();
-  for (int t = threadIdx.x; t < sums; t += BLOCK) {
-    const int q = t / TL, slot = q / b.pjmax;
-    const double v = (red[t] + red[t + sums]) + (red[t + 2 * (size_t)sums] + red[t + 3 * (size_t)sums]);
-    b.partial[((size_t)a.part[blk.z + slot] * b.pjmax + (q - slot * b.pjmax)) * b.L + lt * TL + (t - q * TL)] = v;
-  }
-}
-
 extern __shared__ double2 bra_lds[];
 template <bool SETS, bool PHASE>
 __device__ __forceinline__ void bra_mfma(const BraMfmaArgs& m, int b) {
@@ -312,8 +211,8 @@ __device__ __forceinline__ void bra_mfma(const BraMfmaArgs& m, int b) {
   const int nlt = mfma_lane_tiles(m.b.L);
   const bool wide = (m.b.L & 31) == 0;
   if constexpr (SETS) {
-    if (wide) bra_set_body<2, PHASE>(m, b / nlt, b % nlt, red);
-    else bra_set_body<1, PHASE>(m, b / nlt, b % nlt, red);
+    if (wide) bra_set_body<2, PHASE>(m, b / nlt, b % nlt, red, threadIdx.x, true);
+    else bra_set_body<1, PHASE>(m, b / nlt, b % nlt, red, threadIdx.x, true);
   } else {
     if (wide) bra_mfma_body<2>(m, b / nlt, b % nlt, red);
     else bra_mfma_body<1>(m, b / nlt, b % nlt, red);
@@ -405,7 +304,7 @@ int launch_bra_mfma(BraMfmaArgs& m, size_t lds, hipStream_t s) {
 // A wave's loads are a chain of round trips (group, then its operands), which is what
 // bounds this kernel: a group's record holds its first KET_AHEAD steps, whose operands are
 // loaded together, and a wave has one group.
-template <int TW, bool PHASE>
+template <int TW, bool PHASE, bool ADD>
 __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
   constexpr int TL = 16 * TW;                 // lanes of the tile
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
@@ -417,6 +316,11 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
   const int n = gr.rows, ns = gr.steps;
   const double* const pt = k.pt + 4 * ((size_t)gr.line + min(ii, n - 1)) + kk;
   const double* const pj = k.proj + (size_t)kk * k.L + col;
+  int p[ADD ? 4 : 1];                         // ADD: mesh rows 4r+kk of the group
+  if constexpr (ADD) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] = k.point[gr.row + min(4 * r + kk, n - 1)];
+  }
   d4 acc[TW], tot[TW];
 #pragma unroll
   for (int w = 0; w < TW; ++w) acc[w] = tot[w] = d4{0.0, 0.0, 0.0, 0.0};
@@ -436,6 +340,7 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
       }
     }
   };
+  Vec<TW> old[ADD ? 4 : 1];
   for (int q0 = 0; q0 < ns; q0 += KET_AHEAD) {
     double av[KET_AHEAD];
     Vec<TW> bv[KET_AHEAD];
@@ -444,6 +349,11 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
       const int q = min(q0 + u, ns - 1);
       av[u] = pt[4 * (size_t)(q * n)];
       bv[u] = ldv<TW>(pj + (size_t)(q0 == 0 ? gr.proj[u] : k.step[gr.step + q].x) * k.L);
+    }
+    if constexpr (ADD) {
+      if (q0 == 0)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) old[r] = ldv<TW>(k.out + (size_t)p[r] * k.L + col);
     }
 #pragma unroll
     for (int u = 0; u < KET_AHEAD; ++u) {
@@ -471,17 +381,17 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
     if (4 * r + kk < n) {
       Vec<TW> o;
 #pragma unroll
-      for (int w = 0; w < TW; ++w) o.v[w] = acc[w][r];
-      stv<TW>(k.kbuf + (size_t)(gr.row + 4 * r + kk) * k.L + col, o);
+      for (int w = 0; w < TW; ++w) o.v[w] = ADD ? old[ADD ? r : 0].v[w] + acc[w][r] : acc[w][r];
+      stv<TW>(ADD ? k.out + (size_t)p[ADD ? r : 0] * k.L + col : k.kbuf + (size_t)(gr.row + 4 * r + kk) * k.L + col, o);
     }
   }
 }
 
-template <bool PHASE>
+template <bool PHASE, bool ADD = false>
 __device__ __forceinline__ void ket_mfma(const KetArgs& k, int b) {
   const int nlt = mfma_lane_tiles(k.L);
-  if ((k.L & 31) == 0) ket_mfma_body<2, PHASE>(k, b / nlt, b % nlt);
-  else ket_mfma_body<1, PHASE>(k, b / nlt, b % nlt);
+  if ((k.L & 31) == 0) ket_mfma_body<2, PHASE, ADD>(k, b / nlt, b % nlt);
+  else ket_mfma_body<1, PHASE, ADD>(k, b / nlt, b % nlt);
 }
 
 // plain form, any row length: a wave per group, one thread per (row, lane)
@@ -518,8 +428,8 @@ __device__ __forceinline__ void ket_plain_body(const KetArgs& k, int b) {
   }
 }
 
-template <bool PHASE>
-__global__ __launch_bounds__(BLOCK) void k_ket_mfma(const KetArgs k) { ket_mfma<PHASE>(k, blockIdx.x); }
+template <bool PHASE, bool ADD>
+__global__ __launch_bounds__(BLOCK) void k_ket_mfma(const KetArgs k) { ket_mfma<PHASE, ADD>(k, blockIdx.x); }
 __global__ __launch_bounds__(BLOCK) void k_ket_plain(const KetArgs k) { ket_plain_body(k, blockIdx.x); }
 
 int launch_ket(const KetArgs& k, bool mfma, hipStream_t s) {
@@ -528,10 +438,13 @@ int launch_ket(const KetArgs& k, bool mfma, hipStream_t s) {
   mfma = mfma && k.L >= 16;
   ProfScope prof("k_ket", s);
   const dim3 tiles(nblock * mfma_lane_tiles(k.L));  // 32-lane tiles when the row length allows, else 16
-  if (mfma && k.phase)
-    hipLaunchKernelGGL(k_ket_mfma<true>, tiles, dim3(BLOCK), 0, s, k);
+  if (k.out && (!mfma || k.phase)) return fail(OCTHIP_ERR_STATE, "ket: no form that adds to the output rows");
+  if (k.out)
+    hipLaunchKernelGGL((k_ket_mfma<false, true>), tiles, dim3(BLOCK), 0, s, k);
+  else if (mfma && k.phase)
+    hipLaunchKernelGGL((k_ket_mfma<true, false>), tiles, dim3(BLOCK), 0, s, k);
   else if (mfma)
-    hipLaunchKernelGGL(k_ket_mfma<false>, tiles, dim3(BLOCK), 0, s, k);
+    hipLaunchKernelGGL((k_ket_mfma<false, false>), tiles, dim3(BLOCK), 0, s, k);
   else
     hipLaunchKernelGGL(k_ket_plain, dim3(nblock), dim3(BLOCK), 0, s, k);
   hipError_t e = hipGetLastError();

@@ -369,6 +369,7 @@ int zmarch_sched(octhip_nl_operator_s::ZPlan* pl, int nchunk, const int4** out, 
 }
 
 int launch_zmarch(const ZArgs& z, int lc, int lpt, int epi, int grid, hipStream_t s);
+int launch_zmarch_bra(const ZArgs& z, const BraMfmaArgs& m, int nz, hipStream_t s);
 
 // The z-march addresses rows with 32-bit byte offsets: every row array it touches (psi
 // over np_part rows, the outputs over np, the ket rows) must satisfy
@@ -408,7 +409,8 @@ int prepare_operator(octhip_nl_operator_s* op, int L, bool nl) {
     rc = zmarch_sched(pl, L / lc, &sched, &len);
     if (rc) return rc;
   }
-  return OCTHIP_SUCCESS;
+  // a pass that takes the bra along has no ket rows
+  return nl ? prepare_operator(op, L, false) : OCTHIP_SUCCESS;
 }
 
 // The z-march writes one density partial per lane chunk of a row, the gather kernel one
@@ -421,9 +423,18 @@ int apply_lane_chunks(const octhip_nl_operator_s* op, const ApplyArgs& a) {
   return a.L / lc;
 }
 
+// Whether the pass of `a` (EPI_STORE) can take along a bra by sets whose blocks need lds bytes
+// each: it goes by the z-march in the shape of k_zmarch_bra, whose windows hold two such blocks.
+bool operator_takes_bra(const octhip_nl_operator_s* op, const ApplyArgs& a, size_t lds) {
+  int lc, lpt;
+  zmarch_shape(op, a.L, &lc, &lpt);
+  return op->zmarch_ok && op->kernel != 1 && a.n == 25 && zmarch_fits(op, a) && lc == 16 && lpt == 2 &&
+         lds <= sizeof(double) * ZB_RED;
+}
+
 // Apply through the best kernel for this operator: z-march for the order-4 star on a
 // lattice, the tiled gather otherwise.
-int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t s) {
+int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t s, const BraMfmaArgs* bra = nullptr) {
   if (!a.fi || !a.zrow || (a.kslot && !a.ksum) || (epi == EPI_STORE && !a.fo))
     return fail(OCTHIP_ERR_STATE, "apply: incomplete kernel arguments");
   const bool zm = op->zmarch_ok && op->kernel != 1 && a.n == 25 && zmarch_fits(op, a);
@@ -450,6 +461,7 @@ int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t
   z.a.nt = zmarch_nt(op, a);
   z.rec = op->d_rec;
   z.sched = sched;
+  if (bra) return launch_zmarch_bra(z, *bra, len, s);
   // the phased store takes the plan of the plain one: it adds 16 bytes per row
   return launch_zmarch(z, lc, lpt, a.out_phase ? EPI_PHASE : epi, len, s);
 }

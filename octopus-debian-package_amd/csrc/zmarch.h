@@ -30,7 +30,7 @@
 // (x -4..4, y -4..-1,1..4, z -4..-1,1..4) with fma, so results are bit-identical to it.
 #pragma once
 
-#include "kernels.h"
+#include "bra.h"
 
 namespace octhip {
 
@@ -50,8 +50,10 @@ constexpr int ZPLANE = ZREC * ZNC;    // ints per plane of a tile
 
 // Prefetch depths in planes: rows (own and halo values) and output-point data (potential,
 // ket row, Taylor rows).  One plane each: 85-103 VGPRs, two 512-thread workgroups per CU; deeper
-// rings measured slower (rows 2: 166 against 163 us, output-point data 2: 163).
-template <int EPI>
+// rings measured slower (rows 2: 166 against 163 us, output-point data 2: 163), also for
+// launches of at most one workgroup per CU (rows 3 and output-point data 2, which no longer
+// fits 128 VGPRs with ket rows: 57,777 points, 8 complex states 28.9 against 24.8 us for the
+// apply; without ket rows 20.4 against 20.2; 64^3 points, 8 real functions 11.1 either way).
 struct ZDepth {
   static constexpr int rows = 1, aux = 1;
 };
@@ -169,8 +171,9 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
   const int hx_lds = ((cy + ZR) * ZW + (cx < 4 ? cx : cx + 8)) * LC + kp * LPT;
   const int hy_lds = ((cy < 4 ? cy : cy + 8) * ZW + cx + ZR) * LC + kp * LPT;
 
-  constexpr int RD = ZDepth<EPI>::rows, AD = ZDepth<EPI>::aux;
-  static_assert(RD >= 1 && RD <= 3 && AD >= 1 && AD <= 3, "prefetch depths");
+  constexpr int RD = ZDepth::rows, AD = ZDepth::aux;
+  // (the ket slot of plane 0 is loaded at step 2 - AD)
+  static_assert(RD >= 1 && RD <= 3 && AD >= 1 && AD <= 2 && AD <= RD, "prefetch depths");
   // rings, plane P (relative to the first output plane) in slot P mod the ring length:
   //   ov   own values, P in z-4 .. z+RD;    hv  halo values, P in z .. z+RD
   //   part partial sums, P in z-4 .. z-1;   ro  own row offsets, P in z-4 .. z+RD
@@ -425,6 +428,36 @@ __global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_multi(const ZArgs*
   const int4 sc = sched[blockIdx.x];
   if (sc.y <= 0) return;
   zmarch_body<LPT, LC, EPI, NL>(zs[sc.w], sc.x, sc.y, sc.z);
+}
+
+// The stencil pass without ket rows and the bra of the same input in one launch: blocks
+// 0 .. nz-1 march, the next ones hold two bra blocks each, the rest clear boundary rows
+// (BraMfmaArgs::zf).  The ket then adds its rows to the output.
+constexpr size_t ZB_RED = (size_t)ZS * 16;  // LDS doubles of one of the two bra blocks
+template <int LPT, int LC>
+__global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_bra(const ZArgs za, const BraMfmaArgs m, const int nz) {
+  static_assert(ZNC * LC / LPT == 2 * BLOCK, "two bra blocks of BLOCK threads");
+  extern __shared__ double2 zsh2[];
+  int b = blockIdx.x;
+  if (b < nz) {
+    const int4 sc = za.sched[b];
+    if (sc.y <= 0) return;
+    zmarch_body<LPT, LC, EPI_STORE, false>(za, sc.x, sc.y, sc.z);
+    return;
+  }
+  b -= nz;
+  const int nb = (m.nbra + 1) >> 1;
+  if (b < nb) {
+    const int half = __builtin_amdgcn_readfirstlane(threadIdx.x / BLOCK);
+    const int v = 2 * b + half, vb = min(v, m.nbra - 1), nlt = mfma_lane_tiles(m.b.L);
+    double* const red = reinterpret_cast<double*>(zsh2) + half * ZB_RED;
+    if ((m.b.L & 31) == 0) bra_set_body<2, false>(m, vb / nlt, vb % nlt, red, threadIdx.x % BLOCK, v == vb);
+    else bra_set_body<1, false>(m, vb / nlt, vb % nlt, red, threadIdx.x % BLOCK, v == vb);
+    return;
+  }
+  b -= nb;
+  const size_t stride = (size_t)(gridDim.x - nz - nb) * (2 * BLOCK);
+  for (size_t t = b * (size_t)(2 * BLOCK) + threadIdx.x; t < m.zcount; t += stride) m.zf[m.zfirst + t] = 0.0;
 }
 
 // longest segment a launch accepts for a lane chunk

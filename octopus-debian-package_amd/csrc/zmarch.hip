@@ -150,6 +150,17 @@ int launch_zmarch_multi(const ZArgs* zs, const int4* sched, int len, int lc, int
   return fail(OCTHIP_ERR_INVALID, "no multi z-march instance for lane chunk %d, %d lanes per thread", lc, lpt);
 }
 
+// k_zmarch_bra: 16 lanes a chunk, 2 a thread (nz blocks march)
+int launch_zmarch_bra(const ZArgs& z, const BraMfmaArgs& m, int nz, hipStream_t s) {
+  ProfScope prof("k_zmarch", s);
+  const int zero = m.zf ? (int)std::min<size_t>((m.zcount + 2 * BLOCK - 1) / (2 * BLOCK), 1024) : 0;
+  const dim3 grid(nz + (m.nbra + 1) / 2 + zero), block(2 * BLOCK);
+  hipLaunchKernelGGL((k_zmarch_bra<2, 16>), grid, block, zmarch_shmem(16), s, z, m, nz);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(OCTHIP_ERR_HIP, "k_zmarch_bra launch: %s", hipGetErrorString(e));
+  return OCTHIP_SUCCESS;
+}
+
 int launch_zmarch(const ZArgs& z, int lc, int lpt, int epi, int grid, hipStream_t s) {
   if (lpt == 2) {
     switch (lc) {

@@ -95,10 +95,11 @@ int krylov_bufs(octhip_hamiltonian_s* h, hipStream_t s, int nvec, int ldf, Krylo
   return OCTHIP_SUCCESS;
 }
 
-// factors of the nv vectors (states nst.. of the row get 0) and the scaling (1) to the device
+// factors of the nv vectors (states nst.. of the row get 0) and the scaling (1) to the device;
+// `host` holds them and has to live until the copies are done
 int upload_factors(const std::vector<cplx>& c, int nv, int nst, int ncol, const std::vector<cplx>* scale, double* coef,
-                   double* dscale, hipStream_t s) {
-  std::vector<double> host(2 * (size_t)ncol * (nv + 1));
+                   double* dscale, std::vector<double>& host, hipStream_t s) {
+  host.resize(2 * (size_t)ncol * (nv + 1));
   for (int v = 0; v <= nv; ++v)
     for (int i = 0; i < ncol; ++i) {
       const cplx z = v < nv ? (i < nst ? c[(size_t)v * nst + i] : cplx(0.0))
@@ -110,16 +111,18 @@ int upload_factors(const std::vector<cplx>& c, int nv, int nst, int ncol, const 
     OCTHIP_HIP(hipMemcpyAsync(coef, host.data(), sizeof(double) * 2 * ncol * nv, hipMemcpyHostToDevice, s));
   OCTHIP_HIP(hipMemcpyAsync(dscale, host.data() + 2 * (size_t)ncol * nv, sizeof(double) * 2 * ncol,
                             hipMemcpyHostToDevice, s));
-  OCTHIP_HIP(hipStreamSynchronize(s));  // the host vector goes out of scope
   return OCTHIP_SUCCESS;
 }
 
 // Eigenpairs of the real symmetric tridiagonal matrix (diagonal d[0..n-1], off-diagonal
-// e[0..n-2]): implicit QL with Wilkinson shifts (tql2).  z (n x n, row-major, z[i*n+k] =
-// component i of eigenvector k) starts as the identity.
-bool tridiagonal_eigen(int n, std::vector<double>& d, std::vector<double> e, std::vector<double>& z) {
-  z.assign((size_t)n * n, 0.0);
-  for (int i = 0; i < n; ++i) z[(size_t)i * n + i] = 1.0;
+// e[0..n-2]): implicit QL with Wilkinson shifts (tql2).  z[k*nc + c] = component comp[c] of
+// eigenvector k, starting as the identity; a rotation treats every component alike, so a
+// caller pays for those it asks for (the components of a vector side by side: rotations of
+// all n take the host's vector units).
+bool tridiagonal_eigen(int n, std::vector<double>& d, std::vector<double> e, const int* comp, int nc,
+                       std::vector<double>& z) {
+  z.assign((size_t)n * nc, 0.0);
+  for (int c = 0; c < nc; ++c) z[(size_t)comp[c] * nc + c] = 1.0;
   e.resize(n);
   e[n - 1] = 0.0;
   for (int l = 0; l < n; ++l) {
@@ -154,10 +157,12 @@ bool tridiagonal_eigen(int n, std::vector<double>& d, std::vector<double> e, std
           p = sn * r;
           d[i + 1] = g + p;
           g = c * r - b;
-          for (int k = 0; k < n; ++k) {
-            f = z[(size_t)k * n + i + 1];
-            z[(size_t)k * n + i + 1] = sn * z[(size_t)k * n + i] + c * f;
-            z[(size_t)k * n + i] = c * z[(size_t)k * n + i] - sn * f;
+          double* const z0 = z.data() + (size_t)i * nc;
+          double* const z1 = z0 + nc;
+          for (int k = 0; k < nc; ++k) {
+            const double t = z1[k];
+            z1[k] = sn * z0[k] + c * t;
+            z0[k] = c * z0[k] - sn * t;
           }
         }
         if (r == 0.0 && i >= l) continue;
@@ -173,7 +178,8 @@ bool tridiagonal_eigen(int n, std::vector<double>& d, std::vector<double> e, std
 // First column of f(pp * A) for the n x n Hermitian matrix whose upper triangle is
 // hm(i, j) = a[i + j*ld] (tridiagonal: the diagonal and the first superdiagonal are read),
 // f = exp or phi(x) = (e^x - 1)/x (zlalg_exp / zlalg_phi, src/math/lalg_adv.F90:216-340).
-bool krylov_function(int n, const cplx* a, int ld, cplx pp, bool phi, cplx* col) {
+// last: only its last component, which is all that a residual takes.
+bool krylov_function(int n, const cplx* a, int ld, cplx pp, bool phi, bool last, cplx* col) {
   std::vector<double> d(n), e(std::max(n - 1, 0));
   std::vector<cplx> ph(n);  // D = diag(ph): A = D T D^H with T real
   ph[0] = 1.0;
@@ -185,16 +191,21 @@ bool krylov_function(int n, const cplx* a, int ld, cplx pp, bool phi, cplx* col)
     // T(k, k+1) = conj(ph_k) b ph_{k+1} = |b|
     ph[k + 1] = m > 0.0 ? ph[k] * std::conj(b) / m : ph[k];
   }
+  std::vector<int> comp(last ? std::vector<int>{0, n - 1} : std::vector<int>(n));
+  if (!last)
+    for (int i = 0; i < n; ++i) comp[i] = i;
+  const int nc = (int)comp.size();
   std::vector<double> z;
-  if (!tridiagonal_eigen(n, d, e, z)) return false;
-  for (int i = 0; i < n; ++i) {
+  if (!tridiagonal_eigen(n, d, e, comp.data(), nc, z)) return false;
+  std::vector<cplx> f(n);
+  for (int k = 0; k < n; ++k) {
+    const cplx x = pp * d[k];
+    f[k] = phi ? (std::exp(x) - 1.0) / x : std::exp(x);
+  }
+  for (int c = last ? 1 : 0; c < nc; ++c) {
     cplx s = 0.0;
-    for (int k = 0; k < n; ++k) {
-      const cplx x = pp * d[k];
-      const cplx f = phi ? (std::exp(x) - 1.0) / x : std::exp(x);
-      s += z[(size_t)i * n + k] * f * z[k];  // z[0*n + k]: component 0 of eigenvector k
-    }
-    col[i] = ph[i] * s;  // (D U f U^T D^H e_1)_i with ph[0] = 1
+    for (int k = 0; k < n; ++k) s += z[(size_t)k * nc + c] * f[k] * z[(size_t)k * nc];  // component 0 of eigenvector k
+    col[comp[c]] = ph[comp[c]] * s;  // (D U f U^T D^H e_1)_i with ph[0] = 1
   }
   return true;
 }
@@ -267,7 +278,9 @@ extern "C" int octhip_exponential_lanczos_batch(octhip_hamiltonian_t h, double* 
   // them and sums the norm, and one copy of the results to the host; the next H-apply is
   // queued before the host waits for them, so that it runs while the projected problems are
   // solved.  (137,065 points, 16 states, 12 steps: 8.4 -> 1.7 ms against a pass per dot product,
-  // subtraction and scaling, each with a copy and a wait.)
+  // subtraction and scaling, each with a copy and a wait.)  The host solves only what a step
+  // needs, so that it is done before the H-apply is: the residuals' component from the fourth step
+  // on, all components once at the end.
   // vb(1) = inh or psi (inner rows), beta = |vb(1)|
   rc = launch_gs_update(V(0), inh ? inh : psi, nullptr, 0, L, np, nullptr, nullptr, kb.part, s);
   if (!rc) rc = launch_gs_norms(kb.part, L, np, nst, vol, 0.0, norm, kept(0), nullptr, s);
@@ -317,20 +330,27 @@ extern "C" int octhip_exponential_lanczos_batch(octhip_hamiltonian_t h, double* 
       const double nrm = kb.host[4 * (size_t)ncol + st];
       H(st, iter, iter - 1) = nrm;
       nk[(size_t)iter * nst + st] = nrm >= tiny ? nrm : 1.0;
-      if (!krylov_function(iter, &H(st, 0, 0), M, pp, inh != nullptr, &expo[(size_t)st * M]))
+      if (std::abs(H(st, iter, iter - 1)) >= tiny) happy = false;
+    }
+    // the residuals decide from the fourth step on; the step that ends the loop reports them
+    for (int st = 0; st < nst && (happy || iter > 3 || iter == order); ++st) {
+      if (!krylov_function(iter, &H(st, 0, 0), M, pp, inh != nullptr, true, &expo[(size_t)st * M]))
         return fail(OCTHIP_ERR_HIP, "Lanczos: the projected eigenproblem did not converge");
       res[st] = std::abs(H(st, iter, iter - 1) * std::abs(expo[(size_t)st * M + iter - 1]));
-      if (std::abs(H(st, iter, iter - 1)) >= tiny) happy = false;
     }
     if (happy) break;  // happy breakdown
     if (iter > 3 && *std::max_element(res.begin(), res.end()) < lanczos_tol) break;
   }
   const int used = std::min(iter, order);  // a completed loop adds vb(order+1) with factor 0
+  for (int st = 0; st < nst; ++st)
+    if (!krylov_function(used, &H(st, 0, 0), M, pp, inh != nullptr, false, &expo[(size_t)st * M]))
+      return fail(OCTHIP_ERR_HIP, "Lanczos: the projected eigenproblem did not converge");
   if (iterations) *iterations = used;
   if (residual) *residual = *std::max_element(res.begin(), res.end());
   // inh: psi += deltat nrm V expo(:, 1)  (exponential.F90:883-887); else psi = expo(1,1) psi +
   // sum_{ii >= 2} beta expo(ii,1) vb(ii)  (888-896); GS_MAX vectors per pass
-  for (int ii = inh ? 1 : 2; ii <= used || (!inh && ii == 2); ii += GS_MAX) {
+  std::vector<std::vector<double>> staged;
+  for (int ii = inh ? 1 : 2; !rc && (ii <= used || (!inh && ii == 2)); ii += GS_MAX) {
     const int nv = std::max(0, std::min(GS_MAX, used - ii + 1));
     std::vector<cplx> c((size_t)nv * nst), first(nst);
     const double* x[GS_MAX] = {};
@@ -344,11 +364,15 @@ extern "C" int octhip_exponential_lanczos_batch(octhip_hamiltonian_t h, double* 
     }
     const bool scaled = !inh && ii == 2;
     for (int st = 0; st < nst; ++st) first[st] = expo[(size_t)st * M];
-    rc = upload_factors(c, nv, nst, ncol, scaled ? &first : nullptr, kb.coef, kb.scale, s);
+    staged.emplace_back();
+    rc = upload_factors(c, nv, nst, ncol, scaled ? &first : nullptr, kb.coef, kb.scale, staged.back(), s);
+    if (!rc && hipEventRecord(kb.ready, s) != hipSuccess) rc = fail(OCTHIP_ERR_HIP, "Lanczos: event record failed");
     if (!rc) rc = launch_gs_update(psi, nullptr, x, nv, L, np, scaled ? kb.scale : nullptr, kb.coef, nullptr, s);
-    if (rc) return rc;
   }
-  return OCTHIP_SUCCESS;
+  // the staged factors go out of scope: behind the last upload, or all of the stream's work
+  const hipError_t done = rc ? hipStreamSynchronize(s) : hipEventSynchronize(kb.ready);
+  if (!rc && done != hipSuccess) rc = fail(OCTHIP_ERR_HIP, "Lanczos: %s", hipGetErrorString(done));
+  return rc;
 }
 
 extern "C" int octhip_exponential_cheby_batch(octhip_hamiltonian_t h, double* psi, int ldf, double deltat, int order,

@@ -265,8 +265,8 @@ extern "C" int octhip_batched_create(int npairs, const octhip_hamiltonian_t* hms
   b->nl = all_nl;
   b->lc = std::min(std::min(16, 2048 / ZNC), minL);  // lanes per workgroup: <= 1024 threads
   b->lpt = 2;
-  b->mfma = minL >= 16;
-  for (int i = 0; i < npairs; ++i) b->mfma = b->mfma && hms[i]->use_mfma;
+  b->mfma = true;
+  for (int i = 0; i < npairs; ++i) b->mfma = b->mfma && hms[i]->use_mfma && bra_takes_rows(hms[i], minL);
   if (b->mfma) b->bra_kind = MULTI_BRA_SETS;
   for (int i = 0; i < npairs; ++i)
     if (b->mfma && !bra_by_sets(hms[i])) b->bra_kind = MULTI_BRA_MFMA;

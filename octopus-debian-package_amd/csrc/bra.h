@@ -28,7 +28,7 @@ __device__ __forceinline__ void bra_set_body(const BraMfmaArgs& m, int bl, int l
   const int4 blk = a.blk[bl];
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63;
   const int kk = ln >> 4, ii = ln & 15;
-  const int col = lt * TL + ii * TW;
+  const int col = lt * TL + ii * TW, lc = min(col, b.L - TW);  // lanes past a short row: clamped, not stored
   const int sums = blk.w * b.pjmax * TL;      // LDS doubles of a wave
   double* const mine = red + (size_t)wave * sums;
   const KetGroup gr = a.grp[blk.x + min(wave, blk.y - 1)];
@@ -47,7 +47,7 @@ __device__ __forceinline__ void bra_set_body(const BraMfmaArgs& m, int bl, int l
 #pragma unroll
     for (int k = 0; k < 4; ++k) av[1][k] = pt[4 * (size_t)(min(4 + (ii >> 2), ns - 1) * n + p[k])];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) bv[k] = ldv<TW>(b.psi + (size_t)row[k] * b.L + col);
+  for (int k = 0; k < 4; ++k) bv[k] = ldv<TW>(b.psi + (size_t)row[k] * b.L + lc);
   for (int t = ln; t < sums; t += 64) mine[t] = 0.0;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -103,6 +103,7 @@ __device__ __forceinline__ void bra_set_body(const BraMfmaArgs& m, int bl, int l
   __syncthreads();
   for (int t = tid; t < sums && live; t += BLOCK) {
     const int q = t / TL, slot = q / b.pjmax;
+    if (lt * TL + (t - q * TL) >= b.L) continue;
     const double v = (red[t] + red[t + sums]) + (red[t + 2 * (size_t)sums] + red[t + 3 * (size_t)sums]);
     b.partial[((size_t)a.part[blk.z + slot] * b.pjmax + (q - slot * b.pjmax)) * b.L + lt * TL + (t - q * TL)] = v;
   }

@@ -117,7 +117,7 @@ int run_ket(octhip_hamiltonian_s* h, int L, int pjmax, bool sets, hipStream_t s,
 int run_bra(octhip_hamiltonian_s* h, const double* f, int L, hipStream_t s, double* zero_bc = nullptr) {
   const int np = h->kin->np, np_part = h->kin->np_part;
   if (h->nchunk == 0) return zero_bc ? zero_boundary(zero_bc, np, np_part, L, s) : OCTHIP_SUCCESS;
-  const bool mfma = h->use_mfma && L >= 16;
+  const bool mfma = h->use_mfma && bra_takes_rows(h, L);
   if (zero_bc && !mfma) {
     int rc = zero_boundary(zero_bc, np, np_part, L, s);
     if (rc) return rc;
@@ -141,7 +141,7 @@ int run_bra(octhip_hamiltonian_s* h, const double* f, int L, hipStream_t s, doub
 // to fo afterwards: the bra fills the CUs that the march leaves idle (small systems, the end of
 // a launch), and the march reads no ket rows.  The sums keep their order: results are
 // bit-identical.  With the bra and the ket in front of the march, and with it: 57,777 points,
-// 8 complex states 24.8 -> 20.2 us; 13 real ones on 79,283 points 23.5 -> 19.7; 462,781 points,
+// 8 complex states 24.8 -> 20.2 us; 13 real ones on 79,501 points 23.5 -> 19.7; 462,781 points,
 // 2 x 32 states 410 -> 380; exponential midpoint, 155,331 points, 48 states 755 -> 689.
 int apply_store(octhip_hamiltonian_s* h, ApplyArgs& a, hipStream_t s, double* zero_bc = nullptr) {
   const int L = a.L;
@@ -180,6 +180,8 @@ int padded(int nprojs) { return (nprojs + 3) / 4 * 4; }
 
 bool bra_by_sets(const octhip_hamiltonian_s* h) { return h->nsblk > 0; }
 
+bool bra_takes_rows(const octhip_hamiltonian_s* h, int L) { return L >= 16 || bra_by_sets(h); }
+
 size_t partial_doubles(const octhip_hamiltonian_s* h, size_t L) {
   return std::max((size_t)h->nchunk * h->max_nprojs, (size_t)h->set_parts * padded(h->max_nprojs)) * L;
 }
@@ -189,7 +191,7 @@ int bra_mfma_blocks(const octhip_hamiltonian_s* h, int L) {
 }
 
 size_t bra_mfma_lds(const octhip_hamiltonian_s* h, int L) {
-  const size_t lanes = L / mfma_lane_tiles(L);
+  const size_t lanes = std::max(L / mfma_lane_tiles(L), 16);
   return sizeof(double) * 4 * lanes * (bra_by_sets(h) ? h->set_sums : 16);
 }
 
@@ -213,7 +215,7 @@ void bra_mfma_args(const octhip_hamiltonian_s* h, int L, double* partial, BraMfm
   m.set.phase = h->has_kpoint ? h->d_kphase : nullptr;
   m.pt = h->d_pt;
   m.pjs = h->pjs;
-  m.nbra = L >= 16 ? bra_mfma_blocks(h, L) : 0;
+  m.nbra = bra_takes_rows(h, L) ? bra_mfma_blocks(h, L) : 0;
 }
 
 void ket_args(const octhip_hamiltonian_s* h, int L, const double* proj, double* kbuf, KetArgs& k) {

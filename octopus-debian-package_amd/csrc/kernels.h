@@ -430,6 +430,12 @@ int launch_multi(int kind, const void* args, const int* off, int nseg, int nbloc
 int launch_bra(const BraArgs& b, int nchunk, bool mfma, hipStream_t s);
 // whether the MFMA bra of h goes by sets
 bool bra_by_sets(const octhip_hamiltonian_s* h);
+// whether the MFMA bra takes rows of L lanes: by spheres whole tiles, by sets any.  A tile is
+// partly empty below 16 lanes, but its waves have all their loads in flight together, which the
+// plain form by spheres has not (H apply on 12 atoms, plain and MFMA: 9,843 points, 1 lane
+// 52 / 17.7 us, 8 lanes 30.5 / 18.1; 79,501 points, 1 lane 53 / 18.3, 8 lanes 38 / 21.4;
+// 462,781 points, 1 lane 59 / 22, 4 lanes 42 / 28, 8 lanes 55 / 34).
+bool bra_takes_rows(const octhip_hamiltonian_s* h, int L);
 // MFMA bra arguments (psi and the cleared rows are left to the caller), its blocks and its
 // dynamic LDS at rows of L lanes
 void bra_mfma_args(const octhip_hamiltonian_s* h, int L, double* partial, BraMfmaArgs& m);
@@ -441,9 +447,9 @@ size_t partial_doubles(const octhip_hamiltonian_s* h, size_t L);
 void ket_args(const octhip_hamiltonian_s* h, int L, const double* proj, double* kbuf, KetArgs& k);
 inline int ket_blocks(int ngrp) { return (ngrp + KET_GROUPS - 1) / KET_GROUPS; }
 int launch_ket(const KetArgs& k, bool mfma, hipStream_t s);
-// lane tiles of the MFMA bra and ket over rows of L lanes (L >= 16): 32-lane tiles (two
-// columns per lane) when 32 divides L, else 16-lane tiles
-__host__ __device__ inline int mfma_lane_tiles(int L) { return (L & 31) == 0 ? L >> 5 : L >> 4; }
+// lane tiles of the MFMA bra and ket over rows of L lanes: 32-lane tiles (two columns per lane)
+// when 32 divides L, else 16-lane tiles, of which a shorter row fills a part
+__host__ __device__ inline int mfma_lane_tiles(int L) { return (L & 31) == 0 ? L >> 5 : L < 16 ? 1 : L >> 4; }
 inline int bra_reduce_blocks(const BraReduceArgs& r) {
   return std::min((r.nrow * ((r.L + 15) / 16) + BLOCK / 64 - 1) / (BLOCK / 64), 4096);
 }

@@ -311,11 +311,12 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
   const int g = b * KET_GROUPS + wave;
   const int kk = ln >> 4, ii = ln & 15;
   const int col = lt * TL + ii * TW;          // first column of this lane
+  const int lc = min(col, k.L - TW);          // (columns past a short row: clamped, not stored)
   if (g >= k.ngrp) return;
   const KetGroup gr = k.grp[g];
   const int n = gr.rows, ns = gr.steps;
   const double* const pt = k.pt + 4 * ((size_t)gr.line + min(ii, n - 1)) + kk;
-  const double* const pj = k.proj + (size_t)kk * k.L + col;
+  const double* const pj = k.proj + (size_t)kk * k.L + lc;
   int p[ADD ? 4 : 1];                         // ADD: mesh rows 4r+kk of the group
   if constexpr (ADD) {
 #pragma unroll
@@ -353,7 +354,7 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
     if constexpr (ADD) {
       if (q0 == 0)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) old[r] = ldv<TW>(k.out + (size_t)p[r] * k.L + col);
+        for (int r = 0; r < 4; ++r) old[r] = ldv<TW>(k.out + (size_t)p[r] * k.L + lc);
     }
 #pragma unroll
     for (int u = 0; u < KET_AHEAD; ++u) {
@@ -378,7 +379,7 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    if (4 * r + kk < n) {
+    if (4 * r + kk < n && col < k.L) {
       Vec<TW> o;
 #pragma unroll
       for (int w = 0; w < TW; ++w) o.v[w] = ADD ? old[ADD ? r : 0].v[w] + acc[w][r] : acc[w][r];
@@ -394,7 +395,7 @@ __device__ __forceinline__ void ket_mfma(const KetArgs& k, int b) {
   else ket_mfma_body<1, PHASE, ADD>(k, b / nlt, b % nlt);
 }
 
-// plain form, any row length: a wave per group, one thread per (row, lane)
+// plain form (MFMA switched off): a wave per group, one thread per (row, lane)
 __device__ __forceinline__ void ket_plain_body(const KetArgs& k, int b) {
   static_assert(KET_GROUPS == BLOCK / 64, "a group per wave");
   const int g = b * KET_GROUPS + (threadIdx.x >> 6);
@@ -435,7 +436,6 @@ __global__ __launch_bounds__(BLOCK) void k_ket_plain(const KetArgs k) { ket_plai
 int launch_ket(const KetArgs& k, bool mfma, hipStream_t s) {
   const int nblock = ket_blocks(k.ngrp);
   if (nblock <= 0) return OCTHIP_SUCCESS;
-  mfma = mfma && k.L >= 16;
   ProfScope prof("k_ket", s);
   const dim3 tiles(nblock * mfma_lane_tiles(k.L));  // 32-lane tiles when the row length allows, else 16
   if (k.out && (!mfma || k.phase)) return fail(OCTHIP_ERR_STATE, "ket: no form that adds to the output rows");

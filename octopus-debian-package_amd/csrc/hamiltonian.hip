@@ -142,10 +142,13 @@ int run_bra(octhip_hamiltonian_s* h, const double* f, int L, hipStream_t s, doub
 // a launch), and the march reads no ket rows.  The sums keep their order: results are
 // bit-identical.  With the bra and the ket in front of the march, and with it: 57,777 points,
 // 8 complex states 24.8 -> 20.2 us; 13 real ones on 79,501 points 23.5 -> 19.7; 462,781 points,
-// 2 x 32 states 410 -> 380; exponential midpoint, 155,331 points, 48 states 755 -> 689.
+// 2 x 32 states 410 -> 380; exponential midpoint, 155,331 points, 48 states 755 -> 689; 8 lanes
+// (a bra block per workgroup) 9,843 points 18.0 -> 14.4, 462,781 points 34 -> 30.  Sums of the
+// parts by the block that stores the last one instead of a launch of 5 us: 20 -> 44 and 380 ->
+// 644 us, every block's release to the other XCDs writes back its L2.
 int apply_store(octhip_hamiltonian_s* h, ApplyArgs& a, hipStream_t s, double* zero_bc = nullptr) {
   const int L = a.L;
-  if (a.kslot && h->use_mfma && L >= 16 && bra_by_sets(h) && !h->has_kpoint &&
+  if (a.kslot && h->use_mfma && bra_by_sets(h) && !h->has_kpoint &&
       operator_takes_bra(h->kin, a, bra_mfma_lds(h, L))) {
     BraMfmaArgs m;
     bra_args(h, a.fi, L, zero_bc, m);

@@ -369,7 +369,7 @@ int zmarch_sched(octhip_nl_operator_s::ZPlan* pl, int nchunk, const int4** out, 
 }
 
 int launch_zmarch(const ZArgs& z, int lc, int lpt, int epi, int grid, hipStream_t s);
-int launch_zmarch_bra(const ZArgs& z, const BraMfmaArgs& m, int nz, hipStream_t s);
+int launch_zmarch_bra(const ZArgs& z, const BraMfmaArgs& m, int lc, int nz, hipStream_t s);
 
 // The z-march addresses rows with 32-bit byte offsets: every row array it touches (psi
 // over np_part rows, the outputs over np, the ket rows) must satisfy
@@ -424,11 +424,11 @@ int apply_lane_chunks(const octhip_nl_operator_s* op, const ApplyArgs& a) {
 }
 
 // Whether the pass of `a` (EPI_STORE) can take along a bra by sets whose blocks need lds bytes
-// each: it goes by the z-march in the shape of k_zmarch_bra, whose windows hold two such blocks.
+// each: it goes by the z-march in a shape of k_zmarch_bra, whose windows hold its bra blocks.
 bool operator_takes_bra(const octhip_nl_operator_s* op, const ApplyArgs& a, size_t lds) {
   int lc, lpt;
   zmarch_shape(op, a.L, &lc, &lpt);
-  return op->zmarch_ok && op->kernel != 1 && a.n == 25 && zmarch_fits(op, a) && lc == 16 && lpt == 2 &&
+  return op->zmarch_ok && op->kernel != 1 && a.n == 25 && zmarch_fits(op, a) && (lc == 16 || lc == 8) && lpt == 2 &&
          lds <= sizeof(double) * ZB_RED;
 }
 
@@ -461,7 +461,7 @@ int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t
   z.a.nt = zmarch_nt(op, a);
   z.rec = op->d_rec;
   z.sched = sched;
-  if (bra) return launch_zmarch_bra(z, *bra, len, s);
+  if (bra) return launch_zmarch_bra(z, *bra, lc, len, s);
   // the phased store takes the plan of the plain one: it adds 16 bytes per row
   return launch_zmarch(z, lc, lpt, a.out_phase ? EPI_PHASE : epi, len, s);
 }

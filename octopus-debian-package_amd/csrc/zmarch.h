@@ -430,13 +430,18 @@ __global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_multi(const ZArgs*
   zmarch_body<LPT, LC, EPI, NL>(zs[sc.w], sc.x, sc.y, sc.z);
 }
 
+// dynamic LDS bytes of k_zmarch for a lane chunk: two plane windows
+constexpr size_t zmarch_shmem(int lc) { return sizeof(double) * 2 * ZS * lc; }
+
 // The stencil pass without ket rows and the bra of the same input in one launch: blocks
-// 0 .. nz-1 march, the next ones hold two bra blocks each, the rest clear boundary rows
-// (BraMfmaArgs::zf).  The ket then adds its rows to the output.
-constexpr size_t ZB_RED = (size_t)ZS * 16;  // LDS doubles of one of the two bra blocks
+// 0 .. nz-1 march, the next ones hold one bra block per BLOCK threads (two at 16 lanes a chunk,
+// one at 8), the rest clear boundary rows (BraMfmaArgs::zf).  The ket then adds its rows to the
+// output.
+constexpr size_t ZB_RED = (size_t)ZS * 16;  // LDS doubles of a bra block
 template <int LPT, int LC>
 __global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_bra(const ZArgs za, const BraMfmaArgs m, const int nz) {
-  static_assert(ZNC * LC / LPT == 2 * BLOCK, "two bra blocks of BLOCK threads");
+  constexpr int NT = ZNC * LC / LPT, PER = NT / BLOCK;  // threads and bra blocks of a workgroup
+  static_assert(NT % BLOCK == 0 && PER * ZB_RED * sizeof(double) == zmarch_shmem(LC), "whole bra blocks, their LDS");
   extern __shared__ double2 zsh2[];
   int b = blockIdx.x;
   if (b < nz) {
@@ -446,24 +451,21 @@ __global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_bra(const ZArgs za
     return;
   }
   b -= nz;
-  const int nb = (m.nbra + 1) >> 1;
+  const int nb = (m.nbra + PER - 1) / PER;
   if (b < nb) {
     const int half = __builtin_amdgcn_readfirstlane(threadIdx.x / BLOCK);
-    const int v = 2 * b + half, vb = min(v, m.nbra - 1), nlt = mfma_lane_tiles(m.b.L);
+    const int v = PER * b + half, vb = min(v, m.nbra - 1), nlt = mfma_lane_tiles(m.b.L);
     double* const red = reinterpret_cast<double*>(zsh2) + half * ZB_RED;
     if ((m.b.L & 31) == 0) bra_set_body<2, false>(m, vb / nlt, vb % nlt, red, threadIdx.x % BLOCK, v == vb);
     else bra_set_body<1, false>(m, vb / nlt, vb % nlt, red, threadIdx.x % BLOCK, v == vb);
     return;
   }
   b -= nb;
-  const size_t stride = (size_t)(gridDim.x - nz - nb) * (2 * BLOCK);
-  for (size_t t = b * (size_t)(2 * BLOCK) + threadIdx.x; t < m.zcount; t += stride) m.zf[m.zfirst + t] = 0.0;
+  const size_t stride = (size_t)(gridDim.x - nz - nb) * NT;
+  for (size_t t = b * (size_t)NT + threadIdx.x; t < m.zcount; t += stride) m.zf[m.zfirst + t] = 0.0;
 }
 
 // longest segment a launch accepts for a lane chunk
 constexpr int zmarch_max_seg(int lc) { return lc >= 32 ? 60 : 64; }
-
-// dynamic LDS bytes of k_zmarch for a lane chunk: two plane windows
-constexpr size_t zmarch_shmem(int lc) { return sizeof(double) * 2 * ZS * lc; }
 
 }  // namespace octhip

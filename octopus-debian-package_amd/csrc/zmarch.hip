@@ -150,15 +150,20 @@ int launch_zmarch_multi(const ZArgs* zs, const int4* sched, int len, int lc, int
   return fail(OCTHIP_ERR_INVALID, "no multi z-march instance for lane chunk %d, %d lanes per thread", lc, lpt);
 }
 
-// k_zmarch_bra: 16 lanes a chunk, 2 a thread (nz blocks march)
-int launch_zmarch_bra(const ZArgs& z, const BraMfmaArgs& m, int nz, hipStream_t s) {
+// k_zmarch_bra: chunks of 16 or 8 lanes, 2 a thread (nz blocks march)
+template <int LC>
+int launch_bra_lc(const ZArgs& z, const BraMfmaArgs& m, int nz, hipStream_t s) {
+  constexpr int NT = ZNC * LC / 2, PER = NT / BLOCK;
   ProfScope prof("k_zmarch", s);
-  const int zero = m.zf ? (int)std::min<size_t>((m.zcount + 2 * BLOCK - 1) / (2 * BLOCK), 1024) : 0;
-  const dim3 grid(nz + (m.nbra + 1) / 2 + zero), block(2 * BLOCK);
-  hipLaunchKernelGGL((k_zmarch_bra<2, 16>), grid, block, zmarch_shmem(16), s, z, m, nz);
+  const int zero = m.zf ? (int)std::min<size_t>((m.zcount + NT - 1) / NT, 1024) : 0;
+  hipLaunchKernelGGL((k_zmarch_bra<2, LC>), dim3(nz + (m.nbra + PER - 1) / PER + zero), dim3(NT), zmarch_shmem(LC), s,
+                     z, m, nz);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(OCTHIP_ERR_HIP, "k_zmarch_bra launch: %s", hipGetErrorString(e));
   return OCTHIP_SUCCESS;
+}
+int launch_zmarch_bra(const ZArgs& z, const BraMfmaArgs& m, int lc, int nz, hipStream_t s) {
+  return lc == 16 ? launch_bra_lc<16>(z, m, nz, s) : launch_bra_lc<8>(z, m, nz, s);
 }
 
 int launch_zmarch(const ZArgs& z, int lc, int lpt, int epi, int grid, hipStream_t s) {

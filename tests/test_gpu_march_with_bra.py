@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("set_bc", [False, True])
-@pytest.mark.parametrize("lanes", [16, 32, 64])
+@pytest.mark.parametrize("lanes", [8, 16, 32, 64])
 @pytest.mark.parametrize("name", list(LAYOUTS))
 def test_apply_matches_general_path(gpu, name, lanes, set_bc):
     print(f"[march with bra {name} lanes={lanes} set_bc={set_bc}]", flush=True)

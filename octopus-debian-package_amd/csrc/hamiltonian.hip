@@ -93,7 +93,8 @@ void bra_args(const octhip_hamiltonian_s* h, const double* f, int L, double* zer
 }
 
 // projections from the parts of the bra, and their ket rows into h->d_ksum, or added to out
-int run_ket(octhip_hamiltonian_s* h, int L, int pjmax, bool sets, hipStream_t s, double* out = nullptr) {
+int run_ket(octhip_hamiltonian_s* h, int L, int pjmax, bool sets, hipStream_t s, double* out = nullptr,
+            const double* out_phase = nullptr) {
   BraReduceArgs r;
   r.partial = h->d_partial;
   r.row = h->d_prow;
@@ -109,6 +110,7 @@ int run_ket(octhip_hamiltonian_s* h, int L, int pjmax, bool sets, hipStream_t s,
   ket_args(h, L, h->d_proj, h->d_ksum, k);
   k.out = out;
   k.point = h->d_kpoint;
+  k.out_phase = out_phase;
   return launch_ket(k, h->use_mfma, s);
 }
 
@@ -145,19 +147,21 @@ int run_bra(octhip_hamiltonian_s* h, const double* f, int L, hipStream_t s, doub
 // 2 x 32 states 410 -> 380; exponential midpoint, 155,331 points, 48 states 755 -> 689; 8 lanes
 // (a bra block per workgroup) 9,843 points 18.0 -> 14.4, 462,781 points 34 -> 30.  Sums of the
 // parts by the block that stores the last one instead of a launch of 5 us: 20 -> 44 and 380 ->
-// 644 us, every block's release to the other XCDs writes back its L2.
+// 644 us, every block's release to the other XCDs writes back its L2.  With Bloch phases the march
+// leaves the rows of the ket without the conjugate phase, which the ket multiplies after its sum:
+// 40^3 cell, 16 states 35.9 -> 32.1 us; 32^3 cell, 4 states 24 -> 21.
 int apply_store(octhip_hamiltonian_s* h, ApplyArgs& a, hipStream_t s, double* zero_bc = nullptr) {
   const int L = a.L;
-  if (a.kslot && h->use_mfma && bra_by_sets(h) && !h->has_kpoint &&
+  if (a.kslot && h->use_mfma && bra_by_sets(h) &&
       operator_takes_bra(h->kin, a, bra_mfma_lds(h, L))) {
     BraMfmaArgs m;
     bra_args(h, a.fi, L, zero_bc, m);
-    a.kslot = nullptr;
+    if (!a.out_phase) a.kslot = nullptr;  // else: the rows that the ket multiplies by the phase
     a.ksum = nullptr;
     a.nk = 0;
     int rc = launch_operator(h->kin, a, EPI_STORE, s, &m);
     if (rc) return rc;
-    return run_ket(h, L, m.b.pjmax, true, s, a.fo);
+    return run_ket(h, L, m.b.pjmax, true, s, a.fo, a.out_phase);
   }
   int rc = OCTHIP_SUCCESS;
   if (a.kslot) rc = run_bra(h, a.fi, L, s, zero_bc);
@@ -344,10 +348,6 @@ int periodic_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, 
       if (rc) return rc;
     }
   }
-  if ((terms & OCTHIP_TERM_NON_LOCAL_POTENTIAL) && h->nmat > 0) {
-    rc = run_bra(h, src, L, s, nullptr);
-    if (rc) return rc;
-  }
   ApplyArgs a;
   std::memset(&a, 0, sizeof(a));
   fill_terms(h, terms, a);
@@ -356,7 +356,7 @@ int periodic_apply(octhip_hamiltonian_s* h, double* psi, double* hpsi, int ldf, 
   a.L = L;
   a.lim = np_part;  // boundary rows as set above (or by the caller)
   a.out_phase = set_phase ? h->d_phase : nullptr;
-  return launch_operator(h->kin, a, EPI_STORE, s);
+  return apply_store(h, a, s);
 }
 
 // Ket tables of a handle (KetArgs, BraReduceArgs::row).

@@ -381,8 +381,10 @@ struct KetArgs {
   // hamiltonian_elec_base_inc.F90:955-966); null: none
   const double* __restrict__ phase = nullptr;
   // with out: the rows are added to the mesh rows `point` of out instead (kbuf unused)
+  // (and times the conjugate of out_phase, the Bloch phases of mesh rows, when given)
   double* out = nullptr;
   const int* __restrict__ point = nullptr;
+  const double* __restrict__ out_phase = nullptr;
 };
 
 // Bra by sets: the same groups as the ket's, so the row of a mesh point inside several

@@ -377,6 +377,24 @@ __device__ __forceinline__ void ket_mfma_body(const KetArgs& k, int b, int lt) {
 #pragma unroll
     for (int w = 0; w < TW; ++w) acc[w] = tot[w];
   }
+  if constexpr (ADD && PHASE) {
+    if (k.out_phase) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double pr = k.out_phase[2 * (size_t)p[r]], pi = -k.out_phase[2 * (size_t)p[r] + 1];
+        const double x0 = old[r].v[0] + acc[0][r];
+        old[r].v[0] = 0.0;
+        if constexpr (TW == 2) {
+          const double x1 = old[r].v[1] + acc[1][r];
+          old[r].v[1] = 0.0;
+          acc[0][r] = zmul_lane(pr, pi, x0, x1, false);
+          acc[1][r] = zmul_lane(pr, pi, x1, x0, true);
+        } else {
+          acc[0][r] = zmul_lane(pr, pi, x0, __shfl_xor(x0, 1), (col & 1) != 0);
+        }
+      }
+    }
+  }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     if (4 * r + kk < n && col < k.L) {
@@ -438,8 +456,10 @@ int launch_ket(const KetArgs& k, bool mfma, hipStream_t s) {
   if (nblock <= 0) return OCTHIP_SUCCESS;
   ProfScope prof("k_ket", s);
   const dim3 tiles(nblock * mfma_lane_tiles(k.L));  // 32-lane tiles when the row length allows, else 16
-  if (k.out && (!mfma || k.phase)) return fail(OCTHIP_ERR_STATE, "ket: no form that adds to the output rows");
-  if (k.out)
+  if (k.out && !mfma) return fail(OCTHIP_ERR_STATE, "ket: no form that adds to the output rows");
+  if (k.out && k.phase)
+    hipLaunchKernelGGL((k_ket_mfma<true, true>), tiles, dim3(BLOCK), 0, s, k);
+  else if (k.out)
     hipLaunchKernelGGL((k_ket_mfma<false, true>), tiles, dim3(BLOCK), 0, s, k);
   else if (mfma && k.phase)
     hipLaunchKernelGGL((k_ket_mfma<true, false>), tiles, dim3(BLOCK), 0, s, k);

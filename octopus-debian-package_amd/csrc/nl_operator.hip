@@ -435,7 +435,7 @@ bool operator_takes_bra(const octhip_nl_operator_s* op, const ApplyArgs& a, size
 // Apply through the best kernel for this operator: z-march for the order-4 star on a
 // lattice, the tiled gather otherwise.
 int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t s, const BraMfmaArgs* bra = nullptr) {
-  if (!a.fi || !a.zrow || (a.kslot && !a.ksum) || (epi == EPI_STORE && !a.fo))
+  if (!a.fi || !a.zrow || (a.kslot && !a.ksum && !bra) || (epi == EPI_STORE && !a.fo))
     return fail(OCTHIP_ERR_STATE, "apply: incomplete kernel arguments");
   const bool zm = op->zmarch_ok && op->kernel != 1 && a.n == 25 && zmarch_fits(op, a);
   if (!zm) {
@@ -445,7 +445,7 @@ int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t
   }
   int lc, lpt;
   zmarch_shape(op, a.L, &lc, &lpt);
-  const int zs = zmarch_zseg_for(op, a.L, epi, a.kslot != nullptr);
+  const int zs = zmarch_zseg_for(op, a.L, epi, a.kslot != nullptr && !bra);
   if (zs > zmarch_max_seg(lc))
     return fail(OCTHIP_ERR_INVALID, "z-march: lane chunk %d with z segment %d needs more than 160 KB of LDS", lc, zs);
   octhip_nl_operator_s::ZPlan* pl = nullptr;

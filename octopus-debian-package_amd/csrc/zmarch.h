@@ -144,7 +144,9 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
   const uint32_t np_bytes = (uint32_t)a_np << sh;
   const auto r_fi = zrsrc(A.fi, (uint32_t)A.lim << sh);
   const auto r_v = zrsrc(a_v, a_v ? (uint32_t)a_np * 8u : 0u);
-  const auto r_ks = zrsrc(A.kslot, NL ? (uint32_t)a_np * 4u : 0u);
+  // EPI_PHASE without ket rows: rows that a ket is added to later are stored without the phase
+  constexpr bool KS = NL || EPI == EPI_PHASE;
+  const auto r_ks = zrsrc(A.kslot, KS && A.kslot ? (uint32_t)a_np * 4u : 0u);
   const auto r_k = zrsrc(A.ksum, NL ? (uint32_t)A.nk << sh : 0u);
   const auto r_ai = zrsrc(A.acc_in ? A.acc_in : a_acc, has_acc ? np_bytes : 0u);
   const auto r_fo = zrsrc(A.fo, TAY ? 0u : np_bytes);
@@ -295,6 +297,7 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
           } else {
             o.v[0] = zmul_lane(pr, pi, s.v[0], __shfl_xor(s.v[0], 1), (l & 1) != 0);
           }
+          if (!NL && ks[kk & 3] != 0u) o = s;
           bst<LPT>(r_fo, qo, o, a_nt);
         } else {
           bst<LPT>(r_y, qo, s, a_nt);  // dropped when there is no yout
@@ -344,7 +347,7 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
       // ---- loads, into the registers that the plane staged and the plane completed have left;
       // the ones consumed first in the next step first
       const uint32_t kslot = ks[(kk + AD) & 3];  // of plane z - 4 + AD, loaded two steps ago
-      if constexpr (NL) {
+      if constexpr (KS) {
         const int P = z - 2 + AD;
         const uint32_t qp = (P >= 0 && P < n) ? poff(ro[(kk + 6 + AD) & 7], 2) : NONE;
         ks[(kk + 2 + AD) & 3] = __builtin_amdgcn_raw_buffer_load_b32(r_ks, qp, 0, 0);
@@ -438,7 +441,9 @@ constexpr size_t zmarch_shmem(int lc) { return sizeof(double) * 2 * ZS * lc; }
 // one at 8), the rest clear boundary rows (BraMfmaArgs::zf).  The ket then adds its rows to the
 // output.
 constexpr size_t ZB_RED = (size_t)ZS * 16;  // LDS doubles of a bra block
-template <int LPT, int LC>
+// EPI: EPI_STORE, or EPI_PHASE with the rows of a later ket left without the phase; PHASE: the
+// bra takes the states times the Bloch phases of (point, matrix).
+template <int LPT, int LC, int EPI, bool PHASE>
 __global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_bra(const ZArgs za, const BraMfmaArgs m, const int nz) {
   constexpr int NT = ZNC * LC / LPT, PER = NT / BLOCK;  // threads and bra blocks of a workgroup
   static_assert(NT % BLOCK == 0 && PER * ZB_RED * sizeof(double) == zmarch_shmem(LC), "whole bra blocks, their LDS");
@@ -447,7 +452,7 @@ __global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_bra(const ZArgs za
   if (b < nz) {
     const int4 sc = za.sched[b];
     if (sc.y <= 0) return;
-    zmarch_body<LPT, LC, EPI_STORE, false>(za, sc.x, sc.y, sc.z);
+    zmarch_body<LPT, LC, EPI, false>(za, sc.x, sc.y, sc.z);
     return;
   }
   b -= nz;
@@ -456,8 +461,8 @@ __global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_bra(const ZArgs za
     const int half = __builtin_amdgcn_readfirstlane(threadIdx.x / BLOCK);
     const int v = PER * b + half, vb = min(v, m.nbra - 1), nlt = mfma_lane_tiles(m.b.L);
     double* const red = reinterpret_cast<double*>(zsh2) + half * ZB_RED;
-    if ((m.b.L & 31) == 0) bra_set_body<2, false>(m, vb / nlt, vb % nlt, red, threadIdx.x % BLOCK, v == vb);
-    else bra_set_body<1, false>(m, vb / nlt, vb % nlt, red, threadIdx.x % BLOCK, v == vb);
+    if ((m.b.L & 31) == 0) bra_set_body<2, PHASE>(m, vb / nlt, vb % nlt, red, threadIdx.x % BLOCK, v == vb);
+    else bra_set_body<1, PHASE>(m, vb / nlt, vb % nlt, red, threadIdx.x % BLOCK, v == vb);
     return;
   }
   b -= nb;

@@ -156,8 +156,13 @@ int launch_bra_lc(const ZArgs& z, const BraMfmaArgs& m, int nz, hipStream_t s) {
   constexpr int NT = ZNC * LC / 2, PER = NT / BLOCK;
   ProfScope prof("k_zmarch", s);
   const int zero = m.zf ? (int)std::min<size_t>((m.zcount + NT - 1) / NT, 1024) : 0;
-  hipLaunchKernelGGL((k_zmarch_bra<2, LC>), dim3(nz + (m.nbra + PER - 1) / PER + zero), dim3(NT), zmarch_shmem(LC), s,
-                     z, m, nz);
+  const dim3 grid(nz + (m.nbra + PER - 1) / PER + zero);
+  if (z.a.out_phase)
+    hipLaunchKernelGGL((k_zmarch_bra<2, LC, EPI_PHASE, true>), grid, dim3(NT), zmarch_shmem(LC), s, z, m, nz);
+  else if (m.set.phase)
+    hipLaunchKernelGGL((k_zmarch_bra<2, LC, EPI_STORE, true>), grid, dim3(NT), zmarch_shmem(LC), s, z, m, nz);
+  else
+    hipLaunchKernelGGL((k_zmarch_bra<2, LC, EPI_STORE, false>), grid, dim3(NT), zmarch_shmem(LC), s, z, m, nz);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(OCTHIP_ERR_HIP, "k_zmarch_bra launch: %s", hipGetErrorString(e));
   return OCTHIP_SUCCESS;

@@ -9,7 +9,7 @@ order-4 star stencil, 64 states in two packed batches of 32, 16 Gaussian wells,
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload hamiltonian|laplacian|taylor|adjoint|batched]
 
 Prints one JSON line.  `value` is state-points/s with the states already resident in
-HBM; `roofline` is the dominant kernel (k_zmarch, the fused stencil + local + ket pass)
+HBM; `roofline` is the dominant kernel (k_zmarch, the fused stencil + local pass with the projector bra)
 timed with HIP events on its launch stream over the timed region; `cpu_baseline` is the
 CPU oracle (C/OpenMP restatement of the reference CPU path) on a bounded sample.
 """

@@ -27,6 +27,7 @@ std::vector<int2> zmarch_items(const octhip_nl_operator_s* op, int zs);
 extern const int ZM_SEGS[7];
 double zmarch_makespan(const std::vector<int>& planes, int lc, int resident);
 int zmarch_nt(const octhip_nl_operator_s* op, const ApplyArgs& a);
+int zmarch_ntl(const octhip_nl_operator_s* op, const ApplyArgs& a);
 int zmarch_resident(int lc, int lpt, int epi, bool nl, bool multi);
 bool zmarch_fits(const octhip_nl_operator_s* op, const ApplyArgs& a);
 int launch_zmarch_multi(const ZArgs* zs, const int4* sched, int len, int lc, int lpt, int epi, bool nl,
@@ -166,6 +167,7 @@ int build_zdesc(octhip_batched_s* b, int k, ZArgs** out) {
     h_apply_args(p.h, in, p.L, p.ksum, z.a);
     z.a.reuse = k > 0;
     z.a.nt = zmarch_nt(op, z.a);
+    z.a.ntl = zmarch_ntl(op, z.a);
     const bool deferred = taylor_deferred(b->order);
     if (k == 0) {
       z.a.fo = p.hpsi;

@@ -70,6 +70,7 @@ struct ApplyArgs {
   const double* __restrict__ out_phase;  // EPI_STORE, complex rows: Bloch phases (np pairs) or null
   int reuse;                       // the output rows are read again by the next pass
   int nt;                          // z-march: non-temporal stores of the output rows
+  int ntl;                         // z-march: non-temporal loads of acc_in, ya, yb
 };
 
 __device__ __forceinline__ int tile_of(int b, int chunk) {

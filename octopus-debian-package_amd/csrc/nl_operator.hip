@@ -391,6 +391,16 @@ int zmarch_nt(const octhip_nl_operator_s* op, const ApplyArgs& a) {
   return a.reuse && (double)op->np * a.L * sizeof(double) <= ZM_CACHED_BYTES ? 0 : 1;
 }
 
+// Whether a Taylor pass loads its accumulator and the earlier powers non-temporally: it is the
+// last reader of the powers, and where its four row arrays exceed the 256 MB Infinity Cache they
+// come from memory anyhow and only push out the halo rows.  Non-temporal against cached, whole
+// steps: rows of 20 MB (79,501 points, 16 states) 140 / 136 us; 80 MB (155,331 points, 32-state
+// blocks) 682 / 694, order 6 1180 / 1201; 237 MB (462,781 points, 4 x 32 states) 3242 / 3322.
+constexpr double ZM_TAYLOR_CACHED_BYTES = 64e6;
+int zmarch_ntl(const octhip_nl_operator_s* op, const ApplyArgs& a) {
+  return (double)op->np * a.L * sizeof(double) > ZM_TAYLOR_CACHED_BYTES;
+}
+
 // Build every lazily created device structure an apply with rows of L doubles needs (both
 // epilogues; nl = with ket rows), so that later applies allocate nothing (required before
 // a graph capture).
@@ -459,6 +469,7 @@ int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t
   ZArgs z;
   z.a = a;
   z.a.nt = zmarch_nt(op, a);
+  z.a.ntl = zmarch_ntl(op, a);
   z.rec = op->d_rec;
   z.sched = sched;
   if (bra) return launch_zmarch_bra(z, *bra, lc, len, s);

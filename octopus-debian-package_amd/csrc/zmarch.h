@@ -19,7 +19,7 @@
 //   * loads run ahead (depths in ZDepth) in rings with compile-time slots (the z loop is
 //     unrolled by 8); every load but the ket rows is unconditional, so the compiler's wait
 //     counts stay exact and a step waits only on loads of the steps before it.
-// What bounds it (462,781 points, 32 complex states, H-apply with projectors: 163 us, 518 MB
+// What bounds it (462,781 points, 32 complex states, H-apply with ket rows: 163 us, 518 MB
 // read and 237 MB written for 289 + 237 MB of rows): 102 us go to the LDS reads (16 rows of 16
 // bytes per output) and the vector memory instructions alone, with every row out of range, and
 // the memory traffic overlaps with them only in part.  Measured and not kept: rows two or three
@@ -68,15 +68,16 @@ constexpr int ZM_RSRC_DW3 = 0x00020000;  // dword 3 of a raw buffer resource: 32
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t zrsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, ZM_RSRC_DW3);
 }
-template <int LPT>
+constexpr int ZM_NT = 2;  // cache-policy operand: non-temporal
+template <int LPT, int POLICY = 0>
 __device__ __forceinline__ Vec<LPT> bld(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   Vec<LPT> v;
   if constexpr (LPT == 2) {
-    const double2 t = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    const double2 t = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, POLICY));
     v.v[0] = t.x;
     v.v[1] = t.y;
   } else {
-    v.v[0] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    v.v[0] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, POLICY));
   }
   return v;
 }
@@ -84,18 +85,17 @@ __device__ __forceinline__ Vec<LPT> bld(__amdgpu_buffer_rsrc_t r, uint32_t off) 
 // finds in the 256 MB Infinity Cache are stored cached; beyond that, non-temporal stores leave
 // the XCD's L2 to the input rows that the neighbouring tiles read as their halo (see
 // zmarch_nt in nl_operator.hip for the line between them).
-constexpr int ZM_STORE_NT = 2;  // cache-policy operand: NT
 template <int LPT>
 __device__ __forceinline__ void bst(__amdgpu_buffer_rsrc_t r, uint32_t off, const Vec<LPT>& v, bool nt) {
   if constexpr (LPT == 2) {
     using U4 = decltype(__builtin_amdgcn_raw_buffer_load_b128(r, 0, 0, 0));
     const U4 u = __builtin_bit_cast(U4, make_double2(v.v[0], v.v[1]));
-    if (nt) __builtin_amdgcn_raw_buffer_store_b128(u, r, off, 0, ZM_STORE_NT);
+    if (nt) __builtin_amdgcn_raw_buffer_store_b128(u, r, off, 0, ZM_NT);
     else __builtin_amdgcn_raw_buffer_store_b128(u, r, off, 0, 0);
   } else {
     using U2 = decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0));
     const U2 u = __builtin_bit_cast(U2, v.v[0]);
-    if (nt) __builtin_amdgcn_raw_buffer_store_b64(u, r, off, 0, ZM_STORE_NT);
+    if (nt) __builtin_amdgcn_raw_buffer_store_b64(u, r, off, 0, ZM_NT);
     else __builtin_amdgcn_raw_buffer_store_b64(u, r, off, 0, 0);
   }
 }
@@ -129,7 +129,7 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
   const int a_np = A.np;
   const double* const a_v = A.v;
   double* const a_acc = A.acc;
-  const bool a_nt = A.nt != 0;
+  const bool a_nt = A.nt != 0, a_ntl = A.ntl != 0;
   double a_w[25];
 #pragma unroll
   for (int j = 0; j < 25; ++j) a_w[j] = A.w[j];
@@ -376,9 +376,16 @@ __device__ __forceinline__ void zmarch_body(const ZArgs& za, const int rec0, con
           kr[(kk + AD) & M] = kv;
         }
         if constexpr (TAY) {
-          ar[(kk + AD) & M] = bld<LPT>(r_ai, qa);
-          ra[(kk + AD) & M] = bld<LPT>(r_ya, qa);  // zeros (no memory access) without ya / yb
-          rb[(kk + AD) & M] = bld<LPT>(r_yb, qa);
+          // zeros (no memory access) without ya / yb; as many loads on either side
+          if (a_ntl) {
+            ar[(kk + AD) & M] = bld<LPT, ZM_NT>(r_ai, qa);
+            ra[(kk + AD) & M] = bld<LPT, ZM_NT>(r_ya, qa);
+            rb[(kk + AD) & M] = bld<LPT, ZM_NT>(r_yb, qa);
+          } else {
+            ar[(kk + AD) & M] = bld<LPT>(r_ai, qa);
+            ra[(kk + AD) & M] = bld<LPT>(r_ya, qa);
+            rb[(kk + AD) & M] = bld<LPT>(r_yb, qa);
+          }
         }
       }
       {

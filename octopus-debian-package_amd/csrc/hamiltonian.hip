@@ -50,6 +50,7 @@ int ensure_work(octhip_hamiltonian_s* h, int ldf, hipStream_t s) {
     for (void* p : {(void*)w.partial, (void*)w.proj, (void*)w.ksum})
       if (p) h->retired.push_back(p);
     w.partial = w.proj = w.ksum = nullptr;
+    w.work_ldf = -1;  // until all three are there: after a failure shorter rows get new ones too
     const size_t L = (size_t)1 << ldf;
     int rc = OCTHIP_SUCCESS;
     if (h->nmat > 0) {
@@ -71,6 +72,7 @@ int ensure_taylor(octhip_hamiltonian_s* h, int ldf, hipStream_t s) {
     for (void* p : {(void*)w.y0, (void*)w.y1, (void*)w.y2})
       if (p) h->retired.push_back(p);
     w.y0 = w.y1 = w.y2 = nullptr;
+    w.y_ldf = -1;
     const size_t bytes = sizeof(double) * ((size_t)h->np << ldf);
     int rc = dalloc((void**)&w.y0, bytes);
     if (!rc) rc = dalloc((void**)&w.y1, bytes);

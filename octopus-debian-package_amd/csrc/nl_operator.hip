@@ -473,8 +473,12 @@ int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t
   z.rec = op->d_rec;
   z.sched = sched;
   if (bra) return launch_zmarch_bra(z, *bra, lc, len, s);
-  // the phased store takes the plan of the plain one: it adds 16 bytes per row
-  return launch_zmarch(z, lc, lpt, a.out_phase ? EPI_PHASE : epi, len, s);
+  // The phased store takes the plan of the plain one: it adds 16 bytes per row.  A chunk of one
+  // lane (tuning only) holds no (re, im) pair: its rows get the phase in a pass of their own.
+  const bool phased = a.out_phase && lc >= 2;
+  rc = launch_zmarch(z, lc, lpt, phased ? EPI_PHASE : epi, len, s);
+  if (rc || phased || !a.out_phase) return rc;
+  return launch_phase(a.fo, a.fo, a.out_phase, a.np, a.L, true, s);
 }
 }  // namespace octhip
 

@@ -293,13 +293,14 @@ int zmarch_zseg_for(const octhip_nl_operator_s* op, int L, int epi, bool nl) {
   return zmarch_zseg(op, L / lc, lc, zmarch_resident(lc, lpt, epi, nl, false));
 }
 
-// Index records of every tile (layout in zmarch.h), built once per operator.
+// Index records of every tile (layout in zmarch.h), built once per operator.  The march cube has at
+// most 2^30 sites and a plane of a tile 64 of them, so a plane's number fits an int; the table may
+// have more than 2^31 ints (addressed by plane, 32-bit offsets within an item).
 int zmarch_records(octhip_nl_operator_s* op) {
   if (op->d_rec) return OCTHIP_SUCCESS;
   size_t planes = 0;
   for (size_t t = 0; t < op->tile_zlo.size(); ++t)
     if (op->tile_zhi[t] >= 0) planes += (size_t)(op->tile_zhi[t] - op->tile_zlo[t] + 9);
-  if (planes * ZPLANE > (size_t)INT_MAX) return fail(OCTHIP_ERR_UNSUPPORTED, "z-march index tables too large");
   std::vector<int> rec(planes * ZPLANE);
   int* r = rec.data();
   for (size_t t = 0; t < op->tile_zlo.size(); ++t) {

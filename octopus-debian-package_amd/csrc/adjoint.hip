@@ -162,7 +162,7 @@ struct octhip_adjoint_s {
   double dt = 0.0, vol = 0.0;
   double pol[3] = {0.0, 0.0, 0.0};
   double* d_xp = nullptr;       // np
-  double* d_slot = nullptr;     // 2 x (K+1) x np x L: psi_s of a segment (recomputed), two sets
+  double* d_slot = nullptr;     // 2 x K x np x L: psi_s of a segment behind its checkpoint, two sets
   double* d_ckpt = nullptr;     // nckpt x np x L: psi at every K-th step
   double* d_seg = nullptr;      // 2 x K x (order-1) x np x L: H^k psi_s, k >= 1, two sets
   double* d_ychi = nullptr;     // 2 x order x np x L: H^m chi_{s+1}, m >= 1 (slot 0 unused), two sets
@@ -211,11 +211,11 @@ int step_field(octhip_adjoint_s* a, int s, hipStream_t st) {
 
 size_t rows_bytes(size_t rows, int L) { return sizeof(double) * rows * (size_t)L; }
 
-// Step i of segment c: psi_s (the segment's checkpoint for i = 0) and, from index 1, the
-// terms H^k psi_s, in buffer set c & 1
+// Step i of segment c: psi_s (the segment's checkpoint for i = 0, up to i = K) and, from index 1,
+// the terms H^k psi_s, in buffer set c & 1
 double* segment_psi(const octhip_adjoint_s* a, int c, int i) {
   const size_t arr = (size_t)a->h->np * a->L;
-  return i == 0 ? a->d_ckpt + (size_t)c * arr : a->d_slot + ((size_t)(c & 1) * (a->K + 1) + i) * arr;
+  return i == 0 ? a->d_ckpt + (size_t)c * arr : a->d_slot + ((size_t)(c & 1) * a->K + i - 1) * arr;
 }
 void segment_terms(const octhip_adjoint_s* a, int c, int i, double** ys) {
   const size_t arr = (size_t)a->h->np * a->L;
@@ -258,7 +258,7 @@ extern "C" int octhip_adjoint_create(octhip_hamiltonian_t h, const double* posit
     xp[p] = pol[0] * positions[3 * (size_t)p] + pol[1] * positions[3 * (size_t)p + 1] +
             pol[2] * positions[3 * (size_t)p + 2];
   if (!rc) rc = upload(&a->d_xp, xp.data(), xp.size(), nullptr);
-  if (!rc) rc = dalloc((void**)&a->d_slot, rows_bytes((size_t)2 * (a->K + 1) * np, a->L));
+  if (!rc) rc = dalloc((void**)&a->d_slot, rows_bytes((size_t)2 * a->K * np, a->L));
   if (!rc) rc = dalloc((void**)&a->d_chi2, rows_bytes((size_t)2 * np, a->L));
   if (!rc) rc = dalloc((void**)&a->d_ckpt, rows_bytes((size_t)a->nckpt * np, a->L));
   if (!rc && order > 1) rc = dalloc((void**)&a->d_seg, rows_bytes((size_t)2 * a->K * (order - 1) * np, a->L));
@@ -405,8 +405,7 @@ int backward_run(octhip_adjoint_s* a, double* chi, double* dj_deps, double* dj_d
       field_of(st, f);
       int rc = launch_veff(a->h, vr, f, s2);
       if (!rc)
-        rc = taylor_step(a->h, a->d_slot + ((size_t)b * (a->K + 1) + i + 1) * arr, a->ldf, a->dt, order, 0, ys, s2,
-                         ys[0], vr);
+        rc = taylor_step(a->h, segment_psi(a, c, i + 1), a->ldf, a->dt, order, 0, ys, s2, ys[0], vr);
       if (rc) return rc;
     }
     OCTHIP_HIP(hipEventRecord(a->ev_rec[b], s2));

@@ -56,7 +56,8 @@ void dfree(void* p);
 // library and given back when the call ends (hipMalloc and hipFree cost about 100 us, and
 // hipFree waits for the device).  The caller synchronises its stream first.  The pool keeps at
 // most SCRATCH_KEEP buffers, of at most SCRATCH_MAX bytes each, until octhip_finalize; it is
-// safe with several threads and streams (a buffer has one user at a time).
+// safe with several threads and streams (a buffer has one user at a time).  The largest need is
+// a Gram-Schmidt pass on rows of 1024 lanes: 16 MiB of partial sums, 8 KiB a vector and 48 KiB.
 class Scratch {
  public:
   Scratch() = default;
@@ -71,7 +72,7 @@ class Scratch {
   size_t bytes_ = 0;
 };
 constexpr int SCRATCH_KEEP = 4;
-constexpr size_t SCRATCH_MAX = (size_t)16 << 20;
+constexpr size_t SCRATCH_MAX = (size_t)24 << 20;
 void scratch_clear();
 
 template <typename T>

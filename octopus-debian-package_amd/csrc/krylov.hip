@@ -78,10 +78,9 @@ int krylov_bufs(octhip_hamiltonian_s* h, hipStream_t s, int nvec, int ldf, Krylo
     int rc = dalloc((void**)&k->small, small_bytes);
     if (rc) return rc;
   }
-  if (!k->host && hipHostMalloc((void**)&k->host, sizeof(double) * K_RES, hipHostMallocDefault) != hipSuccess) {
-    k->host = nullptr;
-    (void)hipGetLastError();
-    return fail(OCTHIP_ERR_ALLOC, "hipHostMalloc(%zu bytes) failed", sizeof(double) * K_RES);
+  if (!k->host) {
+    int rc = halloc((void**)&k->host, sizeof(double) * K_RES);
+    if (rc) return rc;
   }
   if (!k->ready) OCTHIP_HIP(hipEventCreateWithFlags(&k->ready, hipEventDisableTiming));
   out->vec = k->vec;
@@ -234,7 +233,7 @@ void drop_krylov(octhip_hamiltonian_s* h, hipStream_t s, bool all) {
     if (all || h->krylov[i].s == s) {
       dfree(h->krylov[i].vec);
       dfree(h->krylov[i].small);
-      if (h->krylov[i].host) (void)hipHostFree(h->krylov[i].host);
+      hfree(h->krylov[i].host);
       if (h->krylov[i].ready) (void)hipEventDestroy(h->krylov[i].ready);
       h->krylov.erase(h->krylov.begin() + (long)i);
     } else {

@@ -47,10 +47,12 @@ const double* zero_row();
       return ::octhip::fail(OCTHIP_ERR_STATE, "octhip_init has not been called");    \
   } while (0)
 
-// Device allocation and release: every allocation of the library goes through dalloc
-// (RAII-free: every handle frees what it owns in its *_destroy).
+// Device allocation and release: every allocation of the library goes through dalloc, pinned host
+// memory through halloc (RAII-free: every handle frees what it owns in its *_destroy).
 int dalloc(void** p, size_t bytes);
 void dfree(void* p);
+int halloc(void** p, size_t bytes);
+void hfree(void* p);
 
 // A device scratch buffer of a call that has no handle to keep it: taken from a pool of the
 // library and given back when the call ends (hipMalloc and hipFree cost about 100 us, and

@@ -37,23 +37,39 @@ namespace {
 std::atomic<long> g_alloc_budget{-1};
 }  // namespace
 
-int dalloc(void** p, size_t bytes) {
+namespace {
+// p from `alloc` (named in the message), or the failure that the hook asks for
+int guarded(const char* name, hipError_t (*alloc)(void**, size_t), void** p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) return OCTHIP_SUCCESS;
   for (long b = g_alloc_budget.load(); b >= 0; b = g_alloc_budget.load()) {
-    if (b == 0) return fail(OCTHIP_ERR_ALLOC, "hipMalloc(%zu bytes): injected allocation failure", bytes);
+    if (b == 0) return fail(OCTHIP_ERR_ALLOC, "%s(%zu bytes): injected allocation failure", name, bytes);
     if (g_alloc_budget.compare_exchange_weak(b, b - 1)) break;
   }
-  hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = alloc(p, bytes);
   if (e != hipSuccess) {
     *p = nullptr;
-    return fail(OCTHIP_ERR_ALLOC, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
+    return fail(OCTHIP_ERR_ALLOC, "%s(%zu bytes): %s", name, bytes, hipGetErrorString(e));
   }
   return OCTHIP_SUCCESS;
+}
+}  // namespace
+
+int dalloc(void** p, size_t bytes) {
+  return guarded("hipMalloc", [](void** q, size_t n) { return hipMalloc(q, n); }, p, bytes);
 }
 
 void dfree(void* p) {
   if (p) (void)hipFree(p);
+}
+
+int halloc(void** p, size_t bytes) {
+  return guarded("hipHostMalloc", [](void** q, size_t n) { return hipHostMalloc(q, n, hipHostMallocDefault); }, p,
+                 bytes);
+}
+
+void hfree(void* p) {
+  if (p) (void)hipHostFree(p);
 }
 
 namespace {

@@ -457,8 +457,9 @@ int launch_operator(octhip_nl_operator_s* op, ApplyArgs& a, int epi, hipStream_t
   int lc, lpt;
   zmarch_shape(op, a.L, &lc, &lpt);
   const int zs = zmarch_zseg_for(op, a.L, epi, a.kslot != nullptr && !bra);
-  if (zs > zmarch_max_seg(lc))
-    return fail(OCTHIP_ERR_INVALID, "z-march: lane chunk %d with z segment %d needs more than 160 KB of LDS", lc, zs);
+  if (lc == 32 && zs > ZM_SEG32)
+    return fail(OCTHIP_ERR_INVALID, "z-march: lane chunk 32 (128 KB of LDS) takes z segments of at most %d planes, not %d",
+                ZM_SEG32, zs);
   octhip_nl_operator_s::ZPlan* pl = nullptr;
   int rc = zmarch_plan(op, zs, &pl);
   if (rc) return rc;

@@ -477,7 +477,9 @@ __global__ __launch_bounds__(ZNC * LC / LPT, 4) void k_zmarch_bra(const ZArgs za
   for (size_t t = b * (size_t)NT + threadIdx.x; t < m.zcount; t += stride) m.zf[m.zfirst + t] = 0.0;
 }
 
-// longest segment a launch accepts for a lane chunk
-constexpr int zmarch_max_seg(int lc) { return lc >= 32 ? 60 : 64; }
+// Longest segment of a workgroup of 32 lanes.  Its windows take 128 KB of LDS at any segment length,
+// so the kernel itself would run longer ones: the limit is part of the interface, from kernels that
+// staged index tables in LDS, and what callers see refused stays refused.
+constexpr int ZM_SEG32 = 60;
 
 }  // namespace octhip

@@ -115,20 +115,21 @@ extern "C" int octhip_hamiltonian_autotune(octhip_hamiltonian_t h, int ldf, int 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) rc = fail(OCTHIP_ERR_HIP, "autotune fill: %s", hipGetErrorString(e));
   }
-  // candidates of the stencil pass (bra fixed to MFMA where it applies), then the bra.
+  // Candidates of the stencil pass with the MFMA bra and ket, then the plain ones on the fastest.
+  // (Rows below 16 lanes too: 17,077 points, 12 atoms, 1 / 4 complex states 18.2 / 13.5 us with
+  // MFMA, 35.7 / 29.5 plain.)
   // The z segment stays automatic (0): its choice depends on the epilogue (the Taylor
   // instance keeps one workgroup per CU, the H-apply instance two), and this timing sees
   // only the H-apply.
   std::vector<TuneVal> cands;
-  const int bra0 = L >= 16 ? 1 : 0;
   if (op->zmarch_ok && op->n == 25) {
     for (int lc : {8, 16, 32})
       for (int lpt : {1, 2}) {
         if (lc > L || lpt > lc || (lc == 32 && lpt == 1)) continue;
-        cands.push_back(TuneVal{2, lc, lpt, 0, op->tile_iters, bra0, 0.0});
+        cands.push_back(TuneVal{2, lc, lpt, 0, op->tile_iters, 1, 0.0});
       }
   }
-  for (int gt : {2, 4}) cands.push_back(TuneVal{1, 0, 0, op->zseg, gt, bra0, 0.0});
+  for (int gt : {2, 4}) cands.push_back(TuneVal{1, 0, 0, op->zseg, gt, 1, 0.0});
   TuneVal best{};
   best.us = 1e300;
   for (size_t i = 0; i < cands.size() && !rc; ++i) {
@@ -136,7 +137,7 @@ extern "C" int octhip_hamiltonian_autotune(octhip_hamiltonian_t h, int ldf, int 
     if (!rc) rc = time_apply(h, psi, hpsi, ldf, reps, s, e0, e1, &cands[i].us);
     if (!rc && cands[i].us < best.us) best = cands[i];
   }
-  if (!rc && bra0 == 1 && h->nmat > 0) {
+  if (!rc && h->nmat > 0) {
     TuneVal plain = best;
     plain.bra = 0;
     rc = apply_config(h, plain);

@@ -173,7 +173,7 @@ def bench_hamiltonian(args, torch, api, _lib, workloads):
     torch.cuda.synchronize()
     _lib.profiling_stop()
     kern = {}
-    for k in (kname, "k_bra", "k_bra_reduce", "k_ket", "k_ket_sum", "k_zero_rows"):
+    for k in (kname, "k_bra", "k_bra_reduce", "k_ket", "k_zero_rows"):
         tot, n = _lib.profiling_get(k)
         kern[k] = {"avg_us": tot * 1e3 / n if n else None, "launches": n}
     kern[kname]["avg_us_timed_region"] = k_apply_us
@@ -278,7 +278,7 @@ def bench_taylor(args, torch, api, _lib, workloads):
 
     ms_eager = timed(eager, True)
     kern = {k: _lib.profiling_get(k) for k in ("k_zmarch", "k_apply", "k_bra", "k_bra_reduce", "k_ket",
-                                               "k_ket_sum", "k_zero_rows")}
+                                               "k_zero_rows")}
     ms_graph = timed(graph.launch, False)
     ms = min(ms_graph, ms_eager)
     return {"metric": "FP64 Taylor-4 step state-point H-applies/s (128 states)",
@@ -352,7 +352,7 @@ def bench_adjoint(args, torch, api, _lib, workloads):
     _lib.profiling_stop()
     acc_ms, acc_n = _lib.profiling_get("k_adj_accum")
     breakdown = {}
-    for k in ("k_zmarch", "k_apply", "k_bra", "k_bra_reduce", "k_ket", "k_ket_sum", "k_adj_accum", "k_zero_rows"):
+    for k in ("k_zmarch", "k_apply", "k_bra", "k_bra_reduce", "k_ket", "k_adj_accum", "k_zero_rows"):
         t, n = _lib.profiling_get(k)
         breakdown[k] = {"total_ms_per_rep": t, "launches_per_rep": n}
     step_ms = t_b * 1e3 / nsteps

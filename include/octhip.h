@@ -408,7 +408,8 @@ int octhip_adjoint_destroy(octhip_adjoint_t adj);
 /* --------------------------------------------------------------- profiling --
  * Per-kernel device timing with HIP events recorded on the launch stream, the device-side
  * counterpart of profiling_in/profiling_out (src/basic/profiling.F90:503-625).  Regions
- * are kernel names ("k_zmarch", "k_apply", "k_bra", "k_bra_reduce", "k_ket", "k_ket_sum", "k_zero_rows", "k_zaxpy", "k_density").
+ * are kernel names ("k_zmarch", "k_apply", "k_bra", "k_bra_reduce", "k_ket", "k_zero_rows",
+ * "k_zaxpy", "k_density"); a z-march that takes the bra along counts as "k_zmarch".
  * start clears earlier records; get synchronises the recorded events and returns the
  * summed milliseconds and the number of launches of one region. */
 int octhip_profiling_start(void);

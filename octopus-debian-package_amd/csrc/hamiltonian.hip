@@ -134,7 +134,7 @@ int run_bra(octhip_hamiltonian_s* h, const double* f, int L, hipStream_t s, doub
     rc = launch_bra_mfma(m, bra_mfma_lds(h, L), s);
   } else {
     m.b.pjmax = h->max_nprojs;
-    rc = launch_bra(m.b, h->nchunk, false, s);
+    rc = launch_bra(m.b, h->nchunk, s);
   }
   if (rc) return rc;
   return run_ket(h, L, m.b.pjmax, mfma && m.sets, s);
@@ -439,12 +439,11 @@ void build_ket(octhip_hamiltonian_s* h, const double* matrices, const std::vecto
   std::stable_sort(pts.begin(), pts.end(), [&](int p, int q) { return cmp(p, q) < 0; });
   h->nslot = (int)pts.size();
   t.slot.assign(h->np, 0);
-  int set = 0, widest = 0;  // most slots of a set
+  int widest = 0;  // most slots of a set
   for (size_t i = 0, e; i < pts.size(); i = e) {
     for (e = i + 1; e < pts.size() && e < i + 16 && cmp(pts[i], pts[e]) == 0;) ++e;
     const int p0 = pos[pts[i]], ne = pos[pts[i] + 1] - p0, n = (int)(e - i);
     const int step0 = (int)t.step.size(), line0 = (int)(t.pt.size() / 4);
-    if (i > 0 && cmp(pts[i - 1], pts[i]) != 0) ++set;
     widest = std::max(widest, ne);
     for (int k = 0; k < ne; ++k) {
       const int a = ent[p0 + k].y;
@@ -466,7 +465,6 @@ void build_ket(octhip_hamiltonian_s* h, const double* matrices, const std::vecto
     g.steps = (int)t.step.size() - step0;
     g.step = step0;
     g.line = line0;
-    g.set = set;
     t.grp.push_back(g);
     for (size_t r = i; r < e; ++r) t.slot[pts[r]] = (int)r + 1;
   }

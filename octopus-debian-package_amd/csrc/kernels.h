@@ -366,7 +366,7 @@ constexpr int KET_AHEAD = 4;
 // those of shared mesh points: 15 + 8 us); R = 10 x 128 lanes 6.5 (10.5 + 6.4).
 struct KetGroup {
   int row, rows, steps, step;         // first ket row, rows, steps, first step
-  int line, set, pad[2];              // first line of pt, number of the group's set
+  int line, pad[3];                   // first line of pt
   int proj[KET_AHEAD];                // the first steps again: one load fetches a group
   int sum[KET_AHEAD];
 };
@@ -413,7 +413,8 @@ struct BraMfmaArgs {
   int sets;                       // the bra by sets (else by spheres)
   const double* __restrict__ pt;  // total_points x pjs
   int pjs;
-  // optional: rows [zfirst, zfirst + zcount) of zf cleared by blocks nbra.. of the launch
+  // optional: zcount doubles of zf from zfirst cleared by blocks of their own (the first ones of
+  // k_bra_mfma, the last ones of k_zmarch_bra)
   double* zf;
   size_t zfirst, zcount;
   int nbra;                       // blocks doing the bra: chunks (blocks) x lane tiles
@@ -430,7 +431,7 @@ enum { MULTI_BRA_MFMA = 1, MULTI_BRA_SETS, MULTI_BRA_PLAIN, MULTI_BRA_REDUCE, MU
 // args: device array of nseg argument blocks; off: device array of nseg+1 block offsets
 int launch_multi(int kind, const void* args, const int* off, int nseg, int nblocks, hipStream_t s, size_t lds = 0);
 
-int launch_bra(const BraArgs& b, int nchunk, bool mfma, hipStream_t s);
+int launch_bra(const BraArgs& b, int nchunk, hipStream_t s);
 // whether the MFMA bra of h goes by sets
 bool bra_by_sets(const octhip_hamiltonian_s* h);
 // whether the MFMA bra takes rows of L lanes: by spheres whole tiles, by sets any.  A tile is

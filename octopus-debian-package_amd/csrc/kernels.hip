@@ -269,13 +269,12 @@ __global__ __launch_bounds__(BLOCK) void k_bra_reduce(const BraReduceArgs r) {
 
 namespace octhip {
 
-int launch_bra(const BraArgs& b, int nchunk, bool mfma, hipStream_t s) {
+int launch_bra(const BraArgs& b, int nchunk, hipStream_t s) {
   if (nchunk <= 0) return OCTHIP_SUCCESS;
   ProfScope prof("k_bra", s);
   hipLaunchKernelGGL(k_bra_plain, dim3(nchunk), dim3(BLOCK), 0, s, b);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(OCTHIP_ERR_HIP, "k_bra launch: %s", hipGetErrorString(e));
-  (void)mfma;
   return OCTHIP_SUCCESS;
 }
 
@@ -294,8 +293,9 @@ int launch_bra_mfma(BraMfmaArgs& m, size_t lds, hipStream_t s) {
   return OCTHIP_SUCCESS;
 }
 
-// One workgroup per (KET_GROUPS groups, lane tile of 16 TW lanes), a group per wave.  MFMA form: D(16 rows x 16 lanes) = A(16 rows x 4
-// projectors) B(4 projectors x 16 lanes); lane (kk, ii) supplies A[ii][kk] = P[row ii, kk]
+// One workgroup per (KET_GROUPS groups, lane tile of 16 TW lanes), a group per wave.  MFMA form:
+// D(16 rows x 16 lanes) = A(16 rows x 4 projectors) B(4 projectors x 16 lanes); lane (kk, ii)
+// supplies A[ii][kk] = P[row ii, kk]
 // and B[kk][ii] = proj[kk, col] of the step; accumulator element r of lane (kk, ii) is
 // D[4r+kk][ii].  Operands past a group's rows are clamped: their D rows are not stored.
 // TW = 2: 32-lane tiles, lane ii computes columns 2ii and 2ii+1 with two MFMAs that share

@@ -43,10 +43,11 @@ constexpr int KCOLS = 1 << (MAX_LDF - 1);  // most complex states of a row
 
 // Device buffers of one stream: nvec batches of np_part rows (Krylov vectors or the
 // Chebyshev recurrence) and a small block, in doubles:
-//   res    [0]      overlaps of a step with two vectors (complex), then the norm: one copy to host
-//   coef   [RES]    factors of up to GS_MAX vectors and the scaling (complex)
-//   kept   [KEPT]   the norms the two latest Krylov vectors are kept with, by parity
-//   part   [PART]   partial sums
+//   res    K_RES    overlaps of a step with two vectors (complex), then the norm: one copy to host
+//   coef   K_COEF   factors of up to GS_MAX vectors, then `scale`, the scaling (complex)
+//   kept   K_KEPT   the norms the two latest Krylov vectors are kept with, by parity
+//   part            partial sums
+// host is the pinned copy of res, ready an event behind that copy.
 struct KrylovBufs {
   double* vec = nullptr;
   double *res = nullptr, *coef = nullptr, *scale = nullptr, *kept = nullptr, *part = nullptr;

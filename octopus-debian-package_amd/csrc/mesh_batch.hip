@@ -1,8 +1,7 @@
-// Batched mesh reductions and per-state BLAS-1 on packed batches (mesh_batch_dotp_vector,
-// mesh_batch_nrm2, mesh_batch_orthogonalization: src/grid/mesh_batch_inc.F90:379-549,
-// 970-1274; batch_axpy / batch_scal with one factor per state: src/grid/batch_ops_inc.F90),
-// and the two Krylov-free alternatives to Taylor built on them: the Lanczos and Chebyshev
-// exponentials (src/electrons/exponential.F90:766-971).
+// Batched mesh reductions on packed batches (mesh_batch_dotp_vector, mesh_batch_nrm2:
+// src/grid/mesh_batch_inc.F90:379-549, 970-1274), the Gram-Schmidt passes of
+// mesh_batch_orthogonalization and of the Lanczos exponential, and the elementwise passes of the
+// Chebyshev exponential (src/electrons/exponential.F90:766-971); csrc/krylov.hip drives them.
 //
 // Dot products are deterministic two-stage sums: every workgroup sums a fixed set of rows
 // per state column (rows p = b*G + g, b*G + g + nblk*G, ... for its G row groups, then the

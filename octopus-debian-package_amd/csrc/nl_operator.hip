@@ -216,10 +216,11 @@ std::vector<size_t> zmarch_cuts(const std::vector<int>& planes) {
 // per CU.  The items are dealt to the XCDs in contiguous parts of equal work; an XCD starts
 // its next item when one ends; an item costs its planes and ZM_OVERHEAD steps (index and row
 // prologue, four planes behind the last one); and all workgroups slow down together once more
-// than ZM_FULL16 (ZM_FULL8) per CU run (they share LDS, the vector caches and the memory).  Fitted to sweeps on MI355X, 16 lanes: 0.47 us per step alone (57,777 points,
-// 8 complex states: 8 planes 13.3 us, 12: 15.1, 16: 16.6, 32: 24.5), 462,781 points, 32 states:
-// 12 planes 183 us, 16: 179, 24: 175, 32: 172, 48: 175; 155,331 points, 32 states: 8 planes
-// 60 us, 16: 52, 24: 55, 48: 49; 64^3 points, 8 real functions: 8 planes 13.8 us, 24: 17.2.
+// than ZM_FULL16 (ZM_FULL8) per CU run (they share LDS, the vector caches and the memory).  Fitted
+// to sweeps on MI355X, 16 lanes: 0.47 us per step alone (57,777 points, 8 complex states: 8 planes
+// 13.3 us, 12: 15.1, 16: 16.6, 32: 24.5), 462,781 points, 32 states: 12 planes 183 us, 16: 179,
+// 24: 175, 32: 172, 48: 175; 155,331 points, 32 states: 8 planes 60 us, 16: 52, 24: 55, 48: 49;
+// 64^3 points, 8 real functions: 8 planes 13.8 us, 24: 17.2.
 double zmarch_makespan(const std::vector<int>& planes, int lc, int resident) {
   static int ncu = 0;
   if (ncu <= 0 && (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, current_device()) != hipSuccess ||
@@ -385,8 +386,10 @@ bool zmarch_fits(const octhip_nl_operator_s* op, const ApplyArgs& a) {
 // (the powers of a Taylor or Krylov chain) and an array of rows is small enough for the 256 MB
 // Infinity Cache to hold what a pass reads and what it writes.  Four passes of a Taylor-4 step,
 // cached against non-temporal: rows of 35 MB 147 against 163 us, 59 MB 247 / 260, 80 MB
-// 289 / 305, 118 MB 436 / 425, 188 MB 694 / 658, 237 MB 881 / 861; a lone apply, whose output
-// nothing reads: 59 MB 50.3 / 49.6 us, 80 MB 53.3 / 50.9, 118 MB 90 / 71, 237 MB 190 / 185.
+// 289 / 305, 118 MB 436 / 425, 188 MB 694 / 658, 237 MB 881 / 861.  A lone apply's rows are read
+// by its own ket at most, where that adds to them (whole apply): 7 MB 20.5 / 19.8 us, 10 MB 20.9 /
+// 20.3, 35 MB 42.1 / 41.6, 50 MB 48.8 / 49.0, 80 MB 63.8 / 64.7, 100 MB 82.2 / 82.4; without a ket
+// 59 MB 50.3 / 49.6, 80 MB 53.3 / 50.9, 118 MB 90 / 71, 237 MB 190 / 185.
 constexpr double ZM_CACHED_BYTES = 100e6;
 int zmarch_nt(const octhip_nl_operator_s* op, const ApplyArgs& a) {
   return a.reuse && (double)op->np * a.L * sizeof(double) <= ZM_CACHED_BYTES ? 0 : 1;

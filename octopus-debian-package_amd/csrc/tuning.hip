@@ -118,9 +118,8 @@ extern "C" int octhip_hamiltonian_autotune(octhip_hamiltonian_t h, int ldf, int 
   // Candidates of the stencil pass with the MFMA bra and ket, then the plain ones on the fastest.
   // (Rows below 16 lanes too: 17,077 points, 12 atoms, 1 / 4 complex states 18.2 / 13.5 us with
   // MFMA, 35.7 / 29.5 plain.)
-  // The z segment stays automatic (0): its choice depends on the epilogue (the Taylor
-  // instance keeps one workgroup per CU, the H-apply instance two), and this timing sees
-  // only the H-apply.
+  // The z segment stays automatic (0): every launch chooses its own from its work list, and this
+  // timing sees only the H-apply.
   std::vector<TuneVal> cands;
   if (op->zmarch_ok && op->n == 25) {
     for (int lc : {8, 16, 32})

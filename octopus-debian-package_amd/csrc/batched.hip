@@ -3,13 +3,15 @@
 // The reference runs the Taylor propagator batch by batch and system by system
 // (src/td/propagation_ops_elec.F90:232-249 over batches, one propagation per system),
 // each H-apply being ~5 kernel launches.  Here every kernel kind of one Taylor order runs
-// once for all pairs: the boundary clear, the projector bra, its reduction and the ket go through multi-segment launches (a block finds its pair
-// from a block-offset table), and the fused stencil + local + ket + Taylor-epilogue pass is one
-// z-march launch over a (pair, tile segment, lane chunk) work list, cut into 8
-// contiguous parts for the 8 XCDs.  A Taylor step is then 1 + 4 * order launches
-// whatever the number of systems and batches.  Every pair has its own work buffers;
-// results are bit-identical to per-pair octhip_exponential_taylor_batch /
-// octhip_hamiltonian_apply_batch calls (same kernel bodies on the same data).
+// once for all pairs: the boundary clear, the projector bra, its reduction and the ket go
+// through multi-segment launches (a block finds its pair from a block-offset table), and the
+// fused stencil + local + ket + Taylor-epilogue pass is one z-march launch over a (pair, tile
+// segment, lane chunk) work list, cut into 8 contiguous parts for the 8 XCDs.  A Taylor step is
+// then 1 + 4 * order launches whatever the number of systems and batches.  Every pair has its
+// own work buffers; results are bit-identical to per-pair octhip_exponential_taylor_batch /
+// octhip_hamiltonian_apply_batch calls (same kernel bodies on the same data) unless a pair's
+// MFMA bra does not take the shortest rows of the launch (bra_takes_rows): all pairs then take
+// the plain bra and ket, whose sums have another order.
 #include <algorithm>
 #include <complex>
 #include <cstring>
